@@ -7,6 +7,7 @@ The structs below mirror the header field for field; `m3s_abi_version` and the
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import os
 
 import torch
@@ -308,10 +309,26 @@ def check(rc: int, what: str) -> None:
     raise RuntimeError(f"{what}: {msg}")
 
 
+def launch(fn, args: C.Structure, dev: torch.device, what: str) -> None:
+    """Call the entry point ``fn(args, stream)`` on ``dev``'s current stream and `check` it.
+    ``torch.cuda.device`` and ``torch.cuda.current_stream`` build Python objects, about 7 us
+    a launch together; a layer forward makes five launches and its backward twelve, so the
+    guard is entered only for a device that is not the current one and the stream's handle
+    is read directly (the host's share of a B=1, L=2048 layer forward: 189 -> 160 us)."""
+    if torch.cuda.current_device() == dev.index:
+        rc = fn(C.byref(args), stream_handle(dev))
+    else:
+        with torch.cuda.device(dev):
+            rc = fn(C.byref(args), stream_handle(dev))
+    check(rc, what)
+
+
+@functools.lru_cache(maxsize=None, typed=True)
 def supported(which: int, dtype: int, chunk: int, state_dim: int, headdim: int) -> bool:
     return bool(load().m3s_supported(which, dtype, chunk, state_dim, headdim))
 
 
+@functools.lru_cache(maxsize=None, typed=True)
 def raw_supported(dtype: int, chunk: int, state_dim: int, headdim: int, n_angles: int) -> bool:
     """Whether ``m3s_fwd`` takes this shape in raw mode (`m3s_fwd_raw_supported`)."""
     return bool(load().m3s_fwd_raw_supported(dtype, chunk, state_dim, headdim, n_angles))
@@ -348,4 +365,8 @@ def blx(t) -> Blx:
 
 
 def stream_handle(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream of ``device`` (a ``torch.device``, an index or None)."""
+    index = getattr(device, "index", None)
+    if index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(index)

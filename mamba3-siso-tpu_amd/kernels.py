@@ -299,8 +299,7 @@ def siso_forward(
     a.y = _lib.bhlp(y)
     a.ybar, a.chunk_states = _lib.ptr(ybar), _lib.ptr(cstates)
     a.final_ssm, a.final_k, a.final_v = final_ssm.data_ptr(), final_k.data_ptr(), final_v.data_ptr()
-    with torch.cuda.device(dev):
-        _lib.check(_lib.load().m3s_fwd(ctypes.byref(a), _lib.stream_handle(dev)), "m3s_fwd")
+    _lib.launch(_lib.load().m3s_fwd, a, dev, "m3s_fwd")
 
     if y.dtype != y_dtype:
         y = y.to(y_dtype)
@@ -419,8 +418,7 @@ def siso_forward_raw(
     a.dt_raw, a.a_raw, a.trap_raw = _lib.blx(dt_raw), _lib.blx(a_raw), _lib.blx(trap_raw)
     a.dt_bias, a.theta_prefix, a.theta_chunk_totals = bias.data_ptr(), pre.data_ptr(), ctot.data_ptr()
     a.phi_init, a.phi_final = _lib.ptr(pinit), phi_final.data_ptr()
-    with torch.cuda.device(dev):
-        _lib.check(_lib.load().m3s_fwd(ctypes.byref(a), _lib.stream_handle(dev)), "m3s_fwd")
+    _lib.launch(_lib.load().m3s_fwd, a, dev, "m3s_fwd")
     return y, final_ssm, final_k, final_v, phi_final
 
 
@@ -504,8 +502,7 @@ def siso_decode(q: Tensor, k: Tensor, v: Tensor, adt: Tensor, dt: Tensor, lam: T
     a.q_bias, a.k_bias, a.d_skip = qb_c.data_ptr(), kb_c.data_ptr(), _lib.ptr(d_c)
     a.ssm, a.k_state, a.v_state, a.phi_state = (t.data_ptr() for t in (ssm, kst, vst, phist))
     a.y = y.data_ptr()
-    with torch.cuda.device(dev):
-        _lib.check(_lib.load().m3s_decode(ctypes.byref(a), _lib.stream_handle(dev)), "m3s_decode")
+    _lib.launch(_lib.load().m3s_decode, a, dev, "m3s_decode")
     y_dtype = v.dtype if v.dtype in (torch.bfloat16, torch.float32) else mt
     if y.dtype != y_dtype:
         y = y.to(y_dtype)
@@ -547,9 +544,7 @@ def decode_layer_step(proj: Tensor, state, *, nheads: int, headdim: int, state_d
     a.q_bias, a.k_bias, a.d_skip = qb_c.data_ptr(), kb_c.data_ptr(), _lib.ptr(d_c)
     a.ssm, a.k_state, a.v_state, a.phi_state = (t.data_ptr() for t in (ssm, kst, vst, phist))
     a.y = y.data_ptr()
-    with torch.cuda.device(dev):
-        _lib.check(_lib.load().m3s_decode_layer(ctypes.byref(a), _lib.stream_handle(dev)),
-                   "m3s_decode_layer")
+    _lib.launch(_lib.load().m3s_decode_layer, a, dev, "m3s_decode_layer")
     return y, SISOState(ssm=ssm, k=kst, v=vst, phi=phist)
 
 
@@ -645,9 +640,7 @@ def decode_scan(q, k, v, adt, dt, lam, angles, q_bias, k_bias, state, d_skip=Non
     a.q_bias, a.k_bias, a.d_skip = qb_c.data_ptr(), kb_c.data_ptr(), _lib.ptr(d_c)
     a.ssm, a.k_state, a.v_state, a.phi_state = (t.data_ptr() for t in (ssm_k, kst_k, vst_k, phist_k))
     a.y = y.data_ptr()
-    with torch.cuda.device(dev):
-        _lib.check(_lib.load().m3s_decode_scan(ctypes.byref(a), _lib.stream_handle(dev)),
-                   "m3s_decode_scan")
+    _lib.launch(_lib.load().m3s_decode_scan, a, dev, "m3s_decode_scan")
     if r > 1:
         kst.copy_(kst_k[:, ::r])
         phist.copy_(phist_k[:, ::r])
@@ -790,8 +783,7 @@ def siso_backward_kernel(
     a.dphi, a.dq_bias, a.dk_bias = dphi.data_ptr(), dqb.data_ptr(), dkb.data_ptr()
     a.k_final, a.dseed_ssm = kfin.data_ptr(), dseed.data_ptr()
     a.workspace = workspace.data_ptr()
-    with torch.cuda.device(dev):
-        _lib.check(_lib.load().m3s_bwd(ctypes.byref(a), _lib.stream_handle(dev)), "m3s_bwd")
+    _lib.launch(_lib.load().m3s_bwd, a, dev, "m3s_bwd")
     return KernelGrads(dq=dq, dk=dk, dv=dv, dadt=dadt, dqk_diag=dqk, dscale=dscale, dphi=dphi,
                        dz=dz, uw=uw, dq_bias=dqb.sum(0), dk_bias=dkb.sum(0), k_final=kfin,
                        dseed_ssm=dseed)
@@ -980,9 +972,7 @@ def bcnorm_forward(xs, weights, eps: float, theta=None):
         a.dt_bias, a.theta_table = bias.data_ptr(), table.data_ptr()
         a.theta_prefix, a.theta_chunk_totals = prefix.data_ptr(), ctot.data_ptr()
         keep = (bias, RawAngles(table, prefix, ctot, chunk))
-    with torch.cuda.device(dev):
-        _lib.check(_lib.load().m3s_norm_fwd(ctypes.byref(a), _lib.stream_handle(dev)),
-                   "m3s_norm_fwd")
+    _lib.launch(_lib.load().m3s_norm_fwd, a, dev, "m3s_norm_fwd")
     if keep is not None:
         return ys, rstds, keep[1]
     return ys, rstds
@@ -1013,8 +1003,7 @@ def bcnorm_backward(xs, weights, rstds, dys, dxs):
         a.weight[i], a.rstd[i] = ws[i].data_ptr(), rstds[i].data_ptr()
         a.dy[i], a.dweight[i] = dyc[i].data_ptr(), dws[i].data_ptr()
     a.workspace = work.data_ptr()
-    with torch.cuda.device(dev):
-        _lib.check(lib.m3s_norm_bwd(ctypes.byref(a), _lib.stream_handle(dev)), "m3s_norm_bwd")
+    _lib.launch(lib.m3s_norm_bwd, a, dev, "m3s_norm_bwd")
     return dws
 
 
@@ -1062,8 +1051,7 @@ def adamw_update(params, grads, exp_avg, exp_avg_sq, lr: float, beta1: float, be
     a.eps, a.param_decay = eps, 1.0 - lr * weight_decay
     a.step_size = lr / (1.0 - beta1 ** count)
     a.bias_correction2_sqrt = math.sqrt(1.0 - beta2 ** count)
-    with torch.cuda.device(dev):
-        _lib.check(_lib.load().m3s_adamw(ctypes.byref(a), _lib.stream_handle(dev)), "m3s_adamw")
+    _lib.launch(_lib.load().m3s_adamw, a, dev, "m3s_adamw")
 
 
 def wgrad_supported(a: Tensor, b: Tensor) -> bool:
@@ -1105,8 +1093,7 @@ def wgrad(a: Tensor, b: Tensor) -> Tensor:
     w.b, w.ldb = b.data_ptr(), b.stride(0)
     w.c, w.ldc = c.data_ptr(), q
     w.workspace = ws.data_ptr() if nbytes > 0 else None
-    with torch.cuda.device(a.device):
-        _lib.check(lib.m3s_wgrad(ctypes.byref(w), _lib.stream_handle(a.device)), "m3s_wgrad")
+    _lib.launch(lib.m3s_wgrad, w, a.device, "m3s_wgrad")
     return c
 
 
@@ -1155,9 +1142,7 @@ def gemv(x: Tensor, w: Tensor) -> Tensor:
     a.x, a.ldx = x.data_ptr(), x.stride(0) if m > 1 else k
     a.w, a.ldw = w.data_ptr(), w.stride(0)
     a.y, a.ldy = y.data_ptr(), n
-    with torch.cuda.device(x.device):
-        _lib.check(_lib.load().m3s_gemv(ctypes.byref(a), _lib.stream_handle(x.device)),
-                   "m3s_gemv")
+    _lib.launch(_lib.load().m3s_gemv, a, x.device, "m3s_gemv")
     return y
 
 
@@ -1201,9 +1186,7 @@ def rms_forward(x: Tensor, weight: Tensor, eps: float, out_dtype: torch.dtype,
         add = add.contiguous()
         s = empty_like(x)
         a.add, a.sum = add.data_ptr(), s.data_ptr()
-    with torch.cuda.device(x.device):
-        _lib.check(_lib.load().m3s_rms_fwd(ctypes.byref(a), _lib.stream_handle(x.device)),
-                   "m3s_rms_fwd")
+    _lib.launch(_lib.load().m3s_rms_fwd, a, x.device, "m3s_rms_fwd")
     return (y, rstd) if add is None else (y, rstd, s)
 
 
@@ -1242,9 +1225,7 @@ def rms_backward(x: Tensor, weight: Tensor, rstd: Tensor, dy: Tensor,
             raise ValueError("rms_backward: the added tensor's dtype must be dy's")
         dadd = empty(x.shape, device=x.device, dtype=add_dtype)
         a.dadd = dadd.data_ptr()
-    with torch.cuda.device(x.device):
-        _lib.check(_lib.load().m3s_rms_bwd(ctypes.byref(a), _lib.stream_handle(x.device)),
-                   "m3s_rms_bwd")
+    _lib.launch(_lib.load().m3s_rms_bwd, a, x.device, "m3s_rms_bwd")
     return (dx, dw) if add_dtype is None else (dx, dw, dadd)
 
 
@@ -1267,9 +1248,7 @@ def swiglu_forward(h: Tensor, width: int) -> Tensor:
     a = _swiglu_args(h, width)
     out = empty(*h.shape[:-1], width, device=h.device, dtype=h.dtype)
     a.a = out.data_ptr()
-    with torch.cuda.device(h.device):
-        _lib.check(_lib.load().m3s_swiglu_fwd(ctypes.byref(a), _lib.stream_handle(h.device)),
-                   "m3s_swiglu_fwd")
+    _lib.launch(_lib.load().m3s_swiglu_fwd, a, h.device, "m3s_swiglu_fwd")
     return out
 
 
@@ -1282,9 +1261,7 @@ def swiglu_backward(h: Tensor, da: Tensor, width: int) -> Tensor:
         raise ValueError("swiglu: da must be (..., width)")
     dh = empty_like(h)
     a.da, a.dh = da.data_ptr(), dh.data_ptr()
-    with torch.cuda.device(h.device):
-        _lib.check(_lib.load().m3s_swiglu_bwd(ctypes.byref(a), _lib.stream_handle(h.device)),
-                   "m3s_swiglu_bwd")
+    _lib.launch(_lib.load().m3s_swiglu_bwd, a, h.device, "m3s_swiglu_bwd")
     return dh
 
 
@@ -1302,7 +1279,5 @@ def transpose_pad(w: Tensor, dtype: torch.dtype, out_rows: int) -> Tensor:
     a.rows, a.cols, a.out_rows = rows, cols, out_rows
     a.in_dtype, a.out_dtype = _lib.dtype_code(w.dtype), _lib.dtype_code(dtype)
     a.inp, a.in_stride, a.out = w.data_ptr(), w.stride(0), out.data_ptr()
-    with torch.cuda.device(dev):
-        _lib.check(_lib.load().m3s_transpose(ctypes.byref(a), _lib.stream_handle(dev)),
-                   "m3s_transpose")
+    _lib.launch(_lib.load().m3s_transpose, a, dev, "m3s_transpose")
     return out

@@ -156,6 +156,7 @@ KERNELS = {
 }
 
 
+@functools.lru_cache(maxsize=None, typed=True)
 def kernel_chunk(policy_name: str, chunk: int, d_state: int, headdim: int) -> Optional[int]:
     """The chunk the scan kernels run for a requested ``chunk``: the largest compiled
     chunk (forward and backward both, so the forward's per-chunk states are the ones the
@@ -173,6 +174,7 @@ def kernel_chunk(policy_name: str, chunk: int, d_state: int, headdim: int) -> Op
     return None
 
 
+@functools.lru_cache(maxsize=None, typed=True)
 def kernel_headdim(policy_name: str, chunk: int, d_state: int, headdim: int) -> Optional[int]:
     """The head width the kernels run for ``headdim``: ``headdim`` itself when it has
     scan (`kernel_chunk`) and decode kernels, else the largest compiled width dividing
@@ -198,6 +200,7 @@ def kernel_headdim(policy_name: str, chunk: int, d_state: int, headdim: int) -> 
     return None
 
 
+@functools.lru_cache(maxsize=None, typed=True)
 def decode_headdim(policy_name: str, d_state: int, headdim: int) -> Optional[int]:
     """`kernel_headdim` for the decode kernels alone (no chunk)."""
     pol = policy(policy_name).name
@@ -242,6 +245,7 @@ def validate_chunk(chunk: int) -> None:
         raise ValueError(f"chunk must be 32, 64 or a positive multiple of 128, got {chunk}")
 
 
+@functools.lru_cache(maxsize=None, typed=True)
 def validate_kernel_shape(policy_name: str, chunk: int, d_state: int, headdim: int) -> None:
     """Raise ``ValueError`` unless forward, backward and decode kernels are all compiled
     to run this (policy, chunk, d_state, headdim) -- the check the reference makes on its

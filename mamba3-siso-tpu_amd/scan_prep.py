@@ -170,8 +170,7 @@ def prep_forward_launch(r_dt: Tensor, r_a: Tensor, r_tr: Tensor, r_ang: Tensor,
         a.phi = phi.data_ptr()
     a.phi_final = phi_final.data_ptr()
     a.workspace = ws.data_ptr()
-    with torch.cuda.device(dev):
-        _lib.check(lib.m3s_prep_fwd(ctypes.byref(a), _lib.stream_handle(dev)), "m3s_prep_fwd")
+    _lib.launch(lib.m3s_prep_fwd, a, dev, "m3s_prep_fwd")
     return adt, gamma, scale, lam, dt, phi, phi_final
 
 
@@ -201,8 +200,7 @@ def prep_backward_launch(r_dt: Tensor, r_a: Tensor, r_tr: Tensor, r_ang: Tensor,
     a.ddt_raw, a.da_raw, a.dtrap_raw, a.dangles = (_lib.blx(t) for t in (d_dt, d_a, d_tr, d_ang))
     a.ddt_bias, a.dphi_init = d_bias.data_ptr(), _lib.ptr(d_init)
     a.workspace = ws.data_ptr()
-    with torch.cuda.device(dev):
-        _lib.check(lib.m3s_prep_bwd(ctypes.byref(a), _lib.stream_handle(dev)), "m3s_prep_bwd")
+    _lib.launch(lib.m3s_prep_bwd, a, dev, "m3s_prep_bwd")
 
 
 class _PrepFn(torch.autograd.Function):
