@@ -517,7 +517,19 @@ int64_t m3s_norm_bwd_workspace_bytes(int32_t width);
  * counterpart in the reference. -1 on a bad width. */
 int64_t m3s_rms_bwd_workspace_bytes(int32_t width);
 
+/* Bytes of m3s_fwd_ws's workspace: the states and decays of the pieces of the sequences
+ * that the scan cuts into segments, where B*H sequences leave its last round of workgroups
+ * half empty or emptier; 0 where none is cut. No counterpart in the reference. -1 on bad
+ * dimensions or a shape without a kernel. */
+int64_t m3s_fwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t seqlen, int32_t nheads,
+                                int32_t headdim, int32_t state_dim, int32_t chunk);
+
+/* m3s_fwd is m3s_fwd_ws without a workspace: every sequence stays in one workgroup. */
 int32_t m3s_fwd(const m3s_fwd_args* args, void* stream);
+/* `workspace`: m3s_fwd_workspace_bytes() bytes of scratch (16-aligned; `workspace_bytes` is
+ * its size), or NULL. Same results to float32 rounding of the carried state. */
+int32_t m3s_fwd_ws(const m3s_fwd_args* args, void* workspace, int64_t workspace_bytes,
+                   void* stream);
 int32_t m3s_bwd(const m3s_bwd_args* args, void* stream);
 int32_t m3s_decode(const m3s_decode_args* args, void* stream);
 int32_t m3s_decode_scan(const m3s_decode_scan_args* args, void* stream);

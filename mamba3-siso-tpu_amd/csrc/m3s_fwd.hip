@@ -27,6 +27,7 @@
 
 #include "m3s_common.h"
 #include "m3s_internal.h"
+#include "m3s_split.h"
 
 namespace m3s {
 
@@ -73,6 +74,10 @@ struct FwdParams {
   const float* ctot;
   const float* phi_init;
   float* phi_final;
+  // split sequences (m3s_split.h): the plan and the chunks' shares; NULL without a split
+  Split split;
+  float* shares;
+  float* decay;
 };
 
 template <typename MT> struct V16;
@@ -689,6 +694,21 @@ struct Fwd2Cfg {
   static_assert(LDS_BYTES <= 163840, "LDS budget of one gfx950 CU");
 };
 
+// One rotated pair, its fused multiply-adds written out so that fwd_bf16_kernel and
+// fwd_state_kernel round khat alike whatever the compiler contracts around them.
+__device__ __forceinline__ float rot_lo(float lo, float hi, float cs, float sn) {
+  return fmaf(lo, cs, -(hi * sn));
+}
+__device__ __forceinline__ float rot_hi(float lo, float hi, float cs, float sn) {
+  return fmaf(hi, cs, lo * sn);
+}
+
+// Raw mode's angle of a row, in turns: the angle entering its strip plus the strip's thetas
+// up to it (lane = row of a 16-lane DPP row).
+__device__ __forceinline__ float raw_turns(float entering, float theta) {
+  return __builtin_amdgcn_fractf((entering + row_prefix16(theta)) * 0.15915494309189535f);
+}
+
 // Compile-time case selector for generic lambdas (`decltype(tag)::value`).
 template <int V> struct IntTag { static constexpr int value = V; };
 
@@ -726,6 +746,235 @@ constexpr bool raw_fits() {
   return NRB > 0 && Fwd2Cfg<C, N, P>::LDS_BYTES + 4 * raw_strip_floats<C, NRB>() <= 163840;
 }
 
+// Raw mode, a workgroup that starts at chunk c0 > 0: the angles entering it, by the carry's
+// own chain (phi_init, then one add and wrap per chunk), from the chunk totals staged in
+// tiles through `tile` (cap floats) so that the chain waits on LDS and not on HBM.
+// out: Nr floats (thread j < Nr returns out[j]). Ends at a barrier.
+template <int NT>
+__device__ __forceinline__ float angle_entering(const FwdParams& p, int64_t bh, int c0, float* tile,
+                                               int cap, float* out) {
+  const int Nr = p.Nr, tid = threadIdx.x;
+  const float* ct = p.ctot + bh * (int64_t)p.nc * Nr;
+  float a = (p.phi_init && tid < Nr) ? p.phi_init[bh * Nr + tid] : 0.f;
+  const int step = cap / Nr;
+  for (int c = 0; c < c0; c += step) {
+    const int n = step < c0 - c ? step : c0 - c;
+    for (int i = tid; i < n * Nr; i += NT) tile[i] = ct[(int64_t)c * Nr + i];
+    __syncthreads();
+    if (tid < Nr)
+      for (int i = 0; i < n; ++i) a = wrap_2pi_fast(a + tile[i * Nr + tid]);
+    __syncthreads();
+  }
+  if (tid < Nr) out[tid] = a;
+  __syncthreads();
+  return a;
+}
+
+// fwd_share_kernel: one chunk's share of the state of a split sequence, (v 2^{A_last - A})^T
+// khat, and its decay 2^{A_last}: fwd_bf16_kernel's state update alone, from the same rounded
+// operands in the same order and fragment ownership, so the chain over the shares gives the
+// very state the scan would have carried. One workgroup per (sequence, chunk); all its loads
+// are issued at the start and there is one pass, so latency bounds it: 52 KB of LDS and at
+// most 128 registers let two to three workgroups share a CU (two blocks of built angles spill
+// there, so that form has the registers of one). NRB = 0: phi and the row scalars are read;
+// RAW: built from the raw slices, as in fwd_bf16_kernel.
+template <int C, int N, int P, int NRB, bool RAW>
+__global__ void __launch_bounds__(C / 16 * 64, NRB > 1 ? 2 : 4) fwd_share_kernel(const FwdParams p) {
+  using F = Fwd2Cfg<C, N, P>;
+  static_assert(RAW == (NRB > 0), "phi is read, or built in raw mode");
+  constexpr int NT = F::NT, LDK = F::LDK, H2 = N / 2, SPW = F::SPW, NSTEP = F::NSTEP;
+  constexpr int SPC = C / 16;
+  constexpr int NQ = RAW ? NRB : F::LOB;      // 32-column blocks that can hold rotary pairs
+  __shared__ __align__(16) bf16 sK[C * LDK];
+  __shared__ __align__(16) bf16 sV[C * P];
+  __shared__ __align__(16) float sKb[N];
+  __shared__ __align__(16) float sFac[C];
+  __shared__ __align__(16) float sP[RAW ? 32 * NRB : 4];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nd = p.split.shares(p.nc, false);
+  const int item = xcd_remap(blockIdx.x, gridDim.x);
+  const int r = item / nd, c = item - r * nd;   // split sequence, chunk
+  const int64_t bh = p.split.whole + r;
+  const int b = (int)(bh / p.H), h = (int)(bh % p.H);
+  const int L = p.L, Nr = p.Nr;
+  const int g = lane >> 4, g8 = 8 * g;
+  const int trow = 16 * wave + (lane & 15);   // this lane's row in the chunk
+
+  const auto rK = make_rsrc(static_cast<const bf16*>(p.k) + (int64_t)b * L * N, (uint32_t)L * N * 2);
+  const bf16* vg = static_cast<const bf16*>(p.v) + b * p.v_sb + h * p.v_sh;
+  const auto rV = make_rsrc(vg, (uint32_t)(((int64_t)(L - 1) * p.v_st + P) * 2));
+  const float* phig = RAW ? p.tht + (int64_t)b * L * Nr : p.phi + bh * (int64_t)L * Nr;
+  const auto rPhi = make_rsrc(phig, (uint32_t)L * Nr * 4);
+  const int64_t sc_st = RAW ? p.sc_st : 0;
+  const bf16* scg = RAW ? static_cast<const bf16*>(p.sc) + b * p.sc_sb + h : nullptr;
+  const auto rSc = make_rsrc(scg, RAW ? (uint32_t)(((int64_t)(L - 1) * sc_st + p.sc_span) * 2) : 0u);
+  const float dtb = RAW ? p.dt_bias[h] : 0.f;
+
+  bf16x8 rk[F::NBK], rv[F::VPL];
+  f32x4 rph[NQ][2], rpre[RAW ? NRB : 1][2];
+  float rs0, rad[F::E], rar[RAW ? F::E : 1];
+#pragma unroll
+  for (int blk = 0; blk < F::NBK; ++blk)
+    rk[blk] = buf_load<bf16x8>(rK, (uint32_t)(trow * N + g8 + 32 * blk) * 2, (uint32_t)c * C * N * 2);
+#pragma unroll
+  for (int i = 0; i < F::VPL; ++i) {
+    const int id = tid + i * NT, row = id >> 3, col = 8 * (id & 7);
+    rv[i] = buf_load<bf16x8>(rV, (uint32_t)(row * p.v_st + col) * 2, (uint32_t)(c * C * p.v_st * 2));
+  }
+  const uint32_t sphi = (uint32_t)c * C * Nr * 4;
+#pragma unroll
+  for (int lb = 0; lb < NQ; ++lb) {
+#pragma unroll
+    for (int qd = 0; qd < 2; ++qd) {
+      const int jq = 32 * lb + g8 + 4 * qd;
+      if (Nr % 4 == 0) {   // quads past Nr hold other angles, never used
+        rph[lb][qd] = buf_load<f32x4>(rPhi, (uint32_t)(trow * Nr + jq) * 4, sphi);
+        if constexpr (RAW)
+          rpre[lb][qd] = gld<f32x4>(p.tpre + bh * (int64_t)(L / 16) * Nr,
+                                    (uint32_t)((c * SPC + wave) * Nr + (jq < Nr ? jq : 0)) * 4);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          rph[lb][qd][i] = jq + i < Nr ? buf_load<float>(rPhi, (uint32_t)(trow * Nr + jq + i) * 4, sphi) : 0.f;
+      }
+    }
+  }
+  if constexpr (RAW) {   // one scalar per lane: dt or trap of row trow or trow + 1
+    const uint32_t sc0 = (uint32_t)(c * C * sc_st * 2);
+    const uint32_t o = (uint32_t)((trow + (g >> 1)) * sc_st + ((g & 1) ? p.t_off : 0)) * 2;
+    rs0 = (float)buf_load<bf16>(rSc, o, sc0);
+    if (wave == 0) {
+#pragma unroll
+      for (int e = 0; e < F::E; ++e) {
+        const uint32_t oa = (uint32_t)((lane * F::E + e) * sc_st) * 2;
+        rad[e] = (float)buf_load<bf16>(rSc, oa, sc0);
+        rar[e] = (float)buf_load<bf16>(rSc, oa + 2 * p.a_off, sc0);
+      }
+    }
+  } else {
+    rs0 = p.scale[bh * L + c * C + trow];
+    if (wave == 0) {
+#pragma unroll
+      for (int e = 0; e < F::E; ++e) rad[e] = p.adt[bh * L + c * C + lane * F::E + e];
+    }
+  }
+  for (int i = tid; i < N; i += NT) sKb[i] = p.kb[h * N + i];
+  if constexpr (RAW)   // sP: the angles entering the chunk
+    angle_entering<NT>(p, bh, c, reinterpret_cast<float*>(sK), C * LDK / 2, sP);
+  else
+    __syncthreads();
+
+  // ---- khat and v into LDS, the decays -------------------------------------------------
+  float scale;
+  float turns[NQ][8];
+  if constexpr (RAW) {   // as fwd_bf16_kernel's build_turns
+    const int rr = lane & 15;
+    const bool isdt = (g & 1) == 0;
+    const float x = rs0 + (isdt ? dtb : 0.f);
+    const float u = 1.f + __builtin_amdgcn_exp2f((isdt ? x : -x) * kLog2e);
+    float v = isdt ? (x > 20.f ? x : __builtin_amdgcn_logf(u) * kLn2) : __builtin_amdgcn_rcpf(u);
+    if (g >= 2 && c * C + trow + 1 >= L) v = 0.f;
+    const float dtt = __shfl(v, rr, 64), lamt = __shfl(v, 16 + rr, 64);
+    const float dtn = __shfl(v, 32 + rr, 64), lamn = __shfl(v, 48 + rr, 64);
+    scale = fmaf(dtn, 1.f - lamn, dtt * lamt);
+#pragma unroll
+    for (int lb = 0; lb < NQ; ++lb) {
+#pragma unroll
+      for (int qd = 0; qd < 2; ++qd) {
+        const f32x4 pc = *reinterpret_cast<const f32x4*>(sP + 32 * lb + g8 + 4 * qd);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          turns[lb][4 * qd + i] = raw_turns(pc[i] + rpre[lb][qd][i], rph[lb][qd][i] * dtt);
+      }
+    }
+  } else {
+    scale = rs0;
+#pragma unroll
+    for (int lb = 0; lb < NQ; ++lb) {
+#pragma unroll
+      for (int s = 0; s < 8; ++s) turns[lb][s] = rph[lb][s >> 2][s & 3] * 0.15915494309189535f;
+    }
+  }
+  if (wave == 0) {
+    float a[F::E], run = 0.f;
+#pragma unroll
+    for (int e = 0; e < F::E; ++e) {
+      float adt;
+      if constexpr (RAW) adt = fminf(-heavy_tail_fast(rar[e]), -p.a_floor) * softplus_fast(rad[e] + dtb);
+      else adt = rad[e];
+      run = fmaf(adt, kLog2e, run);
+      a[e] = run;
+    }
+    float incl = run;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const float o = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += o;
+    }
+    const float excl = incl - run, a_last = __shfl(incl, 63, 64);
+#pragma unroll
+    for (int e = 0; e < F::E; ++e) {
+      const float A = excl + a[e];
+      sFac[lane * F::E + e] = exp2f(a_last - A);
+      if (lane == 63 && e == F::E - 1) p.decay[(int64_t)r * nd + c] = exp2f(A);
+    }
+  }
+#pragma unroll
+  for (int lb = 0; lb < F::LOB; ++lb) {
+    const int hb = lb + F::LOB, nb8 = 32 * lb + g8;
+    bf16x8 kl8, kh8;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      float kl = (float)rk[lb][s] + sKb[nb8 + s], kh = (float)rk[hb][s] + sKb[nb8 + H2 + s];
+      if (lb < NQ && nb8 + s < Nr) {
+        const float tn = turns[lb < NQ ? lb : 0][s];
+        const float sn = __builtin_amdgcn_sinf(tn), cs = __builtin_amdgcn_cosf(tn);
+        const float k0 = rot_lo(kl, kh, cs, sn), k1 = rot_hi(kl, kh, cs, sn);
+        kl = k0;
+        kh = k1;
+      }
+      kl8[s] = (bf16)(kl * scale);
+      kh8[s] = (bf16)(kh * scale);
+    }
+    *reinterpret_cast<bf16x8*>(sK + trow * LDK + nb8) = kl8;
+    *reinterpret_cast<bf16x8*>(sK + trow * LDK + nb8 + H2) = kh8;
+  }
+#pragma unroll
+  for (int i = 0; i < F::VPL; ++i) {
+    const int id = tid + i * NT, row = id >> 3, col = 8 * (id & 7);
+    *reinterpret_cast<bf16x8*>(sV + vz_off(row, col)) = rv[i];
+  }
+  __syncthreads();
+  // ---- sum_t (v_t 2^{A_last - A_t}) khat_t^T --------------------------------------------
+  f32x4 acc[SPW];
+#pragma unroll
+  for (int m = 0; m < SPW; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int pb_w = wave % F::PB, nb0 = wave / F::PB;
+  const int vs0 = vz_tr_off(0, pb_w * 16, lane), vs1 = vz_tr_off(4, pb_w * 16, lane);
+#pragma unroll
+  for (int k0 = 0; k0 < C; k0 += 32) {
+    const int kb = k0 + g8;
+    bf16x4 a0 = ld_tr4_at(sV + kb * 64 + vs0), a1 = ld_tr4_at(sV + kb * 64 + vs1);
+    const f32x4 f0 = *reinterpret_cast<const f32x4*>(sFac + kb);
+    const f32x4 f1 = *reinterpret_cast<const f32x4*>(sFac + kb + 4);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      a0[s] = (bf16)((float)a0[s] * f0[s]);
+      a1[s] = (bf16)((float)a1[s] * f1[s]);
+    }
+#pragma unroll
+    for (int m = 0; m < SPW; ++m) {
+      const int nb = nb0 + NSTEP * m;
+      mma32(acc[m], a0, a1, ld_tr4(sK, LDK, kb, nb * 16, lane), ld_tr4(sK, LDK, kb + 4, nb * 16, lane));
+    }
+  }
+  f32x4* out = reinterpret_cast<f32x4*>(p.shares) + ((int64_t)r * nd + c) * (N * P / 4);
+#pragma unroll
+  for (int m = 0; m < SPW; ++m) out[(wave * SPW + m) * 64 + lane] = acc[m];
+}
+
 // NRB = 0: phi is read. NRB > 0 (phi_strips mode): phi is built from the compact form,
 // and NRB is the number of 32-column blocks that hold rotary pairs (Nr <= 32 NRB).
 // RAW (raw mode, NRB > 0): the row scalars come from the projection's raw dt / a / trap
@@ -736,6 +985,7 @@ template <int C, int N, int P, int NRB, bool RAW = false>
 __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p) {
   using F = Fwd2Cfg<C, N, P>;
   constexpr bool STRIPS = NRB > 0;
+  constexpr bool SHARES = !STRIPS || RAW;      // may be split (m3s_split.h)
   static_assert(NRB <= F::LOB, "rotary blocks lie in the rotated half");
   static_assert(!RAW || raw_fits<C, N, P, NRB>(), "raw mode needs phi built and its LDS");
   constexpr int SPC = C / 16;                  // 16-token strips per chunk
@@ -747,7 +997,13 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
 
   // four groups of each XCD's workgroups start 0, 4, 8 and 12 K cycles late (a chunk takes
   // about 16 K): at B=8 L=8192 H=32 the scan took 2% less
-  if (p.nc >= 16) stagger_start(blockIdx.x, 4, 2);
+  int wid, seg;
+  split_block(p.split, blockIdx.x, gridDim.x, wid, seg);
+  // this workgroup's chunks: all of them, or one segment of a split sequence
+  const bool cut = wid >= p.split.whole;
+  const int cb = cut ? p.split.seg_chunk(seg, p.nc) : 0;
+  const int ce = cut ? p.split.seg_chunk(seg + 1, p.nc) : p.nc;
+  if (ce - cb >= 16) stagger_start(blockIdx.x, 4, 2);
   __shared__ __align__(16) unsigned char smem[F::LDS_BYTES + 4 * (RAW ? raw_strip_floats<C, NRB>() : 0)];
   auto opq = [](int x) { asm volatile("" : "+s"(x)); return x; };
   bf16* sK2 = reinterpret_cast<bf16*>(smem);                                // [2] k-hat tiles
@@ -777,7 +1033,6 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
   // w + NW/2 -- which share a SIMD -- hold strips w and NW-1-w: every SIMD gets the same
   // number of score tiles (NW + 1) and one wave's share of the epilogue
   const int strip = light ? wave : 3 * F::NWL - 1 - wave;
-  const int wid = xcd_remap(blockIdx.x, gridDim.x);
   const int b = wid / p.H, h = wid % p.H;
   const int64_t bh = (int64_t)b * p.H + h;
   const int L = p.L, Nr = p.Nr, nc = p.nc;
@@ -842,14 +1097,20 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int prow = pb_w * 16 + 4 * (lane >> 4) + i;
-        Sacc[m][i] = p.seed_ssm[(bh * P + prow) * N + ncol] + coef * p.seed_v[bh * P + prow] * kp;
+        Sacc[m][i] = seeded(p.seed_ssm[(bh * P + prow) * N + ncol], coef, p.seed_v[bh * P + prow], kp);
       }
     }
+  }
+  if (seg > 0) {   // the state entering this segment, from the chain
+    const f32x4* in = reinterpret_cast<const f32x4*>(p.shares) +
+                      ((int64_t)(wid - p.split.whole) * p.split.shares(nc, false) + cb - 1) * (N * P / 4);
+#pragma unroll
+    for (int m = 0; m < SPW; ++m) Sacc[m] = in[(wave * SPW + m) * 64 + lane];
   }
   // chunk c's state in bf16, stored as the chunk_states residual right after chunk c's
   // products rather than in phase A: there every workgroup's 8-byte state stores joined the
   // same synchronised burst (training forward 0.475-0.483 -> 0.442-0.448 ms at cfg2)
-  bf16x4 csv[SPW];
+  bf16x4 csv[RAW ? 1 : SPW];   // (raw mode saves none)
   auto publish_state = [&](int cidx) {
     // S (registers) -> sS in bf16 (and kept for the chunk_states residual)
 #pragma unroll
@@ -857,13 +1118,13 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
       const int ncol = (nb0 + NSTEP * m) * 16 + (lane & 15);
       const int prow0 = pb_w * 16 + 4 * (lane >> 4);
       const bf16x4 sv = sub_from_f32<bf16>(Sacc[m]);
-      csv[m] = sv;
+      if constexpr (!RAW) csv[m] = sv;
 #pragma unroll
       for (int i = 0; i < 4; ++i) sS[(prow0 + i) * LDK + ncol] = sv[i];
     }
   };
   auto store_state = [&](int cidx) {
-    if (csg && cidx < nc) {
+    if constexpr (!RAW) if (csg) {
 #pragma unroll
       for (int m = 0; m < SPW; ++m) {
         const int ncol = (nb0 + NSTEP * m) * 16 + (lane & 15);
@@ -929,8 +1190,8 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
   float rdr[RAW ? F::E : 1], rar[RAW ? F::E : 1];
   f32x4 rX[TL], rC[TL], Pc[TL];
 
-  auto prefetch_qk = [&](int c) {   // c >= nc: a chunk that does not exist, read as zeros
-    const bool live = c < nc;
+  auto prefetch_qk = [&](int c) {   // c >= ce: not this workgroup's chunk, read as zeros
+    const bool live = c < ce;
     const auto dQ = live ? rQ : rNul, dK = live ? rK : rNul;
     if (!live) c = 0;
     int ln = threadIdx.x;
@@ -947,8 +1208,8 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
   };
   // the rest of chunk c's inputs; issued from the middle of the products, so that the
   // wait for free memory-request slots overlaps MFMA work instead of stalling a phase
-  auto prefetch_rest = [&](int c) {   // c >= nc: read as zeros, as in prefetch_qk
-    const bool live = c < nc;
+  auto prefetch_rest = [&](int c) {   // c >= ce: read as zeros, as in prefetch_qk
+    const bool live = c < ce;
     const auto dPhi = live ? rPhi : rNul, dScl = live ? rScl : rNul;
     const auto dGam = live ? rGam : rNul, dAdt = live ? rAdt : rNul;
     if (!live) c = 0;
@@ -1113,7 +1374,7 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
       const float dtt = __shfl(v, r, 64), lamt = __shfl(v, 16 + r, 64);
       const float dtn = __shfl(v, 32 + r, 64), lamn = __shfl(v, 48 + r, 64);
       rgam = dtt * lamt;
-      rscale = rgam + dtn * (1.f - lamn);
+      rscale = fmaf(dtn, 1.f - lamn, rgam);
       rpdt = dtt;
       // the angle entering this wave's strip, from the carry wave
       const float* er = sE + ((c & 1) * SPC + strip) * ELD + 8 * g;
@@ -1128,8 +1389,7 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
       for (int lb = 0; lb < NRB; ++lb) {
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-          const float th = row_prefix16(rtab[lb][s >> 2][s & 3] * rpdt);
-          trn_pre[lb][s] = __builtin_amdgcn_fractf((rstr[lb][s >> 2][s & 3] + th) * 0.15915494309189535f);
+          trn_pre[lb][s] = raw_turns(rstr[lb][s >> 2][s & 3], rtab[lb][s >> 2][s & 3] * rpdt);
         }
       }
     }
@@ -1187,7 +1447,7 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
         } else {
           adt = radt[e];
         }
-        run += adt * kLog2e;
+        run = fmaf(adt, kLog2e, run);
         a[e] = run;
       }
       float incl = run;
@@ -1237,8 +1497,8 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
     // far below the bf16 rounding of what they feed
     auto rotate = [](float turns, float& ql, float& qh, float& kl, float& kh) {
       const float sn = __builtin_amdgcn_sinf(turns), cs = __builtin_amdgcn_cosf(turns);
-      const float q0 = ql * cs - qh * sn, q1 = qh * cs + ql * sn;
-      const float k0 = kl * cs - kh * sn, k1 = kh * cs + kl * sn;
+      const float q0 = rot_lo(ql, qh, cs, sn), q1 = rot_hi(ql, qh, cs, sn);
+      const float k0 = rot_lo(kl, kh, cs, sn), k1 = rot_hi(kl, kh, cs, sn);
       ql = q0; qh = q1; kl = k0; kh = k1;
     };
     auto load_bias = [&](int lb, f32x4 (&bql)[2], f32x4 (&bqh)[2], f32x4 (&bkl)[2],
@@ -1410,7 +1670,7 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
     // (the next chunk's v and this chunk's gate z, written in the next phase A)
     __builtin_amdgcn_sched_barrier(0);
     prefetch_rest(c + 1);
-    prefetch_vz(c + 1 < nc ? rV : rNul, c + 1 < nc ? c + 1 : 0, rZ, c);
+    prefetch_vz(c + 1 < ce ? rV : rNul, c + 1 < ce ? c + 1 : 0, rZ, c);
     __builtin_amdgcn_sched_barrier(0);
     build_turns(c + 1);   // chunk c+1's angles (phi_strips mode)
     // inter-chunk: out^T[p][t] += 2^{A_t} sum_n S[p][n] q~[t][n]
@@ -1442,50 +1702,53 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
     }
     // state: S <- 2^{A_last} S + sum_t (v_t 2^{A_last - A_t}) khat_t^T   (K = time)
     const float eAl = sExpA[C - 1];
-#pragma unroll
-    for (int m = 0; m < SPW; ++m) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) Sacc[m][i] *= eAl;
-    }
+    // The chunk's share is summed from zero, then one fma per element (m3s_split.h). The
+    // scaled v fragments of all C/32 K steps are made first and kept; then tile by tile, the
+    // next tile's khat fragments read ahead of the current one's MFMAs. (Step by step, with a
+    // share of every tile live, raw mode spilled 19 registers and ran 7% longer.)
+    constexpr int KS = C / 32;
+    __builtin_amdgcn_sched_barrier(0);
     const int g8 = 8 * (lane >> 4);
     const int vs0 = vz_tr_off(0, pb_w * 16, lane), vs1 = vz_tr_off(4, pb_w * 16, lane);
-    // software-pipelined over the C/32 K steps: step i+1's fragments are read into the
-    // other register set before step i's scaling and MFMAs, so LDS latency overlaps them
-    struct StepFrags {
-      bf16x4 a0, a1;
-      f32x4 f0, f1;
-      bf16x4 kb0[SPW], kb1[SPW];
-    };
-    auto load_step = [&](int k0, StepFrags& fr) {
-      const int kb = k0 + g8;                          // a multiple of 8
-      fr.a0 = ld_tr4_at(sV + kb * 64 + vs0);
-      fr.a1 = ld_tr4_at(sV + kb * 64 + vs1);
-      fr.f0 = *reinterpret_cast<const f32x4*>(sFac + kb);
-      fr.f1 = *reinterpret_cast<const f32x4*>(sFac + kb + 4);
+    struct TileFrags { bf16x4 b0[KS], b1[KS]; };
+    auto load_tile = [&](int m, TileFrags& f) {
 #pragma unroll
-      for (int m = 0; m < SPW; ++m) {
-        const int nb = nb0 + NSTEP * m;
-        fr.kb0[m] = ld_tr4(sK, LDK, kb, nb * 16, lane);
-        fr.kb1[m] = ld_tr4(sK, LDK, kb + 4, nb * 16, lane);
+      for (int s = 0; s < KS; ++s) {
+        f.b0[s] = ld_tr4(sK, LDK, 32 * s + g8, (nb0 + NSTEP * m) * 16, lane);
+        f.b1[s] = ld_tr4(sK, LDK, 32 * s + g8 + 4, (nb0 + NSTEP * m) * 16, lane);
       }
     };
-    auto run_step = [&](StepFrags& fr) {
+    TileFrags fa, fb;
+    bf16x4 a0[KS], a1[KS];
+    load_tile(0, fa);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        fr.a0[s] = (bf16)((float)fr.a0[s] * fr.f0[s]);
-        fr.a1[s] = (bf16)((float)fr.a1[s] * fr.f1[s]);
+    for (int s = 0; s < KS; ++s) {
+      const int kb = 32 * s + g8;                      // a multiple of 8
+      a0[s] = ld_tr4_at(sV + kb * 64 + vs0);
+      a1[s] = ld_tr4_at(sV + kb * 64 + vs1);
+      const f32x4 f0 = *reinterpret_cast<const f32x4*>(sFac + kb);
+      const f32x4 f1 = *reinterpret_cast<const f32x4*>(sFac + kb + 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        a0[s][i] = (bf16)((float)a0[s][i] * f0[i]);
+        a1[s][i] = (bf16)((float)a1[s][i] * f1[i]);
       }
+    }
+    auto run_tile = [&](int m, const TileFrags& f) {
+      f32x4 share = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (!SHARES) share = Sacc[m] * eAl;
 #pragma unroll
-      for (int m = 0; m < SPW; ++m) mma32(Sacc[m], fr.a0, fr.a1, fr.kb0[m], fr.kb1[m]);
+      for (int s = 0; s < KS; ++s) mma32(share, a0[s], a1[s], f.b0[s], f.b1[s]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        Sacc[m][i] = SHARES ? fmaf(Sacc[m][i], eAl, share[i]) : share[i];
     };
-    StepFrags fa, fb;
-    load_step(0, fa);
 #pragma unroll
-    for (int k0 = 0; k0 < C; k0 += 64) {
-      if (k0 + 32 < C) load_step(k0 + 32, fb);
-      run_step(fa);
-      if (k0 + 64 < C) load_step(k0 + 64, fa);
-      if (k0 + 32 < C) run_step(fb);
+    for (int m = 0; m < SPW; m += 2) {
+      if (m + 1 < SPW) load_tile(m + 1, fb);
+      run_tile(m, fa);
+      if (m + 2 < SPW) load_tile(m + 2, fa);
+      if (m + 1 < SPW) run_tile(m + 1, fb);
     }
   };
 
@@ -1510,7 +1773,7 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
 #pragma unroll
             for (int u = 0; u < 4; ++u) yb[i + u] = o[u];
           }
-          if (p.save) {
+          if (!RAW && p.save) {   // (raw mode saves none)
             bf16x8 ybv;
 #pragma unroll
             for (int i = 0; i < 8; ++i) ybv[i] = (bf16)yb[i];
@@ -1539,26 +1802,34 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
       for (int e = 0; e < 4; ++e)
         Pc[i][e] = (p.phi_init && j0 + e < Nr) ? p.phi_init[bh * Nr + j0 + e] : 0.f;
     }
-    load_ctot(0);
+    if (seg > 0) {   // past the chunks before this segment
+      angle_entering<NT>(p, bh, cb, sOut, F::SZ_O / 4 - ELD, sOut + F::SZ_O / 4 - ELD);
+#pragma unroll
+      for (int i = 0; i < TL; ++i) {
+        const int j0 = 4 * (q + i * TQ);
+        if (j0 < Nr) Pc[i] = *reinterpret_cast<const f32x4*>(sOut + F::SZ_O / 4 - ELD + j0);
+      }
+    }
+    load_ctot(cb);
     vm_wait_all();
-    if (wave == 1) carry(0);
+    if (wave == 1) carry(cb);
   }
-  prefetch_vz(rV, 0, rNul, 0);
-  prefetch_qk(0);
-  prefetch_rest(0);
-  prefetch_angles(0);   // (raw mode: the carry's inputs for chunk 1)
+  prefetch_vz(rV, cb, rNul, 0);
+  prefetch_qk(cb);
+  prefetch_rest(cb);
+  prefetch_angles(cb);   // (raw mode: the carry's inputs for the chunk after)
   vm_wait_all();
   if constexpr (RAW) {
-    if (wave == 1) carry(1);
+    if (wave == 1) carry(cb + 1);
   }
-  __syncthreads();  // sQb / sKb (raw mode: the strip entries of chunks 0 and 1)
-  build_turns(0);
-  stage_regs();     // chunk 0
-  stage_write(0);
-  prefetch_qk(1);
+  __syncthreads();  // sQb / sKb (raw mode: the strip entries of the first two chunks)
+  build_turns(cb);
+  stage_regs();     // the first chunk
+  stage_write(cb & 1);
+  prefetch_qk(cb + 1);
   // phase A of chunk c (and of the tail): out(c-1) to sOut, S(c) to sS
   auto phase_a = [&](int c) {
-    if (c > 0) {
+    if (c > cb) {
       const int tcol = strip * 16 + (lane & 15);
 #pragma unroll
       for (int pb = 0; pb < PB; ++pb)
@@ -1566,7 +1837,7 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
     }
     publish_state(c);
   };
-  for (int c = 0; c < nc; ++c) {
+  for (int c = cb; c < ce; ++c) {
     // ---------------- phase A: also chunk c's k-hat and scalars, v of c, z of c-1 --------
     phase_a(c);
     write_vz(c == nc - 1);   // (zeros where there is no such chunk)
@@ -1576,7 +1847,7 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
     // theirs: the VALU work overlaps the partner wave's MFMA work on the same SIMD).
     // Every load is issued on every chunk (past the end through a zero-size
     // descriptor), so the compiler's wait counts stay exact across iterations.
-    if (c > 0 && light) epilogue(c - 1);
+    if (c > cb && light) epilogue(c - 1);
     products(c);
     store_state(c);
     if constexpr (RAW) {   // the strip entries of chunk c+2 (its inputs came with c+1's angles)
@@ -1590,9 +1861,9 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
     __syncthreads();
   }
   // tail: out and z of the last chunk, its epilogue
-  phase_a(nc);
+  phase_a(ce);
   write_vz(false);
-  if constexpr (RAW) {   // the carry past the last chunk is phi at L-1: phi_final, and LDS
+  if constexpr (RAW) if (ce == nc) {   // the carry past the last chunk is phi at L-1: phi_final, and LDS
     if (wave == 1) {     // row 0 of the strip table (no longer read) for final_k
       const int st = lane % SPC, q = lane / SPC;
 #pragma unroll
@@ -1606,7 +1877,8 @@ __global__ void __launch_bounds__(C / 16 * 64) fwd_bf16_kernel(const FwdParams p
     }
   }
   __syncthreads();
-  if (light) epilogue(nc - 1);
+  if (light) epilogue(ce - 1);
+  if (ce < nc) return;   // the final outputs are the last segment's
 
   // final state
 #pragma unroll
@@ -1667,21 +1939,55 @@ constexpr int raw_nrb_max() {
   return 0;
 }
 
+// Tokens a split must save (plan_split).
+constexpr int kFwdMinSaved = 3 * 128;
+
+// The first two launches of a split scan: shares and chain. Returns the scan's grid.
+template <int C, int N, int P, int NRB, bool RAW>
+static int launch_shares(const FwdParams& prm, hipStream_t stream) {
+  const int nseq = prm.B * prm.H;
+  if (prm.split.segs == 1) return nseq;
+  const int rem = nseq - prm.split.whole;
+  hipLaunchKernelGGL((fwd_share_kernel<C, N, P, NRB, RAW>), dim3(rem * prm.split.shares(prm.nc, false)),
+                     dim3(C / 16 * 64), 0, stream, prm);
+  ChainParams ch{};
+  ch.split = prm.split; ch.nc = prm.nc; ch.reverse = 0;
+  ch.shares = prm.shares; ch.decay = prm.decay;
+  if (prm.has_seed) {
+    ch.s0 = prm.seed_ssm; ch.seed_k = prm.seed_k; ch.seed_v = prm.seed_v; ch.seed_coef = prm.seed_coef;
+  }
+  hipLaunchKernelGGL((state_chain_kernel<C, N, P>), dim3(N * P / 4 / 256, rem), dim3(256), 0, stream, ch);
+  return prm.split.whole + rem * prm.split.segs;
+}
+
+// Whether a call may be split (Split): the bf16 kernel with phi read or in raw mode.
 template <typename MT, int C, int N, int P>
-static int32_t launch_fwd(const FwdParams& prm, int grid, hipStream_t stream) {
+constexpr bool can_split() { return std::is_same<MT, bf16>::value && N % 64 == 0 && C % 64 == 0; }
+
+template <typename MT, int C, int N, int P>
+static int32_t launch_fwd(FwdParams prm, int grid, hipStream_t stream) {
   const bool strips = prm.pstr != nullptr;
+  prm.split = Split{grid, 1};
+  if constexpr (can_split<MT, C, N, P>()) {
+    if (prm.shares != nullptr && !strips) {
+      prm.split = plan_split(grid, prm.nc, C, kFwdMinSaved);
+      prm.decay = prm.shares + (int64_t)(grid - prm.split.whole) * prm.split.shares(prm.nc, false) * N * P;
+    }
+  }
   if (prm.sc != nullptr) {   // raw mode: the bf16 kernel where it applies, else the generic one
     // the bf16 kernel addresses the raw slices and every stream through buffer descriptors
     const bool fast = fits_rsrc(prm, N, P) &&
                       ((int64_t)(prm.L - 1) * prm.sc_st + prm.sc_span) * (int64_t)sizeof(MT) < (1ll << 31);
     if constexpr (raw_nrb_max<MT, C, N, P>() >= 1) {
       if (fast && prm.Nr <= 32) {
+        grid = launch_shares<C, N, P, 1, true>(prm, stream);
         hipLaunchKernelGGL((fwd_bf16_kernel<C, N, P, 1, true>), dim3(grid), dim3(C / 16 * 64), 0, stream, prm);
         return launch_status("m3s_fwd");
       }
     }
     if constexpr (raw_nrb_max<MT, C, N, P>() >= 2) {
       if (fast && prm.Nr <= 64) {
+        grid = launch_shares<C, N, P, 2, true>(prm, stream);
         hipLaunchKernelGGL((fwd_bf16_kernel<C, N, P, 2, true>), dim3(grid), dim3(C / 16 * 64), 0, stream, prm);
         return launch_status("m3s_fwd");
       }
@@ -1705,6 +2011,7 @@ static int32_t launch_fwd(const FwdParams& prm, int grid, hipStream_t stream) {
         }
       }
       if (!strips) {
+        grid = launch_shares<C, N, P, 0, false>(prm, stream);
         hipLaunchKernelGGL((fwd_bf16_kernel<C, N, P, 0>), dim3(grid), dim3(C / 16 * 64), 0, stream, prm);
         return launch_status("m3s_fwd");
       }
@@ -1768,7 +2075,30 @@ int32_t fwd_raw_supported_impl(int dtype, int chunk, int n, int pdim, int nr) {
 
 }  // namespace m3s
 
+extern "C" int64_t m3s_fwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t seqlen,
+                                           int32_t nheads, int32_t headdim, int32_t state_dim,
+                                           int32_t chunk) {
+  using namespace m3s;
+  if (batch <= 0 || seqlen <= 0 || nheads <= 0 || !fwd_supported(dtype, chunk, state_dim, headdim))
+    return -1;
+#define X(MT, CC, NN, PP)                                                                   \
+  if (dtype == dtype_code<MT>() && chunk == CC && state_dim == NN && headdim == PP) {       \
+    if (!can_split<MT, CC, NN, PP>()) return 0;                                             \
+  }
+  M3S_FWD_CONFIGS(X)
+#undef X
+  const int64_t nseq = (int64_t)batch * nheads;
+  const int nc = seqlen / chunk;
+  return 4 * split_floats(plan_split(nseq, nc, chunk, kFwdMinSaved), nseq, nc, state_dim, headdim,
+                          false);
+}
+
 extern "C" int32_t m3s_fwd(const m3s_fwd_args* a, void* stream) {
+  return m3s_fwd_ws(a, nullptr, 0, stream);
+}
+
+extern "C" int32_t m3s_fwd_ws(const m3s_fwd_args* a, void* workspace, int64_t workspace_bytes,
+                              void* stream) {
   using namespace m3s;
   clear_error();
   M3S_REQUIRE(a != nullptr, "m3s_fwd: args is NULL");
@@ -1846,8 +2176,13 @@ extern "C" int32_t m3s_fwd(const m3s_fwd_args* a, void* stream) {
               "m3s_fwd: residual outputs NULL or misaligned");
   M3S_REQUIRE(a->final_ssm && a->final_k && a->final_v, "m3s_fwd: final state outputs NULL");
   M3S_REQUIRE((int64_t)B * H < (1ll << 31), "m3s_fwd: B*H too large");
+  const int64_t ws_need = m3s_fwd_workspace_bytes(a->dtype, B, L, H, P, N, C);
+  M3S_REQUIRE(workspace == nullptr || (aligned16(workspace) && workspace_bytes >= ws_need),
+              "m3s_fwd: workspace misaligned or smaller than the %lld bytes of this shape",
+              (long long)ws_need);
 
   FwdParams prm{};
+  prm.shares = ws_need > 0 ? static_cast<float*>(workspace) : nullptr;
   prm.B = B; prm.L = L; prm.H = H; prm.Nr = Nr; prm.nc = L / C;
   prm.has_d = a->has_d; prm.has_z = a->has_z; prm.has_seed = a->has_seed;
   prm.save = a->save_residuals;

@@ -196,6 +196,16 @@ def _head_sum(t: Tensor, r: int, dim: int = 1) -> Tensor:
     return t.unflatten(dim, (t.shape[dim] // r, r)).sum(dim + 1)
 
 
+def _launch_fwd(a: "_lib.FwdArgs", dev: torch.device) -> None:
+    """``m3s_fwd_ws`` on the current stream, with the scratch its shape asks for."""
+    lib = _lib.load()
+    nbytes = lib.m3s_fwd_workspace_bytes(a.dtype, a.batch, a.seqlen, a.nheads, a.headdim,
+                                         a.state_dim, a.chunk)
+    ws = empty(nbytes, device=dev, dtype=torch.uint8) if nbytes > 0 else None
+    _lib.launch(lambda args, stream: lib.m3s_fwd_ws(args, _lib.ptr(ws), max(nbytes, 0), stream),
+                a, dev, "m3s_fwd")
+
+
 def siso_forward(
     q: Tensor, k: Tensor, v: Tensor, adt: Tensor, gamma: Tensor, scale: Tensor,
     phi: Tensor, q_bias: Tensor, k_bias: Tensor, d_skip: Optional[Tensor] = None,
@@ -299,7 +309,7 @@ def siso_forward(
     a.y = _lib.bhlp(y)
     a.ybar, a.chunk_states = _lib.ptr(ybar), _lib.ptr(cstates)
     a.final_ssm, a.final_k, a.final_v = final_ssm.data_ptr(), final_k.data_ptr(), final_v.data_ptr()
-    _lib.launch(_lib.load().m3s_fwd, a, dev, "m3s_fwd")
+    _launch_fwd(a, dev)
 
     if y.dtype != y_dtype:
         y = y.to(y_dtype)
@@ -418,7 +428,7 @@ def siso_forward_raw(
     a.dt_raw, a.a_raw, a.trap_raw = _lib.blx(dt_raw), _lib.blx(a_raw), _lib.blx(trap_raw)
     a.dt_bias, a.theta_prefix, a.theta_chunk_totals = bias.data_ptr(), pre.data_ptr(), ctot.data_ptr()
     a.phi_init, a.phi_final = _lib.ptr(pinit), phi_final.data_ptr()
-    _lib.launch(_lib.load().m3s_fwd, a, dev, "m3s_fwd")
+    _launch_fwd(a, dev)
     return y, final_ssm, final_k, final_v, phi_final
 
 
