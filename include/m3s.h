@@ -493,7 +493,8 @@ int32_t m3s_fwd_raw_supported(int32_t dtype, int32_t chunk, int32_t state_dim, i
                               int32_t n_angles);
 
 /* Bytes of m3s_bwd_args.workspace: the per-head dq/dk rows, 2*B*H*L*N elements of
- * the dtype. No counterpart in the reference (its head sum is an in-kernel
+ * the dtype, and, where the scan cuts sequences into segments (m3s_fwd_workspace_bytes),
+ * the chunks' shares of the adjoint. No counterpart in the reference (its head sum is an in-kernel
  * accumulation over an H-innermost grid, kernel_bwd.py:324-333). */
 int64_t m3s_bwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t seqlen, int32_t nheads,
                                 int32_t state_dim);

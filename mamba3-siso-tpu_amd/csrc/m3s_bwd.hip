@@ -24,10 +24,12 @@
 // each head's du/dw rows to the workspace with coalesced 16-byte stores; a second,
 // HBM-bound launch (headsum_kernel) sums them over heads into dq/dk, so the result
 // does not depend on the order in which workgroups finish.
+#include <algorithm>
 #include <type_traits>
 
 #include "m3s_common.h"
 #include "m3s_internal.h"
+#include "m3s_split.h"
 
 namespace m3s {
 
@@ -72,6 +74,14 @@ struct BwdParams {
   float* kfin;
   float* dseed;
   void* part;   // (2, B, H, L, N) per-head du / dw rows, MT
+  // split sequences (m3s_split.h): the plan, the chunks' shares of the adjoint and their
+  // decays, each segment's bias gradients (2, sequences, segs, N), and (sequences, segs, N,
+  // P) scratch; NULL without a split
+  Split split;
+  float* shares;
+  float* decay;
+  float* bias_part;
+  float* dump;
 };
 
 template <typename MT> struct BV16;
@@ -921,6 +931,145 @@ struct Bwd2Cfg {
   static_assert(C <= N, "the dv rows are staged in the adjoint's N-row slot");
 };
 
+// dy silu(z), the hardware exp2 and reciprocal (sg is sigma(z))
+__device__ __forceinline__ float gate_sig(float z) {
+  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-z * kLog2e));
+}
+__device__ __forceinline__ float gated(float dy, float z) { return dy * (z * gate_sig(z)); }
+
+// bwd_share_kernel: one chunk's share of the adjoint of a split sequence, sum_t (2^{A_t} g_t)
+// q~_t^T, and its decay 2^{A_last}: bwd_bf16_kernel's adjoint update alone, from the same
+// rounded operands in the same order and fragment ownership (m3s_split.h). One workgroup per
+// (sequence, chunk) of all but the first segment, every load issued at the start; latency
+// bounds it, so it is kept to 53 KB of LDS and 128 registers: three workgroups to a CU.
+template <int C, int N, int P>
+__global__ void __launch_bounds__(C / 16 * 64, 4) bwd_share_kernel(const BwdParams p) {
+  using F = Bwd2Cfg<C, N, P>;
+  constexpr int NT = F::NT, LDQ = F::LDQ, LDP = F::LDP, H2 = N / 2, SPW = F::SPW, PB = F::PB;
+  constexpr int NSTEP = F::NW / PB, NBK = N / 32, LOB = N / 64, VPL = C * P / (NT * 8);
+  __shared__ __align__(16) bf16 sQ[C * LDQ];
+  __shared__ __align__(16) bf16 sG[C * LDP];
+  __shared__ __align__(16) float sQb[N];
+  __shared__ __align__(16) float sExpA[C];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nd = p.split.shares(p.nc, true);
+  const int item = xcd_remap(blockIdx.x, gridDim.x);
+  const int r = item / nd, slot = item - r * nd;   // split sequence, share
+  const int c = slot + p.split.seg_chunk(1, p.nc);
+  const int64_t bh = p.split.whole + r;
+  const int b = (int)(bh / p.H), h = (int)(bh % p.H);
+  const int L = p.L, Nr = p.Nr;
+  const int g8 = 8 * (lane >> 4), trow = 16 * wave + (lane & 15);
+
+  const auto rQ = make_rsrc(static_cast<const bf16*>(p.q) + (int64_t)b * L * N, (uint32_t)L * N * 2);
+  auto span = [&](int64_t st) { return (uint32_t)(((int64_t)(L - 1) * st + P) * 2); };
+  const auto rDy = make_rsrc(static_cast<const bf16*>(p.dy) + b * p.dy_sb + h * p.dy_sh, span(p.dy_st));
+  const bf16* zg = p.has_z ? static_cast<const bf16*>(p.z) + b * p.z_sb + h * p.z_sh : nullptr;
+  const auto rZ = make_rsrc(zg, zg ? span(p.z_st) : 0u);
+  const auto rPhi = make_rsrc(p.phi + bh * (int64_t)L * Nr, (uint32_t)L * Nr * 4);
+
+  bf16x8 rq[NBK], rdy[VPL], rz[VPL];
+  f32x4 rph[LOB][2];
+#pragma unroll
+  for (int blk = 0; blk < NBK; ++blk)
+    rq[blk] = buf_load<bf16x8>(rQ, (uint32_t)(trow * N + g8 + 32 * blk) * 2, (uint32_t)c * C * N * 2);
+#pragma unroll
+  for (int i = 0; i < VPL; ++i) {
+    const int id = tid + i * NT, row = id / (P / 8), col = 8 * (id % (P / 8));
+    rdy[i] = buf_load<bf16x8>(rDy, (uint32_t)(row * p.dy_st + col) * 2, (uint32_t)(c * C * p.dy_st * 2));
+    rz[i] = buf_load<bf16x8>(rZ, (uint32_t)(row * p.z_st + col) * 2, (uint32_t)(c * C * p.z_st * 2));
+  }
+#pragma unroll
+  for (int lb = 0; lb < LOB; ++lb) {
+#pragma unroll
+    for (int qd = 0; qd < 2; ++qd) {
+      const int jq = 32 * lb + g8 + 4 * qd;
+      const uint32_t o = (uint32_t)(trow * Nr + jq) * 4, s = (uint32_t)c * C * Nr * 4;
+      if (Nr % 4 == 0) {   // quads past Nr hold other angles, never used
+        rph[lb][qd] = buf_load<f32x4>(rPhi, o, s);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rph[lb][qd][i] = jq + i < Nr ? buf_load<float>(rPhi, o + 4 * i, s) : 0.f;
+      }
+    }
+  }
+  for (int i = tid; i < N; i += NT) sQb[i] = p.qb[h * N + i];
+  if (wave == 0) {
+    float a[F::E], run = 0.f;
+#pragma unroll
+    for (int e = 0; e < F::E; ++e) {
+      run = fmaf(p.adt[bh * L + c * C + lane * F::E + e], kLog2e, run);
+      a[e] = run;
+    }
+    float incl = run;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const float o = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += o;
+    }
+    const float excl = incl - run;
+#pragma unroll
+    for (int e = 0; e < F::E; ++e) sExpA[lane * F::E + e] = exp2f(excl + a[e]);
+    if (lane == 63) p.decay[(int64_t)r * nd + slot] = exp2f(excl + a[F::E - 1]);
+  }
+  __syncthreads();   // sQb
+#pragma unroll
+  for (int lb = 0; lb < LOB; ++lb) {
+    const int nb8 = 32 * lb + g8;
+    bf16x8 lo8, hi8;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const float lo = (float)rq[lb][s] + sQb[nb8 + s], hi = (float)rq[lb + LOB][s] + sQb[nb8 + H2 + s];
+      const float turns = rph[lb][s >> 2][s & 3] * 0.15915494309189535f;
+      const float sn = nb8 + s < Nr ? __builtin_amdgcn_sinf(turns) : 0.f;
+      const float cs = nb8 + s < Nr ? __builtin_amdgcn_cosf(turns) : 1.f;
+      lo8[s] = (bf16)rot_lo(lo, hi, cs, sn);
+      hi8[s] = (bf16)rot_hi(lo, hi, cs, sn);
+    }
+    *reinterpret_cast<bf16x8*>(sQ + trow * LDQ + nb8) = lo8;
+    *reinterpret_cast<bf16x8*>(sQ + trow * LDQ + nb8 + H2) = hi8;
+  }
+#pragma unroll
+  for (int i = 0; i < VPL; ++i) {
+    const int id = tid + i * NT, row = id / (P / 8), col = 8 * (id % (P / 8));
+    bf16x8 g;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      float gv = (float)rdy[i][s];
+      if (zg) gv = gated(gv, (float)rz[i][s]);
+      g[s] = (bf16)gv;
+    }
+    *reinterpret_cast<bf16x8*>(sG + row * LDP + col) = g;
+  }
+  __syncthreads();
+  f32x4 acc[SPW];
+#pragma unroll
+  for (int m = 0; m < SPW; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int pb_w = wave % PB, nb0 = wave / PB;
+#pragma unroll
+  for (int k0 = 0; k0 < C; k0 += 32) {
+    const int kb = k0 + 4 * (lane >> 4);
+    bf16x4 a0 = ld_tr4(sG, LDP, kb, pb_w * 16, lane), a1 = ld_tr4(sG, LDP, kb + 16, pb_w * 16, lane);
+    const f32x4 e0 = *reinterpret_cast<const f32x4*>(sExpA + kb);
+    const f32x4 e1 = *reinterpret_cast<const f32x4*>(sExpA + kb + 16);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      a0[s] = (bf16)((float)a0[s] * e0[s]);
+      a1[s] = (bf16)((float)a1[s] * e1[s]);
+    }
+#pragma unroll
+    for (int m = 0; m < SPW; ++m) {
+      const int nb = nb0 + NSTEP * m;
+      mma32(acc[m], a0, a1, ld_tr4(sQ, LDQ, kb, nb * 16, lane), ld_tr4(sQ, LDQ, kb + 16, nb * 16, lane));
+    }
+  }
+  f32x4* out = reinterpret_cast<f32x4*>(p.shares) + ((int64_t)r * nd + slot) * (N * P / 4);
+#pragma unroll
+  for (int m = 0; m < SPW; ++m) out[(wave * SPW + m) * 64 + lane] = acc[m];
+}
+
 template <int C, int N, int P, bool STRIPS>
 __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p) {
   using F = Bwd2Cfg<C, N, P>;
@@ -934,7 +1083,13 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
 
   // half of each XCD's workgroups start ~28 K cycles (about half of phase R plus the
   // staging) late: at B=8 L=8192 H=32 that took the backward from 1.667 to 1.614 ms
-  if (p.nc >= 16) stagger_start(blockIdx.x, 2, 14);
+  int wid, seg;
+  split_block(p.split, blockIdx.x, gridDim.x, wid, seg);
+  // this workgroup's chunks, walked from ce - 1 down to cb: all, or one segment
+  const bool cut = wid >= p.split.whole;
+  const int cb = cut ? p.split.seg_chunk(seg, p.nc) : 0;
+  const int ce = cut ? p.split.seg_chunk(seg + 1, p.nc) : p.nc;
+  if (ce - cb >= 16) stagger_start(blockIdx.x, 2, 14);
   __shared__ __align__(16) unsigned char smem[F::LDS_BYTES];
   auto opq = [](int x) { asm volatile("" : "+s"(x)); return x; };
   bf16* sQ = reinterpret_cast<bf16*>(smem);                                        // q~ [t][n]
@@ -965,7 +1120,6 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wid = xcd_remap(blockIdx.x, gridDim.x);
   const int b = wid / p.H, h = wid % p.H;
   const int64_t bh = (int64_t)b * p.H + h;
   const int L = p.L, Nr = p.Nr, nc = p.nc;
@@ -1048,6 +1202,13 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
       for (int i = 0; i < 4; ++i)
         Gacc[m][i] = p.dfs[(bh * P + pb_w * 16 + 4 * (lane >> 4) + i) * N + nb * 16 + (lane & 15)];
     }
+  }
+  if (ce < nc) {   // the adjoint entering this segment from the right, from the chain
+    const f32x4* in = reinterpret_cast<const f32x4*>(p.shares) +
+                      ((int64_t)(wid - p.split.whole) * p.split.shares(nc, true) + ce -
+                       p.split.seg_chunk(1, nc)) * (N * P / 4);
+#pragma unroll
+    for (int m = 0; m < SPW; ++m) Gacc[m] = in[(wave * SPW + m) * 64 + lane];
   }
   auto publish_adjoint = [&]() {
 #pragma unroll
@@ -1188,11 +1349,11 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
     }
   };
 
-  prefetch_qk(nc - 1);
-  prefetch_rest(nc - 1, 3);
+  prefetch_qk(ce - 1);
+  prefetch_rest(ce - 1, 3);
   __syncthreads();
 
-  for (int c = nc - 1; c >= 0; --c) {
+  for (int c = ce - 1; c >= cb; --c) {
     const int t0 = c * C;
     // ============ phase L: raw -> LDS (q~, khat, g, v, S^T), dz, dqk, uw ==============
     // This chunk's raw rows were prefetched during the previous iteration's pullback and
@@ -1206,7 +1367,7 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
         float run = 0.f;
 #pragma unroll
         for (int e = 0; e < F::E; ++e) {
-          run += radt[e] * kLog2e;
+          run = fmaf(radt[e], kLog2e, run);
           a[e] = run;
         }
         float incl = run;
@@ -1248,7 +1409,7 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
               float gv = dy;
               if (zg) {
                 const float zf = (float)rz[r][e][i];
-                const float sg = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-zf * kLog2e));
+                const float sg = gate_sig(zf);
                 gv = dy * (zf * sg);
                 odz[i] = (bf16)(dy * (float)ryb[r][e][i] * sg * (1.f + zf * (1.f - sg)));
               }
@@ -1307,8 +1468,8 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
               const float sn = (j < Nr) ? __builtin_amdgcn_sinf(turns) : 0.f;
               const float cs = (j < Nr) ? __builtin_amdgcn_cosf(turns) : 1.f;
               const float sc = rscale[r][e];
-              oq0[i] = (bf16)(ulo * cs - uhi * sn);
-              oq1[i] = (bf16)(uhi * cs + ulo * sn);
+              oq0[i] = (bf16)rot_lo(ulo, uhi, cs, sn);
+              oq1[i] = (bf16)rot_hi(ulo, uhi, cs, sn);
               ok0[i] = (bf16)((wlo * cs - whi * sn) * sc);
               ok1[i] = (bf16)((whi * cs + wlo * sn) * sc);
             }
@@ -1340,6 +1501,50 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
       asm volatile("" : "+v"(ln));
       const int lane = ln & 63, g4 = lane >> 4, l16 = lane & 15;
       const int w = wave;
+      // The adjoint first: its update needs only the tiles of phase L, and here its share's
+      // registers do not add to the products' accumulators (after them it spilled 18). The
+      // inter-chunk products below read the published (bf16) adjoint of the chunk's end.
+      // 2^{A_last} <G, S> from this wave's adjoint tiles (before the G update)
+      float gs = 0.f;
+      {
+#pragma unroll
+        for (int m = 0; m < SPW; ++m) {
+          const int nb = nb0 + NSTEP * m;
+          const f32x4 sv = sub_to_f32<bf16>(
+              *reinterpret_cast<const bf16x4*>(sST + (nb * 16 + l16) * LDP + pb_w * 16 + 4 * g4));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) gs += Gacc[m][i] * sv[i];
+        }
+      }
+      // G <- 2^{A_last} G + sum_t (2^{A_t} g[t][p]) q~[t][n]   (K = time, both by columns)
+      // (the chunk's share from zero, then one fma: m3s_split.h)
+      const float eAl = sExpA[C - 1];
+      f32x4 share[SPW];
+#pragma unroll
+      for (int m = 0; m < SPW; ++m) share[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int k0 = 0; k0 < C; k0 += 32) {
+        const int kb = k0 + 4 * g4;
+        bf16x4 a0 = ld_tr4(sG, LDP, kb, pb_w * 16, lane);
+        bf16x4 a1 = ld_tr4(sG, LDP, kb + 16, pb_w * 16, lane);
+        const f32x4 e0 = *reinterpret_cast<const f32x4*>(sExpA + kb);
+        const f32x4 e1 = *reinterpret_cast<const f32x4*>(sExpA + kb + 16);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          a0[s] = (bf16)((float)a0[s] * e0[s]);
+          a1[s] = (bf16)((float)a1[s] * e1[s]);
+        }
+#pragma unroll
+        for (int m = 0; m < SPW; ++m) {
+          const int nb = nb0 + NSTEP * m;
+          mma32(share[m], a0, a1, ld_tr4(sQ, LDQ, kb, nb * 16, lane), ld_tr4(sQ, LDQ, kb + 16, nb * 16, lane));
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < SPW; ++m) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) Gacc[m][i] = fmaf(Gacc[m][i], eAl, share[m][i]);
+      }
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
         dQ[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1455,46 +1660,9 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
           red += (float)vj[i] * iv[i];
         }
       }
-      // 2^{A_last} <G, S> from this wave's adjoint tiles (before the G update)
-      {
-        float gs = 0.f;
-#pragma unroll
-        for (int m = 0; m < SPW; ++m) {
-          const int nb = nb0 + NSTEP * m;
-          const f32x4 sv = sub_to_f32<bf16>(
-              *reinterpret_cast<const bf16x4*>(sST + (nb * 16 + l16) * LDP + pb_w * 16 + 4 * g4));
-#pragma unroll
-          for (int i = 0; i < 4; ++i) gs += Gacc[m][i] * sv[i];
-        }
-        red += sExpA[C - 1] * gs;
-      }
+      red += sExpA[C - 1] * gs;
       red = wave_total(red);
       if (lane == 0) sRed[wave] = red;
-      // G <- 2^{A_last} G + sum_t (2^{A_t} g[t][p]) q~[t][n]   (K = time, both by columns)
-      const float eAl = sExpA[C - 1];
-#pragma unroll
-      for (int m = 0; m < SPW; ++m) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) Gacc[m][i] *= eAl;
-      }
-#pragma unroll 1
-      for (int k0 = 0; k0 < C; k0 += 32) {
-        const int kb = k0 + 4 * g4;
-        bf16x4 a0 = ld_tr4(sG, LDP, kb, pb_w * 16, lane);
-        bf16x4 a1 = ld_tr4(sG, LDP, kb + 16, pb_w * 16, lane);
-        const f32x4 e0 = *reinterpret_cast<const f32x4*>(sExpA + kb);
-        const f32x4 e1 = *reinterpret_cast<const f32x4*>(sExpA + kb + 16);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          a0[s] = (bf16)((float)a0[s] * e0[s]);
-          a1[s] = (bf16)((float)a1[s] * e1[s]);
-        }
-#pragma unroll
-        for (int m = 0; m < SPW; ++m) {
-          const int nb = nb0 + NSTEP * m;
-          mma32(Gacc[m], a0, a1, ld_tr4(sQ, LDQ, kb, nb * 16, lane), ld_tr4(sQ, LDQ, kb + 16, nb * 16, lane));
-        }
-      }
       // dv epilogue: + (D + gamma u.w) g, + dfinal_v on the sequence's last row
       const bool last_chunk = p.dfv && c == nc - 1;
 #pragma unroll
@@ -1676,10 +1844,10 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
           }
           // The previous chunk's v, dy and z rows, for its phase L, into registers this
           // row has freed: the loads overlap the second row's arithmetic. Issued on every
-          // iteration (chunk 0 reloads itself on the last one): a conditional prefetch
+          // iteration (the first chunk reloads itself on the last one): a conditional prefetch
           // would keep the consumed registers alive through the whole loop body for the
           // skipped path. The rest follows the bias butterfly.
-          if (r == F::QKR - 1 && e == 0) prefetch_rest(c > 0 ? c - 1 : 0, 1);
+          if (r == F::QKR - 1 && e == 0) prefetch_rest(c > cb ? c - 1 : cb, 1);
         }
         // The lanes that share j0 differ in lane bits log2(QKG)..5. A transposing
         // butterfly over those bits halves the entries a lane keeps each round (it sends
@@ -1701,14 +1869,14 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
         }
         // the previous chunk's ybar rows, state and row scalars, into registers the
         // butterfly has freed
-        if (r == F::QKR - 1) prefetch_rest(c > 0 ? c - 1 : 0, 2);
+        if (r == F::QKR - 1) prefetch_rest(c > cb ? c - 1 : cb, 2);
 #pragma unroll
         for (int k = 0; k < BFIN; ++k) bsum[k] += bacc[k];
       }
     }
     // the previous chunk's q, k, phi rows for its phase L, into the registers phase R
     // has just consumed: in flight during the barrier wait
-    prefetch_qk(c > 0 ? c - 1 : 0);
+    prefetch_qk(c > cb ? c - 1 : cb);
     __syncthreads();
 
     // ============ phase S: dadt = suffix_sum(dA) + A_last share; publish G ============
@@ -1742,12 +1910,17 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
   }
 
   // ---- per-(b, h) outputs ------------------------------------------------------------
+  // the seed adjoint; a later segment has none and stores to its own scratch: a branch
+  // around these stores made the allocator spill 18 registers in the chunk loop (1.60 ->
+  // 1.71 ms at B=8 L=8192 H=32)
+  float* dseed =
+      cb > 0 ? p.dump + (int64_t)((int)blockIdx.x - p.split.whole) * (N * P) : p.dseed + bh * (N * P);
 #pragma unroll
   for (int m = 0; m < SPW; ++m) {
     const int nb = nb0 + NSTEP * m;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      p.dseed[(bh * P + pb_w * 16 + 4 * (lane >> 4) + i) * N + nb * 16 + (lane & 15)] = Gacc[m][i];
+      dseed[(pb_w * 16 + 4 * (lane >> 4) + i) * N + nb * 16 + (lane & 15)] = Gacc[m][i];
   }
   // bias gradients: each wave's sums into its own LDS slot (the staging area is free
   // now; every entry is held by exactly one lane of each wave), then the slots summed in
@@ -1770,8 +1943,15 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
     for (int i = tid; i < 2 * N; i += NT) {
       float acc = 0.f;
       for (int w = 0; w < NW; ++w) acc += sBias[w * 2 * N + i];
-      if (i < N) p.dqb[bh * N + i] = acc;
-      else p.dkb[bh * N + i - N] = acc;
+      if (cut) {   // one row per segment, summed with the heads (headsum_kernel)
+        const int64_t row = (int64_t)(wid - p.split.whole) * p.split.segs + seg;
+        const int64_t rows = (int64_t)(p.B * p.H - p.split.whole) * p.split.segs;
+        p.bias_part[(i < N ? row : rows + row) * N + i % N] = acc;
+      } else if (i < N) {
+        p.dqb[bh * N + i] = acc;
+      } else {
+        p.dkb[bh * N + i - N] = acc;
+      }
     }
   }
 }
@@ -1783,7 +1963,22 @@ template <typename MT>
 __global__ void __launch_bounds__(256) headsum_kernel(const MT* __restrict__ part,
                                                       float* __restrict__ dq,
                                                       float* __restrict__ dk, int B, int H,
-                                                      int64_t LN) {
+                                                      int64_t LN, Split split,
+                                                      const float* __restrict__ bias_part,
+                                                      float* __restrict__ dqb,
+                                                      float* __restrict__ dkb, int N) {
+  if ((int)blockIdx.z == B) {   // split sequences: their segments' bias gradients, in order
+    const int64_t rows = (int64_t)B * H - split.whole;
+    const float* src = bias_part + blockIdx.y * rows * split.segs * N;
+    float* dst = (blockIdx.y ? dkb : dqb) + (int64_t)split.whole * N;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < rows * N;
+         i += (int64_t)gridDim.x * blockDim.x) {
+      float acc = 0.f;
+      for (int s = 0; s < split.segs; ++s) acc += src[(i / N * split.segs + s) * N + i % N];
+      dst[i] = acc;
+    }
+    return;
+  }
   const int64_t i8 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
   const int which = blockIdx.y;           // 0: dq from du, 1: dk from dw
   const int b = blockIdx.z;
@@ -1812,13 +2007,42 @@ static bool bwd_fits_rsrc(const BwdParams& p, int N, int P) {
          (int64_t)p.nc * N * P * 2 <= lim;
 }
 
+// Tokens a split of the backward must save (plan_split): its chunks take about three times
+// the forward's. B=16 L=2048 H=24, a round and a half of sequences: 798 -> 686 us with the
+// head sum; the layer's training step at B=1 L=4096 H=32: 1.14 -> 0.72 ms.
+constexpr int kBwdMinSaved = 2 * 128;
+
+// Workspace floats past the per-head rows: shares, decays, bias rows and scratch of a split.
+static int64_t bwd_split_floats(const Split& sp, int64_t nseq, int nc, int N, int P) {
+  if (sp.segs < 2) return 0;
+  const int64_t rows = (nseq - sp.whole) * sp.segs;
+  return split_floats(sp, nseq, nc, N, P, true) + rows * (2 * N + N * P);
+}
+
 template <typename MT, int C, int N, int P>
-static int32_t launch_bwd(const BwdParams& prm, int grid, hipStream_t stream) {
+static int32_t launch_bwd(BwdParams prm, int grid, hipStream_t stream) {
   bool done = false;
   const bool strips = prm.pstr != nullptr;
+  const int nseq = grid;
+  prm.split = Split{nseq, 1};
   if constexpr (std::is_same<MT, bf16>::value && N % 64 == 0 && C % 64 == 0 && C <= N &&
                 N / 16 <= 8) {   // N <= 128: a strip's row pairs in one wave (phi strips)
     if (bwd_fits_rsrc(prm, N, P)) {
+      if (!strips) prm.split = plan_split(nseq, prm.nc, C, kBwdMinSaved);
+      if (prm.split.segs > 1) {
+        const int rem = nseq - prm.split.whole;
+        const int64_t nsh = (int64_t)rem * prm.split.shares(prm.nc, true);
+        prm.shares = reinterpret_cast<float*>(static_cast<bf16*>(prm.part) + 2 * (int64_t)nseq * prm.L * N);
+        prm.decay = prm.shares + nsh * N * P;
+        prm.bias_part = prm.decay + (nsh + 3) / 4 * 4;
+        prm.dump = prm.bias_part + (int64_t)2 * rem * prm.split.segs * N;
+        hipLaunchKernelGGL((bwd_share_kernel<C, N, P>), dim3((unsigned)nsh), dim3(C / 16 * 64), 0, stream, prm);
+        ChainParams ch{};
+        ch.split = prm.split; ch.nc = prm.nc; ch.reverse = 1;
+        ch.shares = prm.shares; ch.decay = prm.decay; ch.s0 = prm.dfs;
+        hipLaunchKernelGGL((state_chain_kernel<C, N, P>), dim3(N * P / 4 / 256, rem), dim3(256), 0, stream, ch);
+        grid = prm.split.whole + rem * prm.split.segs;
+      }
       if (strips)
         hipLaunchKernelGGL((bwd_bf16_kernel<C, N, P, true>), dim3(grid), dim3(C / 16 * 64), 0, stream, prm);
       else
@@ -1837,9 +2061,10 @@ static int32_t launch_bwd(const BwdParams& prm, int grid, hipStream_t stream) {
   if (rc != M3S_OK) return rc;
   const int64_t LN = (int64_t)prm.L * N;
   static_assert(N % 8 == 0, "head sum threads take 8 elements");
-  const dim3 hgrid((unsigned)((LN / 8 + 255) / 256), 2, prm.B);
+  const dim3 hgrid((unsigned)((LN / 8 + 255) / 256), 2, prm.B + (prm.split.segs > 1 ? 1 : 0));
   hipLaunchKernelGGL((headsum_kernel<MT>), hgrid, dim3(256), 0, stream,
-                     static_cast<const MT*>(prm.part), prm.dq, prm.dk, prm.B, prm.H, LN);
+                     static_cast<const MT*>(prm.part), prm.dq, prm.dk, prm.B, prm.H, LN, prm.split,
+                     prm.bias_part, prm.dqb, prm.dkb, N);
   return launch_status("m3s_bwd (head sum)");
 }
 
@@ -1883,8 +2108,19 @@ int32_t bwd_supported(int dtype, int chunk, int n, int pdim) {
 
 extern "C" int64_t m3s_bwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t seqlen,
                                            int32_t nheads, int32_t state_dim) {
+  using namespace m3s;
   const int64_t el = dtype == M3S_DTYPE_BF16 ? 2 : 4;
-  return 2 * (int64_t)batch * nheads * seqlen * state_dim * el;
+  const int64_t rows = 2 * (int64_t)batch * nheads * seqlen * state_dim * el;
+  // a split's scratch, at whichever chunk needs the most (the chunk is not an argument)
+  int64_t split = 0;
+  if (dtype == M3S_DTYPE_BF16 && batch > 0 && nheads > 0)
+    for (int c : {64, 128})
+      if (bwd_supported(dtype, c, state_dim, 64) && seqlen > 0 && seqlen % c == 0) {
+        const int64_t nseq = (int64_t)batch * nheads;
+        const Split sp = plan_split(nseq, seqlen / c, c, kBwdMinSaved);
+        split = std::max(split, bwd_split_floats(sp, nseq, seqlen / c, state_dim, 64));
+      }
+  return rows + 4 * split;
 }
 
 extern "C" int32_t m3s_bwd(const m3s_bwd_args* a, void* stream) {

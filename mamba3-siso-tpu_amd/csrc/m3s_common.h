@@ -348,6 +348,16 @@ __device__ __forceinline__ float wrap_2pi_fast(float phi) {
   return r >= kTwoPi ? r - kTwoPi : r;
 }
 
+// One rotated pair, its fused multiply-adds written out so that two kernels that rotate the
+// same rows (a scan and the kernel of its chunks' shares, m3s_split.h) round them alike
+// whatever the compiler contracts around them.
+__device__ __forceinline__ float rot_lo(float lo, float hi, float cs, float sn) {
+  return fmaf(lo, cs, -(hi * sn));
+}
+__device__ __forceinline__ float rot_hi(float lo, float hi, float cs, float sn) {
+  return fmaf(hi, cs, lo * sn);
+}
+
 // ---- two adjacent elements as one LDS store ---------------------------------------
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));

@@ -68,13 +68,7 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float phi_advance(float phi, float tp, float dt) {
   return wrap_2pi(fmaf(tp, dt, phi));
 }
-// the rotated pair: (lo cos - hi sin, hi cos + lo sin)
-__device__ __forceinline__ float rot_lo(float lo, float hi, float cs, float sn) {
-  return fmaf(lo, cs, -(hi * sn));
-}
-__device__ __forceinline__ float rot_hi(float lo, float hi, float cs, float sn) {
-  return fmaf(hi, cs, lo * sn);
-}
+// (the rotated pair: rot_lo / rot_hi of m3s_common.h)
 // S' = alpha S + beta v_prev k_prev + gamma v k~ for one element (bvp = beta v_prev,
 // gv = gamma v)
 __device__ __forceinline__ float state_step(float s, float alpha, float bvp, float kp, float gv,

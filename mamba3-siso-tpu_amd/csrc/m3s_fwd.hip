@@ -694,15 +694,6 @@ struct Fwd2Cfg {
   static_assert(LDS_BYTES <= 163840, "LDS budget of one gfx950 CU");
 };
 
-// One rotated pair, its fused multiply-adds written out so that fwd_bf16_kernel and
-// fwd_state_kernel round khat alike whatever the compiler contracts around them.
-__device__ __forceinline__ float rot_lo(float lo, float hi, float cs, float sn) {
-  return fmaf(lo, cs, -(hi * sn));
-}
-__device__ __forceinline__ float rot_hi(float lo, float hi, float cs, float sn) {
-  return fmaf(hi, cs, lo * sn);
-}
-
 // Raw mode's angle of a row, in turns: the angle entering its strip plus the strip's thetas
 // up to it (lane = row of a 16-lane DPP row).
 __device__ __forceinline__ float raw_turns(float entering, float theta) {

@@ -102,3 +102,45 @@ def test_split_needs_its_workspace(m3, dev):
     finally:
         K._launch_fwd = old
     assert args["rc"] == lib.ERR_INVALID and b"workspace" in lib.load().m3s_last_error()
+
+
+# (H, chunks, chunk, N, Nr, without z): heads of one sequence; padded to whole rounds of 256
+BWD_SHAPES = [(1, 4, 128, 128, 32, False), (3, 7, 128, 128, 32, True), (24, 5, 128, 128, 32, False),
+              (258, 4, 128, 128, 16, False), (4, 9, 64, 128, 64, False), (5, 11, 64, 64, 6, True)]
+
+
+@pytest.mark.parametrize("h,nc,chunk,n,nr,gate", BWD_SHAPES)
+@pytest.mark.parametrize("final", [False, True])
+def test_split_backward_equals_whole(m3, dev, h, nc, chunk, n, nr, gate, final):
+    """The same heads repeated to a full round, where nothing is split: every per-head
+    gradient bit for bit, the bias sums (over the segments, then as before) to f32 rounding."""
+    L, p, full = nc * chunk, 64, (h + 255) // 256 * 256
+    lib = m3._lib.load()
+    rows = lambda hh: 2 * hh * L * n * 2  # noqa: E731
+    assert lib.m3s_bwd_workspace_bytes(m3._lib.DTYPE_BF16, 1, L, h, n) > rows(h), "does not split"
+    assert lib.m3s_bwd_workspace_bytes(m3._lib.DTYPE_BF16, 1, L, full, n) == rows(full)
+    _, d = boundary_inputs(1, h, L, n, p, nr, "bf16", seed=h + nc)
+    gen = torch.Generator().manual_seed(nc)
+    extra = {k: torch.randn(1, h, *s, generator=gen).cuda() if final else None
+             for k, s in (("dfinal_ssm", (p, n)), ("dfinal_v", (p,)))}
+
+    def run(idx):
+        pick = lambda t, dim=1: None if t is None else t.index_select(dim, idx).contiguous()  # noqa: E731
+        z = pick(d["z"]) if gate else None
+        args = [d["q"], d["k"], pick(d["v"]), pick(d["adt"]), pick(d["gamma"]), pick(d["scale"]),
+                pick(d["phi"]), pick(d["q_bias"], 0), pick(d["k_bias"], 0)]
+        skip = pick(d["d_skip"], 0)
+        res = m3.siso_forward(*args, skip, z, chunk=chunk, save_residuals=True)[4]
+        return m3.siso_backward_kernel(
+            pick(d["dy"]), res.ybar, z, *args, res.chunk_states, d_skip=skip, chunk=chunk,
+            **{k: pick(t) for k, t in extra.items()})
+
+    idx = torch.arange(full, device=dev) % h
+    got, ref = run(idx[:h]), run(idx)
+    for name in ("dv", "dadt", "dqk_diag", "dscale", "dphi", "dz", "uw", "k_final", "dseed_ssm"):
+        a, b = getattr(got, name), getattr(ref, name)
+        if a is not None:
+            assert torch.equal(a, b[:, :h]), name
+    for name in ("dq_bias", "dk_bias"):   # at most 16 segments' f32 sums in another order
+        a, b = getattr(got, name), getattr(ref, name)[:h]
+        assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max()), name
