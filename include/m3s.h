@@ -525,6 +525,11 @@ int64_t m3s_rms_bwd_workspace_bytes(int32_t width);
 int64_t m3s_fwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t seqlen, int32_t nheads,
                                 int32_t headdim, int32_t state_dim, int32_t chunk);
 
+/* Bytes of m3s_decode_scan_ws's workspace: the carried k and phi of a run whose few states are
+ * split by rows; 0 where none is. No counterpart in the reference. -1 on bad dimensions. */
+int64_t m3s_decode_scan_workspace_bytes(int32_t batch, int32_t steps, int32_t nheads,
+                                        int32_t headdim, int32_t state_dim, int32_t n_angles);
+
 /* m3s_fwd is m3s_fwd_ws without a workspace: every sequence stays in one workgroup. */
 int32_t m3s_fwd(const m3s_fwd_args* args, void* stream);
 /* `workspace`: m3s_fwd_workspace_bytes() bytes of scratch (16-aligned; `workspace_bytes` is
@@ -533,7 +538,12 @@ int32_t m3s_fwd_ws(const m3s_fwd_args* args, void* workspace, int64_t workspace_
                    void* stream);
 int32_t m3s_bwd(const m3s_bwd_args* args, void* stream);
 int32_t m3s_decode(const m3s_decode_args* args, void* stream);
+/* m3s_decode_scan is m3s_decode_scan_ws without a workspace (one workgroup per state); with
+ * m3s_decode_scan_workspace_bytes() bytes of scratch (16-aligned) the same bits, sooner where
+ * there are few states. */
 int32_t m3s_decode_scan(const m3s_decode_scan_args* args, void* stream);
+int32_t m3s_decode_scan_ws(const m3s_decode_scan_args* args, void* workspace,
+                           int64_t workspace_bytes, void* stream);
 int32_t m3s_decode_layer(const m3s_decode_layer_args* args, void* stream);
 int32_t m3s_prep_fwd(const m3s_prep_fwd_args* args, void* stream);
 int32_t m3s_prep_bwd(const m3s_prep_bwd_args* args, void* stream);

@@ -106,14 +106,12 @@ __device__ __forceinline__ float readout4(const f32x4& s, const QPack<MT>& q) {
   }
 }
 
-// Exchange with the partner across bit B of the lane index: lane shuffles for B >= 4, the
-// row mirror (lane i <-> 15 - i) for B = 3, the half-row mirror (i <-> 7 - i) for B = 2,
-// quad swaps for B = 1, 0. The mirrors also flip the bits below B; the stages below B
+// Exchange with the partner across bit B < 4 of the lane index: the row mirror (lane i <->
+// 15 - i) for B = 3, the half-row mirror (i <-> 7 - i) for B = 2, quad swaps for B = 1, 0. The mirrors also flip the bits below B; the stages below B
 // only need the partner to agree on the bits above B and differ in bit B.
 template <int B>
 __device__ __forceinline__ float lane_xchg(float v) {
-  if constexpr (B >= 4) return __shfl_xor(v, 1 << B, 64);
-  else if constexpr (B == 3) return dpp_mov<kDppRowMirror>(v);
+  if constexpr (B == 3) return dpp_mov<kDppRowMirror>(v);
   else if constexpr (B == 2) return dpp_mov<kDppHalfMirror>(v);
   else if constexpr (B == 1) return dpp_mov<kDppQuadSwap2>(v);
   else return dpp_mov<kDppQuadSwap1>(v);
@@ -128,12 +126,34 @@ constexpr int ilog2(int x) { return x <= 1 ? 0 : 1 + ilog2(x / 2); }
 // it = l >> (log2 RV - log2 IT), the same in each of its 2^(log2 RV - log2 IT) lanes.
 // Every row is summed over the same tree of lane pairs whichever `it` slot carries it.
 // log2(IT) + (log2 RV - log2 IT) exchanges instead of IT * log2(RV).
+// Stages across 16 or 32 lanes are one v_permlane16_swap / v_permlane32_swap and one add:
+// swapping the odd rows (halves) of the low entry with the even ones of the high entry
+// leaves each lane the two terms of its own row's sum, in place of two selects and a
+// lane shuffle through LDS.
+template <int B>
+__device__ __forceinline__ float pair_sum(float lo, float hi) {
+  static_assert(B == 4 || B == 5, "across rows or halves");
+  const unsigned a = __builtin_bit_cast(unsigned, lo), b = __builtin_bit_cast(unsigned, hi);
+  if constexpr (B == 4) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+  } else {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+  }
+}
+
 template <int RV, int IT, int S = 0>
 __device__ __forceinline__ void rows_reduce_scatter(float* w, int lane) {
   constexpr int LR = ilog2(RV), LI = ilog2(IT);
   if constexpr (S < LR) {
     constexpr int B = LR - 1 - S;
-    if constexpr (S < LI) {
+    if constexpr (B >= 4) {
+      constexpr int HALF = S < LI ? IT >> (S + 1) : 0;
+      if constexpr (HALF == 0) w[0] = pair_sum<B>(w[0], w[0]);
+#pragma unroll
+      for (int k = 0; k < HALF; ++k) w[k] = pair_sum<B>(w[k], w[HALF + k]);
+    } else if constexpr (S < LI) {
       constexpr int HALF = IT >> (S + 1);
       const bool hi = (lane >> B) & 1;
 #pragma unroll
@@ -352,57 +372,74 @@ struct DecScanParams {
   float* vst;
   float* phist;
   void* y;              // (B, H, T, P)
+  float* carry;         // (B, H, N + Nr) scratch of a run in parts, or NULL
 };
 
-// (The waves-per-EU hint only steers register allocation. Without it the N = 128 kernels
-// take 189 VGPRs: two workgroups per CU. A hint of five waves makes the allocator stop at
-// 127 without spilling (a hint of four spills), and LDS then allows four workgroups; the
-// compiler warns that five is not met. N = 256 holds 64 state floats per thread and is
-// left at two waves per SIMD.)
-template <typename MT, int N, int P>
+// (The waves-per-EU hint only steers register allocation: the N = 128 kernel of whole states
+// takes 164 VGPRs, three workgroups to a CU; the compiler warns that five waves are not met.
+// N = 256 holds 64 state floats per thread and is left at two waves per SIMD, a part at four.)
+// The sines and cosines are made one (step, angle) per thread, not by the half of each
+// wave's lanes that hold a rotary pair, and the rows' sums cross 16 lanes by permlane swaps:
+// 512 states, 256 steps 292 -> 241 us; 8192 states, 64 steps 800 -> 754 us.
+//
+// PARTS > 1 splits a state's P rows over that many workgroups (rows are independent but for
+// the phi chain and the rotated q~ / k~, which every part makes for itself), for runs of few
+// states: one workgroup of the whole state holds 32 floats a thread, about 180 VALU
+// instructions a step, and leaves most CUs idle. There the next window's inputs are read
+// into registers under the steps, too. The parts cannot write the carried k~ and phi in
+// place, since another part may not have started: part 0 leaves them in `carry`, which
+// dec_carry_kernel copies back. B=1, H=32: 512 steps 408 -> 209 us, 48 steps
+// 43 -> 26; B=8, 256 steps (4 parts) 217 -> 186.
+template <typename MT, int N, int P, int PARTS>
 __global__ void __launch_bounds__(kDecThreads)
-__attribute__((amdgpu_waves_per_eu(N >= 256 ? 2 : 5, 8)))
+__attribute__((amdgpu_waves_per_eu(N >= 256 ? 2 : PARTS > 1 ? 4 : 5, 8)))
 decode_scan_kernel(const DecScanParams p) {
   constexpr int NT = kDecThreads;
+  constexpr int PP = P / PARTS;               // rows of this workgroup
   constexpr int H2 = N / 2;
   constexpr int RV = N / 4;                   // float4 per state row = lanes per row group
-  constexpr int NV = P * N / 4;               // float4 per state
+  constexpr int NV = PP * N / 4;              // float4 per workgroup
   constexpr int IT = (NV + NT - 1) / NT;      // float4 (rows) per thread
   constexpr int G = NT / RV;                  // row groups; group g owns rows g*IT .. +IT
   constexpr int W = N >= 256 ? 8 : 16;        // steps per window
   constexpr int W2 = 2 * W;                   // ring slots of k~ and v
   constexpr int LO = ilog2(RV) - ilog2(IT);
+  constexpr bool AHEAD = PARTS > 1;           // the next window's inputs under the steps
   static_assert(RV <= 64 && (RV & (RV - 1)) == 0, "row must fit a wave");
   static_assert(NT % RV == 0 && NT % H2 == 0 && (P & (P - 1)) == 0, "layout");
-  static_assert(IT == 1 || G * IT == P, "row groups cover the state");
-  static_assert((W * P * sizeof(MT)) % 16 == 0, "y window in 16-byte vectors");
+  static_assert(IT == 1 || G * IT == PP, "row groups cover the state");
+  static_assert((PP * sizeof(MT)) % 16 == 0 || PARTS == 1, "a part's y row in 16-byte vectors");
+  static_assert((W * PP * sizeof(MT)) % 16 == 0, "y window in 16-byte vectors");
 
   __shared__ __align__(16) float sK[W2][N];   // k~ by step (slot t mod 2W)
-  __shared__ __align__(16) float sV[W2][P];   // v by step (slot t mod 2W)
+  __shared__ __align__(16) float sV[W2][PP];  // v by step (slot t mod 2W)
   __shared__ __align__(16) MT sQ[W][N];       // q~, by window step
-  __shared__ __align__(16) float sZ[W][P];    // silu(z)
+  __shared__ __align__(16) float sZ[W][PP];   // silu(z)
   __shared__ __align__(16) float sC[W][4];    // alpha, beta, gamma, dt
-  __shared__ float sPh[W][H2];                // angle increments, then phi
-  __shared__ __align__(16) MT sY[W][P];       // gated y of the window
+  __shared__ float sPh[W][H2];                // angle increments, then phi, then cos phi
+  __shared__ float sSn[W][H2];                // sin phi
+  __shared__ __align__(16) MT sY[W][PP];      // gated y of the window
 
   const int tid = threadIdx.x;
   const int wid = xcd_remap(blockIdx.x, gridDim.x);
-  const int b = wid / p.H, h = wid % p.H;
-  const int64_t bh = (int64_t)b * p.H + h;
+  const int64_t bh = wid / PARTS;
+  const int part = wid % PARTS, row0 = part * PP;
+  const int b = (int)(bh / p.H), h = (int)(bh % p.H);
   const int T = p.T, Nr = p.Nr;
   const int g = tid / RV, lane = tid % RV, n0 = lane * 4;
+  const DivMod by_nr(Nr > 0 ? Nr : 1);
 
-  // the state: thread (g, lane) holds S[g*IT + it, n0 : n0 + 4]
-  f32x4* sg = reinterpret_cast<f32x4*>(p.ssm + bh * P * N);
+  // the state: thread (g, lane) holds S[row0 + g*IT + it, n0 : n0 + 4]
+  f32x4* sg = reinterpret_cast<f32x4*>(p.ssm + (bh * P + row0) * N);
   f32x4 st[IT];
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
     st[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (g * IT + it < P) st[it] = __builtin_nontemporal_load(sg + (g * IT + it) * RV + lane);
+    if (g * IT + it < PP) st[it] = __builtin_nontemporal_load(sg + (g * IT + it) * RV + lane);
   }
   // the carried (k~, v) pair is step -1's, in ring slot 2W - 1
   for (int i = tid; i < N; i += NT) sK[W2 - 1][i] = p.kst[bh * N + i];
-  for (int i = tid; i < P; i += NT) sV[W2 - 1][i] = p.vst[bh * P + i];
+  for (int i = tid; i < PP; i += NT) sV[W2 - 1][i] = p.vst[bh * P + row0 + i];
   float ph = tid < Nr ? p.phist[bh * Nr + tid] : 0.f;   // phi of angle `tid`
   const int jr = tid % H2, wr = tid / H2;                // rotation: pair jr of steps wr + k NT/H2
   const float qbl = p.qb[h * N + jr], qbh = p.qb[h * N + H2 + jr];
@@ -410,34 +447,77 @@ decode_scan_kernel(const DecScanParams p) {
   const float dsk = p.has_d ? p.dsk[h] : 0.f;
   const MT* qg = static_cast<const MT*>(p.q) + (int64_t)b * T * N;
   const MT* kg = static_cast<const MT*>(p.k) + (int64_t)b * T * N;
-  const MT* vg = static_cast<const MT*>(p.v) + bh * T * P;
-  const MT* zg = p.has_z ? static_cast<const MT*>(p.z) + bh * T * P : nullptr;
+  const MT* vg = static_cast<const MT*>(p.v) + bh * T * P + row0;
+  const MT* zg = p.has_z ? static_cast<const MT*>(p.z) + bh * T * P + row0 : nullptr;
   const float* ag = p.angles + (int64_t)b * T * Nr;
   const float* adtg = p.adt + bh * T;
   const float* dtg = p.dt + bh * T;
   const float* lamg = p.lam + bh * T;
-  char* yb = reinterpret_cast<char*>(static_cast<MT*>(p.y) + bh * T * P);
-  constexpr int YV = W * P * (int)sizeof(MT) / 16;        // 16-byte vectors of a full window
+  char* yb = reinterpret_cast<char*>(static_cast<MT*>(p.y) + bh * T * P + row0);
+  constexpr int YR = PP * (int)sizeof(MT) / 16;           // 16-byte vectors of a part's y row
+
+  // A window's raw inputs: v, z, the step scalars, the angles, q and k. Past the run's last
+  // step the last one is read again, unused, so every load is unconditional.
+  constexpr int VN = (W * PP + NT - 1) / NT, AN = (W * H2 + NT - 1) / NT, RN = AN;
+  MT rv[VN], rz[VN], rql[RN], rqh[RN], rkl[RN], rkh[RN];
+  float rang[AN], radt = 0.f, rdt = 0.f, rlam = 0.f;
+  auto fetch = [&](int t0) {
+    const int last = T - 1;
+#pragma unroll
+    for (int u = 0; u < VN; ++u) {
+      const int i = tid + u * NT, t = min(t0 + (i / PP) % W, last);
+      rv[u] = vg[(int64_t)t * P + i % PP];
+      if (zg) rz[u] = zg[(int64_t)t * P + i % PP];
+    }
+    const int ts = min(t0 + tid % W, last);
+    radt = adtg[ts];
+    rdt = dtg[ts];
+    rlam = lamg[ts];
+    if (Nr > 0) {
+#pragma unroll
+      for (int u = 0; u < AN; ++u) {   // entry i of the window's (W, Nr) angles
+        int w, j;
+        by_nr(tid + u * NT, w, j);
+        rang[u] = ag[(int64_t)min(t0 + w, last) * Nr + j];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < RN; ++u) {
+      const int64_t t = min(t0 + wr + u * (NT / H2), last);
+      rql[u] = qg[t * N + jr];
+      rqh[u] = qg[t * N + H2 + jr];
+      rkl[u] = kg[t * N + jr];
+      rkh[u] = kg[t * N + H2 + jr];
+    }
+  };
+  if (AHEAD) fetch(0);
 
   for (int t0 = 0; t0 < T; t0 += W) {
     const int wn = T - t0 < W ? T - t0 : W;
+    if (!AHEAD) fetch(t0);
     // ---- window inputs: v, z, the step coefficients, the angle increments ----------
-    for (int i = tid; i < wn * P; i += NT) {
-      const int w = i / P, pp = i % P;
-      sV[(t0 + w) & (W2 - 1)][pp] = (float)vg[(int64_t)(t0 + w) * P + pp];
-      if (zg) sZ[w][pp] = silu((float)zg[(int64_t)(t0 + w) * P + pp]);
+#pragma unroll
+    for (int u = 0; u < VN; ++u) {
+      const int i = tid + u * NT, w = i / PP, pp = i % PP;
+      if (w < wn) {
+        sV[(t0 + w) & (W2 - 1)][pp] = (float)rv[u];
+        if (zg) sZ[w][pp] = silu((float)rz[u]);
+      }
     }
     if (tid < wn) {
-      const float adt = adtg[t0 + tid], dt = dtg[t0 + tid], lam = lamg[t0 + tid];
-      const float alpha = expf(adt);
+      const float alpha = expf(radt);
       sC[tid][0] = alpha;
-      sC[tid][1] = alpha * dt * (1.0f - lam);
-      sC[tid][2] = dt * lam;
-      sC[tid][3] = dt;
+      sC[tid][1] = alpha * rdt * (1.0f - rlam);
+      sC[tid][2] = rdt * rlam;
+      sC[tid][3] = rdt;
     }
-    for (int i = tid; i < wn * H2; i += NT) {
-      const int w = i / H2, j = i % H2;
-      if (j < Nr) sPh[w][j] = tanhf(ag[(int64_t)(t0 + w) * Nr + j]) * kPi;
+    if (Nr > 0) {
+#pragma unroll
+      for (int u = 0; u < AN; ++u) {
+        int w, j;
+        by_nr(tid + u * NT, w, j);
+        if (w < wn) sPh[w][j] = tanhf(rang[u]) * kPi;
+      }
     }
     __syncthreads();
     // ---- phi, one serial chain per angle ---------------------------------------------
@@ -448,22 +528,41 @@ decode_scan_kernel(const DecScanParams p) {
       }
     }
     __syncthreads();
+    // ---- its sines and cosines, spread over all threads ------------------------------
+    if (Nr > 0) {
+#pragma unroll
+      for (int u = 0; u < AN; ++u) {
+        int w, j;
+        by_nr(tid + u * NT, w, j);
+        if (w < wn) {
+          float sn, cs;
+          sincosf(sPh[w][j], &sn, &cs);
+          sSn[w][j] = sn;
+          sPh[w][j] = cs;
+        }
+      }
+      __syncthreads();
+    }
     // ---- rotated q~ / k~ of the window -----------------------------------------------
-    for (int w = wr; w < wn; w += NT / H2) {
-      const int64_t t = t0 + w;
-      const float ulo = (float)qg[t * N + jr] + qbl;
-      const float uhi = (float)qg[t * N + H2 + jr] + qbh;
-      const float wlo = (float)kg[t * N + jr] + kbl;
-      const float whi = (float)kg[t * N + H2 + jr] + kbh;
-      float sn = 0.f, cs = 1.f;
-      if (jr < Nr) sincosf(sPh[w][jr], &sn, &cs);
-      sQ[w][jr] = (MT)rot_lo(ulo, uhi, cs, sn);
-      sQ[w][H2 + jr] = (MT)rot_hi(ulo, uhi, cs, sn);
-      sK[t & (W2 - 1)][jr] = rot_lo(wlo, whi, cs, sn);
-      sK[t & (W2 - 1)][H2 + jr] = rot_hi(wlo, whi, cs, sn);
+#pragma unroll
+    for (int u = 0; u < RN; ++u) {
+      const int w = wr + u * (NT / H2), t = t0 + w;
+      if (w < wn) {
+        const float ulo = (float)rql[u] + qbl, uhi = (float)rqh[u] + qbh;
+        const float wlo = (float)rkl[u] + kbl, whi = (float)rkh[u] + kbh;
+        const float sn = jr < Nr ? sSn[w][jr] : 0.f, cs = jr < Nr ? sPh[w][jr] : 1.f;
+        sQ[w][jr] = (MT)rot_lo(ulo, uhi, cs, sn);
+        sQ[w][H2 + jr] = (MT)rot_hi(ulo, uhi, cs, sn);
+        sK[t & (W2 - 1)][jr] = rot_lo(wlo, whi, cs, sn);
+        sK[t & (W2 - 1)][H2 + jr] = rot_hi(wlo, whi, cs, sn);
+      }
     }
     __syncthreads();
+    if (AHEAD) fetch(t0 + W);
     // ---- the window's steps: update + readout, no barrier between them ---------------
+    // (a part has one or two rows a thread: four steps at once hide their LDS reads and the
+    // readouts' exchange chains)
+#pragma unroll(PARTS > 1 ? 4 : 1)
     for (int w = 0; w < wn; ++w) {
       const int t = t0 + w;
       const int sc = t & (W2 - 1), sp = (t - 1) & (W2 - 1);
@@ -487,49 +586,93 @@ decode_scan_kernel(const DecScanParams p) {
       } else {
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
-          const int prow = g * IT + it < P ? g * IT + it : 0;
+          const int prow = g * IT + it < PP ? g * IT + it : 0;
           vp[it] = sV[sp][prow];
           vc[it] = sV[sc][prow];
         }
       }
-      float part[IT];
+      float part_y[IT];
 #pragma unroll
       for (int it = 0; it < IT; ++it) {
         const float bvp = cf[1] * vp[it];
         const float gv = cf[2] * vc[it];
 #pragma unroll
         for (int i = 0; i < 4; ++i) st[it][i] = state_step(st[it][i], cf[0], bvp, kp[i], gv, kt[i]);
-        part[it] = readout4<MT>(st[it], qt);
+        part_y[it] = readout4<MT>(st[it], qt);
       }
-      rows_reduce_scatter<RV, IT>(part, lane);
+      rows_reduce_scatter<RV, IT>(part_y, lane);
       const int prow = g * IT + (lane >> LO);
-      if ((lane & ((1 << LO) - 1)) == 0 && prow < P) {
-        float yv = fmaf(dsk, sV[sc][prow], part[0]);
+      if ((lane & ((1 << LO) - 1)) == 0 && prow < PP) {
+        float yv = fmaf(dsk, sV[sc][prow], part_y[0]);
         if (zg) yv *= sZ[w][prow];
         sY[w][prow] = (MT)yv;
       }
     }
     __syncthreads();
-    // ---- the window's y, as contiguous 16-byte stores ---------------------------------
-    const int nv = wn == W ? YV : wn * P * (int)sizeof(MT) / 16;
-    for (int i = tid; i < nv; i += NT)
-      reinterpret_cast<uint4*>(yb + (int64_t)t0 * P * sizeof(MT))[i] =
-          reinterpret_cast<const uint4*>(&sY[0][0])[i];
+    // ---- the window's y, as 16-byte stores (contiguous where one workgroup has all rows) --
+    if constexpr (PARTS == 1) {
+      for (int i = tid; i < wn * PP * (int)sizeof(MT) / 16; i += NT)
+        reinterpret_cast<uint4*>(yb + (int64_t)t0 * P * sizeof(MT))[i] =
+            reinterpret_cast<const uint4*>(&sY[0][0])[i];
+    } else {
+      for (int i = tid; i < wn * YR; i += NT)
+        reinterpret_cast<uint4*>(yb + (int64_t)(t0 + i / YR) * P * sizeof(MT))[i % YR] =
+            reinterpret_cast<const uint4*>(&sY[0][0])[i];
+    }
   }
   // ---- write back: the state, the last step's (k~, v) pair and phi -------------------
 #pragma unroll
   for (int it = 0; it < IT; ++it)
-    if (g * IT + it < P) sg[(g * IT + it) * RV + lane] = st[it];
+    if (g * IT + it < PP) sg[(g * IT + it) * RV + lane] = st[it];
   const int sl = (T - 1) & (W2 - 1);
-  for (int i = tid; i < N; i += NT) p.kst[bh * N + i] = sK[sl][i];
-  for (int i = tid; i < P; i += NT) p.vst[bh * P + i] = sV[sl][i];
-  if (tid < Nr) p.phist[bh * Nr + tid] = ph;
+  for (int i = tid; i < PP; i += NT) p.vst[bh * P + row0 + i] = sV[sl][i];
+  float* kout = PARTS > 1 ? p.carry + bh * (N + Nr) : p.kst + bh * N;
+  float* pout = PARTS > 1 ? p.carry + bh * (N + Nr) + N : p.phist + bh * Nr;
+  if (part == 0) {
+    for (int i = tid; i < N; i += NT) kout[i] = sK[sl][i];
+    if (tid < Nr) pout[tid] = ph;
+  }
+}
+
+// The k~ and phi that a run in parts left in `carry`, into the state: one thread an entry.
+__global__ void __launch_bounds__(256) dec_carry_kernel(const float* carry, float* kst, float* phist,
+                                                        int N, int Nr, int64_t total) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const int64_t bh = i / (N + Nr);
+  const int j = (int)(i - bh * (N + Nr));
+  if (j < N) kst[bh * N + j] = carry[i];
+  else phist[bh * Nr + j - N] = carry[i];
+}
+
+// Parts of a run: 8, or 4, of a 64-row state, as keep the launch within four workgroups per
+// CU (two parts at 512 states were 2% slower than none), and only for runs of two windows,
+// from where the copy of the carry pays.
+static int dec_scan_parts(int64_t states, int steps, int n, int pdim) {
+  if (pdim != 64 || n > 128 || steps < 32) return 1;
+  return states <= 128 ? 8 : states <= 256 ? 4 : 1;
+}
+
+template <typename MT, int N, int P, int PARTS>
+static int32_t launch_dec_parts(const DecScanParams& prm, int grid, hipStream_t stream) {
+  hipLaunchKernelGGL((decode_scan_kernel<MT, N, P, PARTS>), dim3(grid * PARTS), dim3(kDecThreads), 0,
+                     stream, prm);
+  if constexpr (PARTS > 1) {
+    const int64_t total = (int64_t)grid * (N + prm.Nr);
+    hipLaunchKernelGGL(dec_carry_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream,
+                       prm.carry, prm.kst, prm.phist, N, prm.Nr, total);
+  }
+  return launch_status("m3s_decode_scan");
 }
 
 template <typename MT, int N, int P>
 static int32_t launch_dec_scan(const DecScanParams& prm, int grid, hipStream_t stream) {
-  hipLaunchKernelGGL((decode_scan_kernel<MT, N, P>), dim3(grid), dim3(kDecThreads), 0, stream, prm);
-  return launch_status("m3s_decode_scan");
+  const int parts = prm.carry ? dec_scan_parts(grid, prm.T, N, P) : 1;
+  if constexpr (P == 64 && N <= 128) {
+    if (parts == 8) return launch_dec_parts<MT, N, P, 8>(prm, grid, stream);
+    if (parts == 4) return launch_dec_parts<MT, N, P, 4>(prm, grid, stream);
+  }
+  return launch_dec_parts<MT, N, P, 1>(prm, grid, stream);
 }
 
 template <typename MT, int N, int P, bool LAYER>
@@ -647,7 +790,20 @@ extern "C" int32_t m3s_decode_layer(const m3s_decode_layer_args* a, void* stream
   return M3S_ERR_UNSUPPORTED;
 }
 
+extern "C" int64_t m3s_decode_scan_workspace_bytes(int32_t batch, int32_t steps, int32_t nheads,
+                                                   int32_t headdim, int32_t state_dim,
+                                                   int32_t n_angles) {
+  if (batch <= 0 || steps <= 0 || nheads <= 0 || headdim <= 0 || state_dim <= 0 || n_angles < 0) return -1;
+  const int64_t states = (int64_t)batch * nheads;
+  return m3s::dec_scan_parts(states, steps, state_dim, headdim) > 1 ? states * (state_dim + n_angles) * 4 : 0;
+}
+
 extern "C" int32_t m3s_decode_scan(const m3s_decode_scan_args* a, void* stream) {
+  return m3s_decode_scan_ws(a, nullptr, 0, stream);
+}
+
+extern "C" int32_t m3s_decode_scan_ws(const m3s_decode_scan_args* a, void* workspace,
+                                      int64_t workspace_bytes, void* stream) {
   using namespace m3s;
   clear_error();
   M3S_REQUIRE(a != nullptr, "m3s_decode_scan: args is NULL");
@@ -675,7 +831,12 @@ extern "C" int32_t m3s_decode_scan(const m3s_decode_scan_args* a, void* stream) 
               "m3s_decode_scan: state/output pointers NULL, or ssm / y not 16-byte aligned");
   M3S_REQUIRE((int64_t)B * H < (1ll << 31) && (int64_t)B * H * T * (P > N ? P : N) < (1ll << 40),
               "m3s_decode_scan: B*H or B*H*T too large");
+  const int64_t need = m3s_decode_scan_workspace_bytes(B, T, H, P, N, Nr);
+  M3S_REQUIRE(workspace == nullptr || (aligned16(workspace) && workspace_bytes >= need),
+              "m3s_decode_scan: workspace misaligned or smaller than the %lld bytes of this run",
+              (long long)need);
   DecScanParams prm{};
+  prm.carry = need > 0 ? static_cast<float*>(workspace) : nullptr;
   prm.B = B; prm.H = H; prm.Nr = Nr; prm.T = T; prm.has_d = a->has_d; prm.has_z = a->has_z;
   prm.q = a->q; prm.k = a->k; prm.v = a->v; prm.z = a->z;
   prm.adt = a->adt; prm.dt = a->dt; prm.lam = a->lam; prm.angles = a->angles;

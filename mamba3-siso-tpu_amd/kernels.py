@@ -650,7 +650,11 @@ def decode_scan(q, k, v, adt, dt, lam, angles, q_bias, k_bias, state, d_skip=Non
     a.q_bias, a.k_bias, a.d_skip = qb_c.data_ptr(), kb_c.data_ptr(), _lib.ptr(d_c)
     a.ssm, a.k_state, a.v_state, a.phi_state = (t.data_ptr() for t in (ssm_k, kst_k, vst_k, phist_k))
     a.y = y.data_ptr()
-    _lib.launch(_lib.load().m3s_decode_scan, a, dev, "m3s_decode_scan")
+    lib = _lib.load()
+    nbytes = lib.m3s_decode_scan_workspace_bytes(batch, steps, a.nheads, width, state_dim, n_angles)
+    ws = empty(nbytes, device=dev, dtype=torch.uint8) if nbytes > 0 else None
+    _lib.launch(lambda args, stream: lib.m3s_decode_scan_ws(args, _lib.ptr(ws), max(nbytes, 0), stream),
+                a, dev, "m3s_decode_scan")
     if r > 1:
         kst.copy_(kst_k[:, ::r])
         phist.copy_(phist_k[:, ::r])

@@ -294,3 +294,36 @@ def test_decode_scan_of_no_steps_keeps_the_state(m3):
     assert_same_run(m3.decode_scan(*args, s1, d_skip=d["d_skip"], z=d["z"]),
                     m3.kernels.decode_loop(*args, dev_state(st), d_skip=d["d_skip"], z=d["z"]),
                     "after an empty run")
+
+
+@pytest.mark.parametrize("policy,b,h,T,n,p,nr,gated", [
+    ("bf16", 1, 1, 32, 128, 64, 32, True),       # the fewest steps and states that are split
+    ("bf16", 1, 128, 47, 128, 64, 32, True),     # the most for eight parts
+    ("bf16", 3, 43, 33, 128, 64, 6, False),      # the fewest for four
+    ("bf16", 2, 128, 48, 64, 64, 16, True),      # the most
+    ("bf16", 2, 3, 40, 128, 128, 64, True),      # sub-heads
+    ("f32", 1, 5, 37, 128, 64, 32, True),
+    ("f32", 1, 130, 34, 64, 64, 0, True),
+])
+def test_decode_scan_in_parts_bit_for_bit(m3, monkeypatch, policy, b, h, T, n, p, nr, gated):
+    """A run whose states are split by rows over workgroups (``m3s_decode_scan_ws`` with its
+    workspace) against the same run with one workgroup per state."""
+    _, d, st = chain_inputs(b, h, T, n, p, nr, policy, seed=T)
+    z, dsk = (d["z"], d["d_skip"]) if gated else (None, None)
+    args = (d["q"], d["k"], d["v"], d["adt"], d["dt"], d["lam"], d["angles"], d["q_bias"], d["k_bias"])
+    lib = m3._lib.load()
+    assert lib.m3s_decode_scan_workspace_bytes(b, T, h * (p // 64), 64, n, nr) > 0, "not split"
+    got = m3.decode_scan(*args, dev_state(st), dsk, z, dtype_policy=policy)
+    launch = m3._lib.launch
+    monkeypatch.setattr(m3._lib, "launch", lambda fn, a, dev, what: launch(lib.m3s_decode_scan, a, dev, what))
+    ref = m3.decode_scan(*args, dev_state(st), dsk, z, dtype_policy=policy)
+    assert_same_run(got, ref, f"{policy} B={b} H={h} T={T}")
+
+
+def test_decode_scan_parts_need_their_workspace(m3):
+    lib = m3._lib.load()
+    size = lib.m3s_decode_scan_workspace_bytes
+    assert size(1, 512, 32, 64, 128, 32) == 32 * (128 + 32) * 4
+    assert size(1, 31, 32, 64, 128, 32) == 0 and size(1, 512, 257, 64, 128, 32) == 0
+    assert size(1, 512, 32, 16, 32, 8) == 0 and size(1, 512, 32, 64, 256, 64) == 0
+    assert size(0, 512, 32, 64, 128, 32) == -1
