@@ -573,6 +573,28 @@ int64_t m3s_wgrad_workspace_bytes(int32_t tokens, int32_t rows, int32_t cols);
 int32_t m3s_wgrad(const m3s_wgrad_args* args, void* stream);
 int32_t m3s_gemv(const m3s_gemv_args* args, void* stream);
 
+/* m3s_gemv for one or two rows with the pass before it folded in, for the decode step of the LM
+ * (model.py:266-296). NORM: y = bf16(rms_norm(x + add, gain)) w, x the residual stream, and
+ * `sum` receives x + add in the stream's dtype when add is given (as m3s_rms_fwd). GATE: y =
+ * (value silu(gate)) w with x = value | gate, (rows, 2 k) bf16. HEAD: the norm, then the tied
+ * head, y (rows, n) float32 = bf16(norm) . bf16(w[v]) with w the (n, k) embedding in w_dtype.
+ * All tensors dense; k <= 1024 and a multiple of 4 with a norm. */
+enum { M3S_GEMV_NORM = 1, M3S_GEMV_GATE = 2, M3S_GEMV_HEAD = 3 };
+typedef struct m3s_gemv_fused_args {
+  int32_t struct_size;  /* sizeof(m3s_gemv_fused_args) */
+  int32_t rows, k, n;
+  int32_t mode;         /* M3S_GEMV_* */
+  int32_t x_dtype, w_dtype;
+  float eps;
+  const void* x;        /* (rows, k) stream, or (rows, 2 k) bf16 */
+  const void* add;      /* (rows, k) bf16, or NULL */
+  const float* gain;    /* (k) */
+  void* sum;            /* out (rows, k) in x_dtype, not x itself */
+  const void* w;        /* (k, n) bf16, or the (n, k) table */
+  void* y;              /* out (rows, n) bf16, or float32 */
+} m3s_gemv_fused_args;
+int32_t m3s_gemv_fused(const m3s_gemv_fused_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

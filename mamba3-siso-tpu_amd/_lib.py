@@ -216,6 +216,17 @@ class GemvArgs(C.Structure):
     ]
 
 
+class GemvFusedArgs(C.Structure):
+    _fields_ = [
+        ("struct_size", i32), ("rows", i32), ("k", i32), ("n", i32), ("mode", i32),
+        ("x_dtype", i32), ("w_dtype", i32), ("eps", C.c_float),
+        ("x", vp), ("add", vp), ("gain", vp), ("sum", vp), ("w", vp), ("y", vp),
+    ]
+
+
+#: ``M3S_GEMV_*``
+GEMV_NORM, GEMV_GATE, GEMV_HEAD = 1, 2, 3
+
 #: Every symbol ``include/m3s.h`` declares.
 EXPORTS = ("m3s_abi_version", "m3s_last_error", "m3s_supported", "m3s_fwd_raw_supported",
            "m3s_bwd_workspace_bytes",
@@ -225,7 +236,8 @@ EXPORTS = ("m3s_abi_version", "m3s_last_error", "m3s_supported", "m3s_fwd_raw_su
            "m3s_prep_fwd", "m3s_prep_bwd", "m3s_norm_bwd_workspace_bytes", "m3s_norm_fwd",
            "m3s_norm_bwd", "m3s_decode_layer", "m3s_transpose", "m3s_swiglu_fwd",
            "m3s_swiglu_bwd", "m3s_rms_fwd", "m3s_rms_bwd", "m3s_rms_bwd_workspace_bytes",
-           "m3s_norm_bwd_noalloc", "m3s_adamw", "m3s_wgrad", "m3s_wgrad_workspace_bytes", "m3s_gemv")
+           "m3s_norm_bwd_noalloc", "m3s_adamw", "m3s_wgrad", "m3s_wgrad_workspace_bytes", "m3s_gemv",
+           "m3s_gemv_fused")
 
 _lib = None
 
@@ -302,6 +314,8 @@ def load(path: str = LIB_PATH) -> C.CDLL:
     lib.m3s_wgrad_workspace_bytes.argtypes = [i32, i32, i32]
     lib.m3s_gemv.restype = i32
     lib.m3s_gemv.argtypes = [C.POINTER(GemvArgs), vp]
+    lib.m3s_gemv_fused.restype = i32
+    lib.m3s_gemv_fused.argtypes = [C.POINTER(GemvFusedArgs), vp]
     ver = lib.m3s_abi_version()
     if ver != ABI_VERSION:
         raise RuntimeError(f"{path} has ABI version {ver}, expected {ABI_VERSION}; rebuild it")

@@ -12,6 +12,8 @@
 // lane r reads rows r, r + RL, ... . TN is chosen on the host so that the launch has at
 // least 128 workgroups. Sums over the row lanes: xor shuffles inside a wave (a fixed
 // tree), then the four waves' partials added in wave order through LDS. Deterministic.
+#include <type_traits>
+
 #include "m3s_common.h"
 #include "m3s_internal.h"
 
@@ -27,10 +29,67 @@ struct GvParams {
   bf16* y;
   int M, K, N;
   int64_t ldx, ldw, ldy;
+  // the fused products (gemv_kernel's PRO): the residual stream, the block output to add to
+  // it, the norm's gain and epsilon, and where the sum goes
+  const void* stream;
+  const bf16* add;
+  const float* gain;
+  void* sum;
+  float eps;
 };
 
-template <int CL, int NL>
+// What a product's x is made of on the way in, one or two rows of it: kPlain, the bf16 rows;
+// kNorm32 / kNorm16, the block norm of a float32 / bf16 residual stream plus a block output
+// (m3s_rms_fwd's arithmetic, rounded to bf16 as it stores it); kGate, value silu(gate) of the
+// fc1 product (m3s_swiglu_fwd's). Every workgroup makes x for itself under its weight loads:
+// at one row a launch of its own for the norm (4.8 us in a recorded step) or the gate (4.4)
+// costs as much as the product.
+enum GvPro { kPlain, kNorm32, kNorm16, kGate };
+
+template <typename T> __device__ __forceinline__ f32x4 ld_stream4(const T* q);
+template <> __device__ __forceinline__ f32x4 ld_stream4<float>(const float* q) {
+  return *reinterpret_cast<const f32x4*>(q);
+}
+template <> __device__ __forceinline__ f32x4 ld_stream4<bf16>(const bf16* q) {
+  return sub_to_f32<bf16>(*reinterpret_cast<const bf16x4*>(q));
+}
+
+// One wave's copy of a normalised row: lane l holds columns 4 l + 256 k (k < NP; D <= 256 NP),
+// s = x + add rounded to the stream's type, and returns 1 / rms(s). The sum's order is
+// m3s_rms_fwd's.
+template <typename TX, int NP>
+__device__ __forceinline__ float norm_row(const TX* x, const bf16* add, int D, float eps, int lane,
+                                          f32x4 (&v)[NP]) {
+#pragma unroll
+  for (int k = 0; k < NP; ++k) {
+    const int c = 4 * lane + 256 * k;
+    v[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (c < D) {
+      v[k] = ld_stream4<TX>(x + c);
+      if (add) {
+        const f32x4 d = ld_stream4<bf16>(add + c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[k][i] = (float)(TX)(v[k][i] + d[i]);
+      }
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < NP; ++k) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ss += v[k][i] * v[k][i];
+  }
+  return 1.f / sqrtf(wave_total(ss) / (float)D + eps);
+}
+
+constexpr int kGvNormPieces = 4;                      // rows up to 1024 wide
+constexpr int kGvNormMax = 256 * kGvNormPieces;
+
+template <int CL, int NL, int PRO>
 __global__ void __launch_bounds__(kGvThreads) gemv_kernel(const GvParams p) {
+  constexpr bool NORM = PRO == kNorm32 || PRO == kNorm16;
+  using TX = std::conditional_t<PRO == kNorm16, bf16, float>;
+  __shared__ __align__(16) float sx[NORM ? 2 * kGvNormMax : 4];
   constexpr int RL = kGvThreads / CL;   // row lanes
   constexpr int TN = 8 * CL;
   __shared__ float part[kGvThreads / 64][kGvMaxRows][TN];
@@ -46,6 +105,41 @@ __global__ void __launch_bounds__(kGvThreads) gemv_kernel(const GvParams p) {
     wv[i] = (col_ok && k < p.K) ? *reinterpret_cast<const bf16x8*>(p.w + (int64_t)k * p.ldw + n)
                                 : bf16x8{};
   }
+  if constexpr (NORM) {   // wave m normalises row m for the workgroup
+    if (wave < p.M) {
+      f32x4 v[kGvNormPieces];
+      const TX* xr = static_cast<const TX*>(p.stream) + (int64_t)wave * p.K;
+      const float rs = norm_row<TX, kGvNormPieces>(
+          xr, p.add ? p.add + (int64_t)wave * p.K : nullptr, p.K, p.eps, lane, v);
+#pragma unroll
+      for (int k = 0; k < kGvNormPieces; ++k) {
+        const int c = 4 * lane + 256 * k;
+        if (c < p.K) {
+          const f32x4 g = *reinterpret_cast<const f32x4*>(p.gain + c);
+          f32x4 o;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = (float)(bf16)(v[k][i] * rs * g[i]);
+          *reinterpret_cast<f32x4*>(sx + wave * kGvNormMax + c) = o;
+          if (blockIdx.x == 0 && p.add) {
+            TX* so = static_cast<TX*>(p.sum) + (int64_t)wave * p.K + c;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) so[i] = (TX)v[k][i];
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+  // x[m][k]
+  auto xval = [&](int m, int k) {
+    if constexpr (NORM) return sx[m * kGvNormMax + k];
+    const bf16* xr = p.x + m * p.ldx;
+    if constexpr (PRO == kGate) {
+      const float g = (float)xr[p.K + k];
+      return (float)(bf16)((float)xr[k] * (float)(bf16)(g / (1.f + expf(-g))));
+    }
+    return (float)xr[k];
+  };
   float acc[kGvMaxRows][8];
 #pragma unroll
   for (int m = 0; m < kGvMaxRows; ++m) {
@@ -58,7 +152,7 @@ __global__ void __launch_bounds__(kGvThreads) gemv_kernel(const GvParams p) {
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int k = rl + i * RL;
-      const float xv = k < p.K ? (float)p.x[m * p.ldx + k] : 0.f;
+      const float xv = k < p.K ? xval(m, k) : 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[m][j] = fmaf(xv, (float)wv[i][j], acc[m][j]);
     }
@@ -106,14 +200,14 @@ inline int gemv_col_lanes(int K, int N) {
   return cl;
 }
 
-template <int CL>
+template <int CL, int PRO>
 int32_t gemv_launch(const GvParams& p, hipStream_t s) {
   constexpr int RL = kGvThreads / CL;
   const int nl = (p.K + RL - 1) / RL;
   const dim3 grid((unsigned)((p.N + 8 * CL - 1) / (8 * CL)));
 #define M3S_GV(NL)                                                                \
   if (nl <= NL) {                                                                 \
-    hipLaunchKernelGGL((gemv_kernel<CL, NL>), grid, dim3(kGvThreads), 0, s, p);   \
+    hipLaunchKernelGGL((gemv_kernel<CL, NL, PRO>), grid, dim3(kGvThreads), 0, s, p);   \
     return launch_status("m3s_gemv");                                             \
   }
   M3S_GV(2) M3S_GV(4) M3S_GV(8) M3S_GV(16)
@@ -257,6 +351,52 @@ int32_t gemm_rows_launch(GmParams p, hipStream_t s) {
   return launch_status("m3s_gemv");
 }
 
+template <int PRO>
+int32_t gemv_dispatch(const GvParams& p, hipStream_t s) {
+  switch (gemv_col_lanes(p.K, p.N)) {
+    case 8: return gemv_launch<8, PRO>(p, s);
+    case 4: return gemv_launch<4, PRO>(p, s);
+    case 2: return gemv_launch<2, PRO>(p, s);
+    default: return gemv_launch<1, PRO>(p, s);
+  }
+}
+
+// The head of a decode step: logits[m][v] = bf16(norm(x_m + add_m)) . bf16(table[v]), float32
+// sums and output, for a tied (vocab, D) embedding. One wave per vocabulary row, which
+// normalises x for itself; lane l holds columns 4 l + 256 k of both. The composed head cast
+// the whole table twice and ran a float32 library product, 35 us of the byte LM's step.
+template <typename TX, typename TE>
+__global__ void __launch_bounds__(256) head_kernel(const GvParams p, const TE* table, float* out) {
+  const int lane = threadIdx.x & 63, D = p.K;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= p.N) return;
+  f32x4 e[kGvNormPieces];
+#pragma unroll
+  for (int k = 0; k < kGvNormPieces; ++k) {
+    const int c = 4 * lane + 256 * k;
+    e[k] = c < D ? ld_stream4<TE>(table + (int64_t)row * D + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int m = 0; m < p.M; ++m) {
+    f32x4 v[kGvNormPieces];
+    const float rs = norm_row<TX, kGvNormPieces>(
+        static_cast<const TX*>(p.stream) + (int64_t)m * D, p.add ? p.add + (int64_t)m * D : nullptr,
+        D, p.eps, lane, v);
+    float acc = 0.f;
+#pragma unroll
+    for (int k = 0; k < kGvNormPieces; ++k) {
+      const int c = 4 * lane + 256 * k;
+      if (c < D) {
+        const f32x4 g = *reinterpret_cast<const f32x4*>(p.gain + c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc = fmaf((float)(bf16)(v[k][i] * rs * g[i]), (float)(bf16)e[k][i], acc);
+      }
+    }
+    acc = wave_total(acc);
+    if (lane == 0) out[(int64_t)m * p.N + row] = acc;
+  }
+}
+
 }  // namespace m3s
 
 extern "C" int32_t m3s_gemv(const m3s_gemv_args* a, void* stream) {
@@ -291,14 +431,63 @@ extern "C" int32_t m3s_gemv(const m3s_gemv_args* a, void* stream) {
     if (t64 >= 128) return gemm_rows_launch<64, 4>(g, s);
     return gemm_rows_launch<32, 4>(g, s);
   }
-  GvParams p{static_cast<const bf16*>(a->x), static_cast<const bf16*>(a->w),
-             static_cast<bf16*>(a->y), a->rows, a->k, a->n, a->ldx, a->ldw, a->ldy};
+  GvParams p{};
+  p.x = static_cast<const bf16*>(a->x); p.w = static_cast<const bf16*>(a->w);
+  p.y = static_cast<bf16*>(a->y);
+  p.M = a->rows; p.K = a->k; p.N = a->n; p.ldx = a->ldx; p.ldw = a->ldw; p.ldy = a->ldy;
   M3S_REQUIRE(a->k <= kGvThreads * kGvMaxLoads, "m3s_gemv: k %d > %d", a->k,
               kGvThreads * kGvMaxLoads);
-  switch (gemv_col_lanes(a->k, a->n)) {
-    case 8: return gemv_launch<8>(p, s);
-    case 4: return gemv_launch<4>(p, s);
-    case 2: return gemv_launch<2>(p, s);
-    default: return gemv_launch<1>(p, s);
+  return gemv_dispatch<kPlain>(p, s);
+}
+
+extern "C" int32_t m3s_gemv_fused(const m3s_gemv_fused_args* a, void* stream) {
+  using namespace m3s;
+  clear_error();
+  M3S_REQUIRE(a != nullptr, "m3s_gemv_fused: args is NULL");
+  M3S_REQUIRE(a->struct_size == (int32_t)sizeof(m3s_gemv_fused_args),
+              "m3s_gemv_fused: struct_size %d != %d (ABI mismatch)", a->struct_size,
+              (int)sizeof(m3s_gemv_fused_args));
+  M3S_REQUIRE(a->rows >= 1 && a->rows <= 2, "m3s_gemv_fused: rows %d not 1 or 2", a->rows);
+  M3S_REQUIRE(a->k > 0 && a->n > 0 && a->x && a->w && a->y, "m3s_gemv_fused: a bad size or NULL operand");
+  M3S_REQUIRE(a->mode >= M3S_GEMV_NORM && a->mode <= M3S_GEMV_HEAD, "m3s_gemv_fused: bad mode %d", a->mode);
+  M3S_REQUIRE(a->x_dtype == M3S_DTYPE_F32 || a->x_dtype == M3S_DTYPE_BF16, "m3s_gemv_fused: bad x_dtype");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  GvParams p{};
+  p.w = static_cast<const bf16*>(a->w); p.y = static_cast<bf16*>(a->y);
+  p.M = a->rows; p.K = a->k; p.N = a->n; p.ldx = 2 * (int64_t)a->k; p.ldw = a->n; p.ldy = a->n;
+  if (a->mode == M3S_GEMV_GATE) {
+    M3S_REQUIRE(a->x_dtype == M3S_DTYPE_BF16, "m3s_gemv_fused: the gate reads bf16");
+    p.x = static_cast<const bf16*>(a->x);
+  } else {
+    M3S_REQUIRE(a->k % 4 == 0 && a->k <= kGvNormMax, "m3s_gemv_fused: k %d is not a multiple of 4 up to %d",
+                a->k, kGvNormMax);
+    M3S_REQUIRE(a->gain && aligned16(a->x) && aligned16(a->gain) && (!a->add || aligned16(a->add)),
+                "m3s_gemv_fused: stream, gain or add NULL or misaligned");
+    M3S_REQUIRE(a->mode == M3S_GEMV_HEAD || !a->add || a->sum, "m3s_gemv_fused: add without sum");
+    p.stream = a->x; p.add = static_cast<const bf16*>(a->add); p.gain = a->gain; p.sum = a->sum;
+    p.eps = a->eps;
   }
+  const bool x32 = a->x_dtype == M3S_DTYPE_F32;
+  if (a->mode == M3S_GEMV_HEAD) {
+    M3S_REQUIRE(aligned16(a->w), "m3s_gemv_fused: the table is misaligned");
+    const dim3 grid((unsigned)((a->n + 3) / 4));
+    float* out = static_cast<float*>(a->y);
+#define M3S_HEAD(TX, TE) \
+    hipLaunchKernelGGL((head_kernel<TX, TE>), grid, dim3(256), 0, s, p, static_cast<const TE*>(a->w), out)
+    if (a->w_dtype == M3S_DTYPE_F32) {
+      if (x32) M3S_HEAD(float, float);
+      else M3S_HEAD(bf16, float);
+    } else {
+      if (x32) M3S_HEAD(float, bf16);
+      else M3S_HEAD(bf16, bf16);
+    }
+#undef M3S_HEAD
+    return launch_status("m3s_gemv_fused (head)");
+  }
+  M3S_REQUIRE(a->w_dtype == M3S_DTYPE_BF16 && aligned16(a->w) && a->n % 8 == 0,
+              "m3s_gemv_fused: w must be dense bf16, 16-byte aligned, n a multiple of 8");
+  M3S_REQUIRE(a->k <= kGvThreads * kGvMaxLoads, "m3s_gemv_fused: k %d > %d", a->k,
+              kGvThreads * kGvMaxLoads);
+  if (a->mode == M3S_GEMV_GATE) return gemv_dispatch<kGate>(p, s);
+  return x32 ? gemv_dispatch<kNorm32>(p, s) : gemv_dispatch<kNorm16>(p, s);
 }

@@ -1172,6 +1172,56 @@ def matmul(x: Tensor, w: Tensor) -> Tensor:
     return x @ w
 
 
+#: Rows and widths of the products with a norm or the gate folded in (``m3s_gemv_fused``).
+FUSED_ROWS_MAX, FUSED_NORM_MAX = 2, 1024
+
+
+def _gemv_fused(mode: int, x: Tensor, w: Tensor, k: int, n: int, out_dtype: torch.dtype,
+                add: Optional[Tensor] = None, gain: Optional[Tensor] = None, eps: float = 0.0):
+    rows = x.shape[0]
+    tensors = [t for t in (x, w, add, gain) if t is not None]
+    dev = _device_of(*tensors)
+    if (not 1 <= rows <= FUSED_ROWS_MAX or not all(t.is_contiguous() for t in tensors)
+            or (add is not None and (add.dtype != torch.bfloat16 or add.shape != x.shape))
+            or (gain is not None and (gain.dtype != torch.float32 or gain.shape != (k,)))):
+        raise ValueError("gemv_fused: one or two dense rows, add in bf16 like x, gain (k,) float32")
+    y = empty(rows, n, device=dev, dtype=out_dtype)
+    total = x
+    a = _lib.GemvFusedArgs()
+    a.struct_size = ctypes.sizeof(_lib.GemvFusedArgs)
+    a.rows, a.k, a.n, a.mode, a.eps = rows, k, n, mode, float(eps)
+    a.x_dtype, a.w_dtype = _lib.dtype_code(x.dtype), _lib.dtype_code(w.dtype)
+    a.x, a.w, a.y = x.data_ptr(), w.data_ptr(), y.data_ptr()
+    a.add, a.gain = _lib.ptr(add), _lib.ptr(gain)
+    if add is not None and mode == _lib.GEMV_NORM:
+        total = empty_like(x)
+        a.sum = total.data_ptr()
+    _lib.launch(_lib.load().m3s_gemv_fused, a, dev, "m3s_gemv_fused")
+    return y, total
+
+
+def gemv_norm(x: Tensor, add: Optional[Tensor], gain: Tensor, eps: float, w: Tensor):
+    """``s = x + add`` and ``bf16(rms_norm(s, gain)) @ w`` in one launch, for the one or two
+    rows of a decode step: `rms_forward` and `gemv` with their roundings. ``x`` is the
+    residual stream (float32 or bf16), ``add`` a bf16 block output or None. Returns
+    ``(product, s)``."""
+    return _gemv_fused(_lib.GEMV_NORM, x, w, w.shape[0], w.shape[1], torch.bfloat16, add, gain, eps)
+
+
+def gemv_gate(h: Tensor, w: Tensor) -> Tensor:
+    """`swiglu_forward` of ``h`` = value | gate, then ``@ w``, in one launch (one or two rows)."""
+    if h.dtype != torch.bfloat16 or h.shape[1] != 2 * w.shape[0]:
+        raise ValueError("gemv_gate: h must be (rows, 2 k) bf16 for w (k, n)")
+    return _gemv_fused(_lib.GEMV_GATE, h, w, w.shape[0], w.shape[1], torch.bfloat16)[0]
+
+
+def head_logits(x: Tensor, add: Optional[Tensor], gain: Tensor, eps: float, table: Tensor) -> Tensor:
+    """``bf16(rms_norm(x + add, gain)) @ bf16(table).T`` in float32, one launch (one or two
+    rows): the final norm and the tied head of a decode step."""
+    return _gemv_fused(_lib.GEMV_HEAD, x, table, table.shape[1], table.shape[0], torch.float32, add,
+                       gain, eps)[0]
+
+
 def rms_forward(x: Tensor, weight: Tensor, eps: float, out_dtype: torch.dtype,
                 add: Optional[Tensor] = None):
     """LM block norm: ``x`` (..., D) in f32 or bf16 -> ``(y (..., D) in out_dtype, rstd

@@ -387,6 +387,56 @@ def _add_residual(x: Tensor, y: Tensor) -> Tensor:
     return x.to(wide) + y.to(wide)
 
 
+def _decode_fused_ok(params: LMParams, x: Tensor, cfg: LMConfig) -> bool:
+    """Whether a token step folds its norms, gates and head into the products
+    (``m3s_gemv_fused``): one or two rows without autograd, bf16 products, a tied head, widths
+    the kernels take, and dense tensors. Other steps run them one by one."""
+    c, d = cfg.siso, cfg.d_model
+    if (torch.is_grad_enabled() or not x.is_cuda or not 1 <= x.shape[0] <= K.FUSED_ROWS_MAX
+            or _mm_dtype(cfg) != torch.bfloat16 or x.dtype not in (torch.float32, torch.bfloat16)
+            or not cfg.tie_head or d % 8 or d > K.FUSED_NORM_MAX or c.d_in_proj % 8
+            or c.d_inner > 4096 or L.decode_headdim(c.policy_name, c.d_state, c.headdim) != c.headdim
+            or params.embed.dtype != x.dtype or not params.embed.is_contiguous()
+            or params.embed.data_ptr() % 16):
+        return False
+    gains = [params.final_norm]
+    for b in params.blocks:
+        ws = [b.siso.in_proj, b.siso.out_proj]
+        gains.append(b.norm_gain)
+        if b.mlp is not None:
+            ws += b.mlp
+            gains.append(b.mlp_norm_gain)
+            if b.mlp.fc2.shape[0] % 8 or b.mlp.fc2.shape[0] > 4096:
+                return False
+        if not all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0
+                   for w in ws):
+            return False
+    return all(g.dtype == torch.float32 and g.is_contiguous() and g.data_ptr() % 16 == 0
+               for g in gains) and bool(params.blocks)
+
+
+def _decode_step_fused(params: LMParams, x: Tensor, states: list, cfg: LMConfig):
+    """`lm_decode_step` on the embedded rows with five launches a layer instead of eight: each
+    norm with its residual add in the product that reads it, the gate in fc2's, the final norm
+    in the head's."""
+    c, out_states, y = cfg.siso, [], None
+    c.require_kernels()
+    for b, state in zip(params.blocks, states):
+        p = b.siso
+        proj, x = K.gemv_norm(x, y, b.norm_gain, c.norm_eps, p.in_proj)
+        y, st = K.decode_layer_step(
+            proj, state, nheads=c.nheads, headdim=c.headdim, state_dim=c.d_state,
+            n_angles=c.n_angles, b_norm_weight=p.b_norm_weight, c_norm_weight=p.c_norm_weight,
+            dt_bias=p.dt_bias, q_bias=p.c_bias, k_bias=p.b_bias, d_skip=p.d_skip,
+            a_floor=c.a_floor, norm_eps=c.norm_eps)
+        out_states.append(st)
+        y = K.matmul(y.reshape(x.shape[0], c.d_inner), p.out_proj)
+        if b.mlp is not None:
+            h, x = K.gemv_norm(x, y, b.mlp_norm_gain, c.norm_eps, b.mlp.fc1)
+            y = K.gemv_gate(h, b.mlp.fc2)
+    return K.head_logits(x, y, params.final_norm, c.norm_eps, params.embed), out_states
+
+
 def lm_decode_step(params: LMParams, token: Tensor, states: list, cfg: LMConfig,
                    interpret: Any = False):
     """One token through the stack (``model.py:244-296``): ``(B,)`` -> ``((B, vocab)
@@ -397,6 +447,8 @@ def lm_decode_step(params: LMParams, token: Tensor, states: list, cfg: LMConfig,
     c = cfg.siso
     eps = c.norm_eps
     x = _embed(params.embed, token)
+    if token.dim() == 1 and _decode_fused_ok(params, x, cfg):
+        return _decode_step_fused(params, x, states, cfg)
     out_states = []
     blocks = params.blocks
     # as in lm_forward: each residual add fused with the norm that reads the sum next

@@ -341,3 +341,37 @@ def test_released_checkpoint_runs_and_matches_oracle(m3, dev, tmp_path):
     ids = [7, 11, 42]
     out = m3.train.generate(params, cfg, 0, ids, n_tokens=4, rep_penalty=1.0)
     assert out[:3] == ids and len(out) == 7 and all(0 <= t < cfg.vocab_size for t in out)
+
+
+@pytest.mark.parametrize("d,di,vocab,rows,layers,dtype", [
+    (768, 1536, 256, 1, 2, torch.float32), (768, 1536, 256, 2, 2, torch.float32),
+    (1024, 2048, 250, 1, 1, torch.float32), (256, 0, 257, 2, 2, torch.float32),
+    (256, 360, 64, 1, 2, torch.bfloat16), (512, 4096, 256, 1, 1, torch.float32),
+])
+def test_decode_step_with_folded_norms_and_gates(m3, dev, monkeypatch, d, di, vocab, rows, layers, dtype):
+    """The one- and two-row step's folded products against the pass-by-pass step: the norms,
+    gates and products keep their roundings and sum orders, so states are equal bit for bit;
+    the head's float32 sums over d run in another order (d roundings of 2^-24 at most, of terms
+    whose magnitudes add up to at most sqrt(d) times a logit's scale)."""
+    M = m3.model
+    cfg = M.LMConfig(vocab_size=vocab, n_layers=layers, d_intermediate=di,
+                     siso=m3.SISOConfig(d_model=d))
+    gen = torch.Generator().manual_seed(d + rows)
+    params = M.decode_params(M.init_lm(cfg, gen, device=dev), cfg)
+    params = params._replace(embed=params.embed.to(dtype) * 20)
+    states = [M.zero_states(cfg, rows, device=dev) for _ in range(2)]
+    assert torch.is_grad_enabled() and not M._decode_fused_ok(params, params.embed[:rows], cfg)
+    with torch.no_grad():
+        assert M._decode_fused_ok(params, params.embed[:rows], cfg)
+        assert not M._decode_fused_ok(params, params.embed[:3], cfg)
+        for t in range(3):
+            tok = torch.randint(0, vocab, (rows,), generator=gen).to(dev)
+            got, states[0] = M.lm_decode_step(params, tok, states[0], cfg)
+            with monkeypatch.context() as mp:
+                mp.setattr(M, "_decode_fused_ok", lambda *a: False)
+                ref, states[1] = M.lm_decode_step(params, tok, states[1], cfg)
+            for a, b in zip(states[0], states[1]):
+                for x, y in zip(a, b):
+                    assert torch.equal(x, y), t
+            assert got.shape == ref.shape == (rows, vocab) and got.dtype == ref.dtype
+            assert float((got - ref).abs().max()) <= d ** 1.5 * 2.0 ** -24 * float(ref.abs().max())
