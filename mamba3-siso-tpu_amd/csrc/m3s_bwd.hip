@@ -922,7 +922,7 @@ struct Bwd2Cfg {
   static constexpr int SZ_STAGE = 2 * C * LDF * 4;            // dq~, dkhat f32
   static constexpr int SZ_R = cmax(SZ_X, SZ_STAGE);
   static constexpr int SZ_GAT = N * LDP * 2;                  // G^T [n][p]
-  static constexpr int SZ_SC = (8 * C + 4 * N + 16) * 4;
+  static constexpr int SZ_SC = (10 * C + 4 * N + 16) * 4;
   static constexpr int LDS_BYTES = SZ_R + SZ_GAT + SZ_SC;
   static_assert(N % 64 == 0 && P % 16 == 0 && C % 64 == 0, "tile shape");
   static_assert(T4 % NW == 0 && NW % PB == 0, "adjoint tiles split evenly, one pb per wave");
@@ -1108,7 +1108,10 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
   float* sDqk = sScl + C;
   float* sCoef = sDqk + C;
   float* sDA = sCoef + C;
-  float* sQb = sDA + C;
+  // a row's decay from the end of the strip before its own, and to the end of its strip
+  float* sDt = sDA + C;
+  float* sDk = sDt + C;
+  float* sQb = sDk + C;
   float* sKb = sQb + N;
   // [w]: wave w's share of 2^{A_last}<G,S> + <v, dv_inter> for the current chunk, summed
   // in wave order (no float atomics: the result does not depend on wave timing)
@@ -1378,6 +1381,10 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
         }
         const float excl = incl - run;
         const float a_last = __shfl(incl, 63, 64);
+        // A at the last row of this lane's 16-row strip, and of the one before (0 at the start)
+        const float a_end = __shfl(incl, lane | (16 / F::E - 1), 64);
+        const float a_prev = __shfl(incl, (lane & ~(16 / F::E - 1)) - 1, 64);
+        const float a_in = lane < 16 / F::E ? 0.f : a_prev;
 #pragma unroll
         for (int e = 0; e < F::E; ++e) {
           const int tt = lane * F::E + e;
@@ -1385,6 +1392,8 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
           sA[tt] = A;
           sExpA[tt] = exp2f(A);
           sFac[tt] = exp2f(a_last - A);
+          sDt[tt] = exp2f(A - a_in);
+          sDk[tt] = exp2f(a_end - A);
         }
       }
       if (tid < C) {
@@ -1555,7 +1564,18 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
       float red = 0.f;
       const int jcol = w * 16 + l16;     // this lane's key position (cols of W, dM)
       const float Aj = sA[jcol];
-      // W[t][j] and dM[t][j] for query strip tb (rows t) and key strip w (cols j)
+      // this wave's own key rows, the B operands of every W and dM tile: read once (the
+      // barriers of the instruction scheduler below keep the compiler from hoisting them; six
+      // of a tile's thirteen LDS reads)
+      bf16x8 kf[N / 32], vf[P / 32];
+#pragma unroll
+      for (int i = 0; i < N / 32; ++i) kf[i] = ld_nat8(sK, LDQ, w * 16, 32 * i, lane);
+#pragma unroll
+      for (int i = 0; i < P / 32; ++i) vf[i] = ld_nat8(sV, LDP, w * 16, 32 * i, lane);
+      // W[t][j] and dM[t][j] for query strip tb (rows t) and key strip w (cols j). Below the
+      // diagonal the decay factors through the last row m before the query strip: 2^{A_t - A_j}
+      // = 2^{A_t - A_m} 2^{A_m - A_j}, both in (0, 1] since A falls (t > m >= j): one exp per
+      // lane and tile, as in the forward. The diagonal tile keeps the exact decay and the mask.
       auto wdm = [&](int tb, bf16x4& wt, bf16x4& mt) {
         if (tb < w) {
           wt = sub_from_f32<bf16>(f32x4{0.f, 0.f, 0.f, 0.f});
@@ -1564,21 +1584,28 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
         }
         f32x4 aw = {0.f, 0.f, 0.f, 0.f}, am = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int k0 = 0; k0 < N; k0 += 32)
-          mma32x(aw, ld_nat8(sQ, LDQ, tb * 16, k0, lane), ld_nat8(sK, LDQ, w * 16, k0, lane));
+        for (int k0 = 0; k0 < N; k0 += 32) mma32x(aw, ld_nat8(sQ, LDQ, tb * 16, k0, lane), kf[k0 / 32]);
 #pragma unroll
-        for (int k0 = 0; k0 < P; k0 += 32)
-          mma32x(am, ld_nat8(sG, LDP, tb * 16, k0, lane), ld_nat8(sV, LDP, w * 16, k0, lane));
-        // branch-free mask: 2^{min(A_t - A_j, 0)} is finite for every entry
-        const f32x4 at = *reinterpret_cast<const f32x4*>(sA + tb * 16 + 4 * g4);
+        for (int k0 = 0; k0 < P; k0 += 32) mma32x(am, ld_nat8(sG, LDP, tb * 16, k0, lane), vf[k0 / 32]);
+        f32x4 dec;
+        if (tb > w) {
+          const f32x4 dt = *reinterpret_cast<const f32x4*>(sDt + tb * 16 + 4 * g4);
+          const float ej = __builtin_amdgcn_exp2f(sA[tb * 16 - 1] - Aj);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) dec[i] = dt[i] * ej;
+        } else {   // branch-free mask: 2^{min(A_t - A_j, 0)} is finite for every entry
+          const f32x4 at = *reinterpret_cast<const f32x4*>(sA + tb * 16 + 4 * g4);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float e = __builtin_amdgcn_exp2f(fminf(at[i] - Aj, 0.f));
+            dec[i] = (tb * 16 + 4 * g4 + i > jcol) ? e : 0.f;
+          }
+        }
         f32x4 vw, vm;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int t = tb * 16 + 4 * g4 + i;
-          const float e = __builtin_amdgcn_exp2f(fminf(at[i] - Aj, 0.f));
-          const float dec = (t > jcol) ? e : 0.f;
-          vw[i] = aw[i] * dec;
-          vm[i] = am[i] * dec;
+          vw[i] = aw[i] * dec[i];
+          vm[i] = am[i] * dec[i];
         }
         wt = sub_from_f32<bf16>(vw);
         mt = sub_from_f32<bf16>(vm);
@@ -1600,19 +1627,29 @@ __global__ void __launch_bounds__(C / 16 * 64) bwd_bf16_kernel(const BwdParams p
       // dq~[t][n] += sum_j dM^T[j][t] khat[j][n]   (query strip w, key strips jb <= w)
       const int tcol = w * 16 + l16;
       const float At = sA[tcol];
+      bf16x8 gf[P / 32];
+#pragma unroll
+      for (int i = 0; i < P / 32; ++i) gf[i] = ld_nat8(sG, LDP, w * 16, 32 * i, lane);
       auto dmt = [&](int jb) {
         if (jb > w) return sub_from_f32<bf16>(f32x4{0.f, 0.f, 0.f, 0.f});
         f32x4 am = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int k0 = 0; k0 < P; k0 += 32)
-          mma32x(am, ld_nat8(sV, LDP, jb * 16, k0, lane), ld_nat8(sG, LDP, w * 16, k0, lane));
-        const f32x4 aj = *reinterpret_cast<const f32x4*>(sA + jb * 16 + 4 * g4);
+          mma32x(am, ld_nat8(sV, LDP, jb * 16, k0, lane), gf[k0 / 32]);
         f32x4 vm;
+        if (jb < w) {   // the same factoring, through the key strip's last row
+          const f32x4 dk = *reinterpret_cast<const f32x4*>(sDk + jb * 16 + 4 * g4);
+          const float et = __builtin_amdgcn_exp2f(At - sA[jb * 16 + 15]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int j = jb * 16 + 4 * g4 + i;
-          const float e = __builtin_amdgcn_exp2f(fminf(At - aj[i], 0.f));
-          vm[i] = (tcol > j) ? am[i] * e : 0.f;
+          for (int i = 0; i < 4; ++i) vm[i] = am[i] * (dk[i] * et);
+        } else {
+          const f32x4 aj = *reinterpret_cast<const f32x4*>(sA + jb * 16 + 4 * g4);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int j = jb * 16 + 4 * g4 + i;
+            const float e = __builtin_amdgcn_exp2f(fminf(At - aj[i], 0.f));
+            vm[i] = (tcol > j) ? am[i] * e : 0.f;
+          }
         }
         return sub_from_f32<bf16>(vm);
       };
