@@ -23,8 +23,9 @@ Two execution paths, same results:
   (``m3s_norm_fwd``). In the backward every kernel writes its slice of one projection
   gradient buffer in place -- dz, dx from the scan, dB, dC from ``m3s_norm_bwd``, the
   raw-scalar and angle slices from ``m3s_prep_bwd`` -- so no concatenation is needed.
-* the composed path (a carried ``state``, or shapes the in-place kernels cannot
-  address): torch autograd over `rms_norm`, the differentiable `preprocess` and `siso`.
+* the composed path (a carried ``state`` with gradients, or shapes the in-place kernels
+  cannot address): torch autograd over `rms_norm`, the differentiable `preprocess` and
+  `siso`. Without gradients a carried state runs the same steps as `_segment_forward`.
 """
 
 from __future__ import annotations
@@ -336,6 +337,43 @@ class _LayerFn(torch.autograd.Function):
                 None)
 
 
+def _segment_fused_ok(params: SISOParams, u: Tensor, cfg: SISOConfig, state) -> bool:
+    """Whether a segment with a carried state runs as `_segment_forward`: no gradient is taken,
+    `_fused_ok` holds, the projection's own rows are 16-byte aligned, and the carry has the
+    layer's shapes on ``u``'s device (anything else is left to the composed path)."""
+    if state is None or not _fused_ok(u, cfg, None) or cfg.d_in_proj % (16 // u.element_size()):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in (u, *params, *state)):
+        return False
+    b, h = u.shape[0], cfg.nheads
+    shapes = ((b, h, cfg.headdim, cfg.d_state), (b, h, cfg.d_state), (b, h, cfg.headdim),
+              (b, h, cfg.n_angles))
+    return all(tuple(t.shape) == s and t.device == u.device for t, s in zip(state, shapes))
+
+
+def _segment_forward(params: SISOParams, u: Tensor, cfg: SISOConfig, state: SISOState):
+    """The composed path of a segment without gradients as direct launches: both norms in one
+    ``m3s_norm_fwd`` (thirteen framework kernels as `rms_norm`), the preprocess and the scan
+    without their autograd nodes. B=1, L=896, d_model 768: 187 us of kernels and 300 us of host
+    work before."""
+    batch, seqlen, dm = u.shape
+    m = batch * seqlen
+    proj = (u.reshape(m, dm) @ params.in_proj.to(u.dtype)).view(batch, seqlen, cfg.d_in_proj)
+    z, x, b, c, dt_raw, a_raw, trap_raw, angles = split_in_proj(proj, cfg)
+    (k, q), _ = K.bcnorm_forward([b, c], [params.b_norm_weight, params.c_norm_weight], cfg.norm_eps)
+    adt, gamma, scale, lam, dt, phi, phi_final = SP.prep_forward_launch(
+        dt_raw, a_raw, trap_raw, angles, params.dt_bias.float().contiguous(),
+        state.phi.float().contiguous(), cfg.a_floor)
+    y, fs, fk, fv = K.siso_forward(
+        q, k, x.permute(0, 2, 1, 3), adt, gamma, scale, phi, params.c_bias, params.b_bias,
+        d_skip=params.d_skip, z=z.permute(0, 2, 1, 3), seed_ssm=state.ssm, seed_k=state.k,
+        seed_v=state.v, seed_coef=dt[:, :, 0] * (1.0 - lam[:, :, 0]), chunk=cfg.chunk,
+        dtype_policy=cfg.policy_name)
+    y2 = y.permute(0, 2, 1, 3).reshape(m, cfg.d_inner)
+    out = (y2 @ params.out_proj.to(u.dtype)).view(batch, seqlen, dm)
+    return out, SISOState(ssm=fs, k=fk, v=fv, phi=phi_final)
+
+
 def mamba3_siso_layer(params: SISOParams, u: Tensor, cfg: SISOConfig,
                       state: Optional[SISOState] = None, interpret: Any = False,
                       device_kind: str | None = None, phi_in_kernel: Optional[bool] = None):
@@ -358,6 +396,8 @@ def mamba3_siso_layer(params: SISOParams, u: Tensor, cfg: SISOConfig,
             params.c_norm_weight, params.b_bias, params.c_bias, params.d_skip, cfg,
             phi_in_kernel)
         return out, SISOState(ssm=fs, k=fk, v=fv, phi=phi_final)
+    if _segment_fused_ok(params, u, cfg, state):
+        return _segment_forward(params, u, cfg, state)
     batch, seqlen, _ = u.shape
     proj = u @ params.in_proj.to(u.dtype)
     z, x, b, c, dt_raw, a_raw, trap_raw, angles = split_in_proj(proj, cfg)

@@ -632,3 +632,46 @@ def test_layer_gradients_cfg3_full_size(m3):
     for f in p_cpu._fields:
         report(f"cfg3 layer d{f} vs bf16 layer model", getattr(params, f).grad, pd[f].grad)
         assert_maxrel(getattr(params, f).grad, pd[f].grad, BF16_GRAD_MAXREL, f"d{f}")
+
+
+@pytest.mark.parametrize("policy,batch,seqlen,kw", [
+    ("bf16", 1, 896, dict(d_model=256, chunk=128)),
+    ("bf16", 3, 128, dict(d_model=256, chunk=128)),             # a single chunk
+    ("bf16", 2, 384, dict(d_model=512, chunk=128, headdim=128)),   # sub-heads
+    ("bf16", 2, 320, dict(d_model=256, chunk=64, d_state=64, rope_fraction=1.0)),
+    ("f32", 2, 128, dict(d_model=64, d_state=16, headdim=16, expand=1, chunk=64)),
+])
+def test_segment_without_gradients_equals_composed(m3, dev, monkeypatch, policy, batch, seqlen, kw):
+    """A carried state without gradients (direct launches) against the composed path that
+    gradients take: the same projection and scan; the norm's f32 reciprocal root may round a
+    normalised bf16 entry the other way (one operand rounding, the bound of the bf16 tests; a
+    few f32 roundings in f32)."""
+    LY = m3.layer
+    cfg = m3.SISOConfig(policy_name=policy, **kw)
+    dt = BF16 if policy == "bf16" else torch.float32
+    g = torch.Generator().manual_seed(seqlen)
+    p = m3.init_params(cfg, 3, device=dev)
+    u = torch.randn(batch, seqlen, cfg.d_model, generator=g).to(dt).to(dev)
+    h, n = cfg.nheads, cfg.d_state
+    st = m3.SISOState(torch.randn(batch, h, cfg.headdim, n, generator=g).to(dev) * 0.1,
+                      torch.randn(batch, h, n, generator=g).to(dev),
+                      torch.randn(batch, h, cfg.headdim, generator=g).to(dev),
+                      (torch.rand(batch, h, cfg.n_angles, generator=g) * 6.28).to(dev))
+    with torch.no_grad():
+        assert LY._segment_fused_ok(p, u, cfg, st)
+        assert not LY._segment_fused_ok(p, u, cfg, st._replace(phi=st.phi[..., :-1]))
+        assert not LY._segment_fused_ok(p, u, cfg, None)
+        got, sg = m3.mamba3_siso_layer(p, u, cfg, state=st)
+        with monkeypatch.context() as mp:
+            mp.setattr(LY, "_segment_fused_ok", lambda *a: False)
+            ref, sr = m3.mamba3_siso_layer(p, u, cfg, state=st)
+    assert LY._segment_fused_ok(p, u, cfg, st)       # no tensor requires a gradient
+    assert not LY._segment_fused_ok(p._replace(d_skip=p.d_skip.clone().requires_grad_(True)), u, cfg, st)
+    if policy == "bf16":
+        assert_bf16_bound(got, cpu(ref), what="out")
+    else:
+        assert_maxrel(got, cpu(ref), 1e-5, "out")
+    assert got.dtype == ref.dtype == dt
+    for name, a, b in zip(("ssm", "k", "v", "phi"), sg, sr):
+        assert a.dtype == b.dtype and a.shape == b.shape, name
+        assert_maxrel(a, cpu(b), 2e-3 if policy == "bf16" else 1e-5, name)
