@@ -675,3 +675,24 @@ def test_segment_without_gradients_equals_composed(m3, dev, monkeypatch, policy,
     for name, a, b in zip(("ssm", "k", "v", "phi"), sg, sr):
         assert a.dtype == b.dtype and a.shape == b.shape, name
         assert_maxrel(a, cpu(b), 2e-3 if policy == "bf16" else 1e-5, name)
+
+
+@pytest.mark.parametrize("batch,seqlen,d_model", [(1, 128, 256), (2, 1024, 1024)])   # the most tokens it takes
+def test_forward_with_row_major_weights(m3, dev, monkeypatch, batch, seqlen, d_model):
+    """Few tokens multiply by the weights as they are: against the laid-out weights, whose
+    product may round a bf16 projection entry the other way (the operand-rounding bound)."""
+    LY = m3.layer
+    cfg = m3.SISOConfig(d_model=d_model)
+    p = m3.init_params(cfg, 5, device=dev)
+    p = p._replace(in_proj=p.in_proj.to(BF16), out_proj=p.out_proj.to(BF16))
+    u = torch.randn(batch, seqlen, d_model, generator=torch.Generator().manual_seed(1)).to(BF16).to(dev)
+    assert LY._weights_direct(u, p.in_proj, p.out_proj, cfg)
+    assert not LY._weights_direct(torch.cat([u, u[:, :1]], 1), p.in_proj, p.out_proj, cfg) or d_model < 1024
+    assert not LY._weights_direct(u, p.in_proj.float(), p.out_proj, cfg)
+    with torch.no_grad():
+        got, sg = m3.mamba3_siso_layer(p, u, cfg)
+        monkeypatch.setattr(LY, "_weights_direct", lambda *a: False)
+        ref, sr = m3.mamba3_siso_layer(p, u, cfg)
+    assert_bf16_bound(got, cpu(ref), what="out")
+    for name, a, b in zip(("ssm", "k", "v"), sg, sr):
+        assert_maxrel(a, cpu(b), BF16_MAXREL, name)
