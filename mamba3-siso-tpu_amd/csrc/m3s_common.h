@@ -268,6 +268,35 @@ __device__ __forceinline__ float wave_total(float v) {
           __builtin_bit_cast(float, __builtin_amdgcn_readlane(i, 48)));
 }
 
+// Sum of nblk partial rows (row b's entry at part[b * stride], the thread's own column) over a
+// block of 16 waves that share 64 columns: wave w takes rows w, w + 16, ..., eight loads in
+// flight, and the waves' sums are added in wave order, returned to wave 0. A few hundred KB
+// on two to twelve blocks is latency, not bandwidth: with four waves the 1024 partials of a
+// gain took 15 us.
+constexpr int kColSumThreads = 1024;
+__device__ __forceinline__ float column_sum(const float* part, int64_t stride, int nblk, bool ok) {
+  __shared__ float sums[kColSumThreads / 64][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int NW = kColSumThreads / 64;
+  float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (ok) {
+    int b = wave;
+    for (; b + 7 * NW < nblk; b += 8 * NW) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) a[u] += part[(int64_t)(b + u * NW) * stride];
+    }
+    for (; b < nblk; b += NW) a[0] += part[(int64_t)b * stride];
+  }
+  sums[wave][lane] = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+  __syncthreads();
+  float t = 0.f;
+  if (wave == 0) {
+    t = sums[0][lane];
+    for (int w = 1; w < NW; ++w) t += sums[w][lane];
+  }
+  return t;
+}
+
 // n / d and n % d for 0 <= n < 2^20 by a divisor d known only at run time, without an
 // integer division (a software routine on the GPU): a float estimate of the quotient
 // (relative error below 2^-21, so off by at most one in this range), then one correction.

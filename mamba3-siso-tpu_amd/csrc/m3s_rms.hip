@@ -210,28 +210,13 @@ __global__ void __launch_bounds__(kRmsThreads) rms_bwd_kernel(const TX* __restri
   }
 }
 
-// dw[c] = sum over blocks of part[b][c]: a block takes 64 columns; its 4 waves take every
-// 4th block row (unrolled, so the loads of a run are in flight together), then the 4
-// wave sums are added in wave order
-__global__ void __launch_bounds__(kRmsThreads) rms_dw_kernel(const float* __restrict__ part,
-                                                             float* __restrict__ dw, int nblk,
-                                                             int D) {
-  __shared__ float sSum[kRmsWaves][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int c = blockIdx.x * 64 + lane;
-  float t = 0.f;
-  if (c < D) {
-#pragma unroll 8
-    for (int b = wave; b < nblk; b += kRmsWaves) t += part[(int64_t)b * D + c];
-  }
-  sSum[wave][lane] = t;
-  __syncthreads();
-  if (wave == 0 && c < D) {
-    float s = 0.f;
-#pragma unroll
-    for (int v = 0; v < kRmsWaves; ++v) s += sSum[v][lane];
-    dw[c] = s;
-  }
+// dw[c] = sum over blocks of part[b][c], 64 columns a block (column_sum).
+__global__ void __launch_bounds__(kColSumThreads) rms_dw_kernel(const float* __restrict__ part,
+                                                                float* __restrict__ dw, int nblk,
+                                                                int D) {
+  const int c = blockIdx.x * 64 + (threadIdx.x & 63);
+  const float t = column_sum(part + c, D, nblk, c < D);
+  if (threadIdx.x < 64 && c < D) dw[c] = t;
 }
 
 static int32_t check_rms(const m3s_rms_args* a, const char* who, bool bwd) {
@@ -287,7 +272,7 @@ static void launch_rms_bwd(const m3s_rms_args* a, hipStream_t s) {
   if (a->width <= 1024) go(rms_bwd_kernel<TX, TY, 4>);
   else if (a->width <= 2048) go(rms_bwd_kernel<TX, TY, 8>);
   else go(rms_bwd_kernel<TX, TY, kRmsMaxChunks>);
-  hipLaunchKernelGGL(rms_dw_kernel, dim3((a->width + 63) / 64), dim3(kRmsThreads), 0, s, part,
+  hipLaunchKernelGGL(rms_dw_kernel, dim3((a->width + 63) / 64), dim3(kColSumThreads), 0, s, part,
                      a->dweight, nblk, a->width);
 }
 
