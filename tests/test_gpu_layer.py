@@ -495,6 +495,22 @@ def test_weight_grad_matches_float64(m3, dev, m, p, q, dtype):
     assert torch.equal(got, m3.layer.weight_grad(ad, bd))
 
 
+@pytest.mark.parametrize("m", [32, 64, 96, 544])       # 1, 2, 3 and 17 steps: 1 or 2 splits
+@pytest.mark.parametrize("p,q", [(1540, 264), (3000, 8), (260, 1800)])   # 7, 12 and 2 tile rows
+def test_weight_grad_tile_bands_and_steps(m3, dev, m, p, q):
+    """``m3s_wgrad`` over tile grids whose rows fill a band of 6 with a remainder, exactly, or
+    not at all, at the step counts where its two wave groups start and end: against float64
+    within m float32 roundings of sum |a||b|, every tile written, bit-identical again."""
+    g = torch.Generator().manual_seed(m * p + q)
+    ad = torch.randn(m, (p + 7) // 8 * 8, generator=g).to(torch.bfloat16).to(dev)[:, :p]
+    bd = torch.randn(m, q, generator=g).to(torch.bfloat16).to(dev)
+    got = m3.kernels.wgrad(ad, bd)
+    a, b = ad.cpu().double(), bd.cpu().double()
+    bound = m * 2.0 ** -24 * (a.abs().t() @ b.abs())
+    assert ((got.cpu().double() - a.t() @ b).abs() <= bound).all()
+    assert torch.equal(got, m3.kernels.wgrad(ad, bd))
+
+
 @pytest.mark.parametrize("m,k,n,ldw", [
     (1, 768, 3432, 3432),    # the LM's in_proj at one row
     (2, 1536, 768, 776),     # out_proj / fc2 widths, a padded weight row stride
