@@ -18,7 +18,7 @@
 // values: each 32-token step is staged in LDS as it lies in memory (rows = tokens, 16-byte
 // pieces), and the fragments are read with ds_read_b64_tr_b16, which hands each lane four
 // consecutive tokens of one column. Staging: registers one step ahead, two LDS stages,
-// one barrier per step.
+// one barrier per step; the two waves of a SIMD read and multiply in opposite order.
 #include "m3s_common.h"
 #include "m3s_internal.h"
 
@@ -74,7 +74,8 @@ __global__ void __launch_bounds__(kWgThreads) wgrad_kernel(const WgParams p) {
   int k0, k1;
   split_range(p.nks, p.S, s, k0, k1);
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wp = wave % kWgWP, wq = wave / kWgWP;   // this wave's block of the tile
   const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a, p.ea), rb = make_rsrc(p.b, p.eb);
 
@@ -90,13 +91,16 @@ __global__ void __launch_bounds__(kWgThreads) wgrad_kernel(const WgParams p) {
     vb[r] = row * p.ldb2 + (uint32_t)(q0 + col) * 2;
     lo[r] = row * kWgLd + col;
   }
-  bf16x8 ga[kWgPieces], gb[kWgPieces];
-  auto gload = [&](int ks) {
+  struct Set { bf16x8 a[kWgPieces], b[kWgPieces]; };
+  Set g;
+  const int n = k1 - k0;
+  auto gload = [&](int it) {   // past the last step: that step again, unused (n > 0)
+    const int ks = k0 + (it < n ? it : n - 1);
     const uint32_t sa = (uint32_t)ks * kWgK * p.lda2, sb = (uint32_t)ks * kWgK * p.ldb2;
 #pragma unroll
     for (int r = 0; r < kWgPieces; ++r) {
-      ga[r] = buf_load<bf16x8>(ra, va[r], sa);
-      gb[r] = buf_load<bf16x8>(rb, vb[r], sb);
+      g.a[r] = buf_load<bf16x8>(ra, va[r], sa);
+      g.b[r] = buf_load<bf16x8>(rb, vb[r], sb);
     }
   };
   auto swrite = [&](int st) {
@@ -104,8 +108,8 @@ __global__ void __launch_bounds__(kWgThreads) wgrad_kernel(const WgParams p) {
     bf16* sb = sa + kWgK * kWgLd;
 #pragma unroll
     for (int r = 0; r < kWgPieces; ++r) {
-      *reinterpret_cast<bf16x8*>(sa + lo[r]) = ga[r];
-      *reinterpret_cast<bf16x8*>(sb + lo[r]) = gb[r];
+      *reinterpret_cast<bf16x8*>(sa + lo[r]) = g.a[r];
+      *reinterpret_cast<bf16x8*>(sb + lo[r]) = g.b[r];
     }
   };
 
@@ -119,46 +123,66 @@ __global__ void __launch_bounds__(kWgThreads) wgrad_kernel(const WgParams p) {
   // eight) and 16 + 4g .. 16 + 4g + 3 (second half), the same for both operands. One
   // transposed read then covers 16 consecutive token rows across the four groups.
   const int kh0 = 4 * (lane >> 4), kh1 = 16 + kh0;
-  auto compute = [&](int st) {
+  static_assert(kWgK == 32, "one MFMA K block per step");
+  bf16x4 fa0[kWgRT], fa1[kWgRT], fb0[kWgCT], fb1[kWgCT];
+  auto read_frags = [&](int st) {
     const bf16* sa = lds + st * kWgStage;
     const bf16* sb = sa + kWgK * kWgLd;
 #pragma unroll
-    for (int k = 0; k < kWgK; k += 32) {
-      bf16x4 a0[kWgRT], a1[kWgRT], b0[kWgCT], b1[kWgCT];
+    for (int i = 0; i < kWgRT; ++i) {
+      fa0[i] = ld_tr4(sa, kWgLd, kh0, wp * 16 * kWgRT + 16 * i, lane);
+      fa1[i] = ld_tr4(sa, kWgLd, kh1, wp * 16 * kWgRT + 16 * i, lane);
+    }
 #pragma unroll
-      for (int i = 0; i < kWgRT; ++i) {
-        a0[i] = ld_tr4(sa, kWgLd, k + kh0, wp * 16 * kWgRT + 16 * i, lane);
-        a1[i] = ld_tr4(sa, kWgLd, k + kh1, wp * 16 * kWgRT + 16 * i, lane);
-      }
+    for (int j = 0; j < kWgCT; ++j) {
+      fb0[j] = ld_tr4(sb, kWgLd, kh0, wq * 16 * kWgCT + 16 * j, lane);
+      fb1[j] = ld_tr4(sb, kWgLd, kh1, wq * 16 * kWgCT + 16 * j, lane);
+    }
+  };
+  auto products = [&]() {
 #pragma unroll
-      for (int j = 0; j < kWgCT; ++j) {
-        b0[j] = ld_tr4(sb, kWgLd, k + kh0, wq * 16 * kWgCT + 16 * j, lane);
-        b1[j] = ld_tr4(sb, kWgLd, k + kh1, wq * 16 * kWgCT + 16 * j, lane);
-      }
+    for (int i = 0; i < kWgRT; ++i) {
 #pragma unroll
-      for (int i = 0; i < kWgRT; ++i) {
-#pragma unroll
-        for (int j = 0; j < kWgCT; ++j) mma32(acc[i][j], a0[i], a1[i], b0[j], b1[j]);
-      }
+      for (int j = 0; j < kWgCT; ++j) mma32(acc[i][j], fa0[i], fa1[i], fb0[j], fb1[j]);
     }
   };
 
-  // Step k is read from LDS stage k & 1; step k + 1 waits in registers (loaded during
-  // step k - 1) and goes to the other stage after step k's products, then step k + 2's
-  // loads are issued into the same registers.
-  const int n = k1 - k0;
+  // What bounds a step: 96 KB of fragment reads and 32 KB of writes keep the LDS busy as long
+  // (about 1030 cycles) as the products keep the matrix pipes. So the waves are in two groups,
+  // one of each on every SIMD (waves w and w + 4), in opposite order: in the phase after
+  // barrier k the first reads step k's fragments and then multiplies them, the second
+  // multiplies step k - 1's and then reads step k's. Every wave writes step k + 1 to the stage
+  // that phase k - 1 read. All waves in one order took 769 us where this takes 748 (65536
+  // tokens, 1024 x 6352), 241 -> 238 (32768, 768 x 4880), 104 -> 101 (32768, 768 x 2048); a strict half-step offset with a third stage and two barriers a step was 9% slower.
   if (n > 0) {
-    gload(k0);
+    gload(0);
     swrite(0);
-    if (n > 1) gload(k0 + 1);
-    for (int it = 0; it < n; ++it) {
-      // after this barrier stage it & 1 holds step it, and every wave is done reading
-      // stage (it + 1) & 1 (step it - 1), which is refilled after this step's products:
-      // the fragment reads start right after the barrier, not behind a burst of writes
+    gload(1);
+    if (wave < kWgThreads / 128) {
+      for (int k = 0; k < n; ++k) {
+        __syncthreads();
+        read_frags(k & 1);
+        swrite((k + 1) & 1);
+        gload(k + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        products();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
       __syncthreads();
-      compute(it & 1);
-      if (it + 1 < n) swrite((it + 1) & 1);
-      if (it + 2 < n) gload(k0 + it + 2);
+      swrite(1);
+      gload(2);
+      read_frags(0);
+      for (int k = 1; k < n; ++k) {
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        products();
+        __builtin_amdgcn_sched_barrier(0);
+        swrite((k + 1) & 1);
+        gload(k + 2);
+        read_frags(k & 1);
+      }
+      products();
     }
   }
 
