@@ -35,6 +35,7 @@ import math
 from typing import Any, NamedTuple, Optional
 
 import torch
+import torch.autograd.forward_ad as fwd_ad
 import torch.nn.functional as F
 
 from . import kernels as K
@@ -365,6 +366,10 @@ def _segment_fused_ok(params: SISOParams, u: Tensor, cfg: SISOConfig, state) -> 
     if state is None or not _fused_ok(u, cfg, None) or cfg.d_in_proj % (16 // u.element_size()):
         return False
     if torch.is_grad_enabled() and any(t.requires_grad for t in (u, *params, *state)):
+        return False
+    # a forward-mode tangent would be dropped here without a word; the composed path's nodes refuse it
+    if fwd_ad._current_level >= 0 and any(
+            fwd_ad.unpack_dual(t).tangent is not None for t in (u, *params, *state)):
         return False
     b, h = u.shape[0], cfg.nheads
     shapes = ((b, h, cfg.headdim, cfg.d_state), (b, h, cfg.d_state), (b, h, cfg.headdim),

@@ -712,3 +712,23 @@ def test_forward_with_row_major_weights(m3, dev, monkeypatch, batch, seqlen, d_m
     assert_bf16_bound(got, cpu(ref), what="out")
     for name, a, b in zip(("ssm", "k", "v"), sg, sr):
         assert_maxrel(a, cpu(b), BF16_MAXREL, name)
+
+
+def test_segment_with_a_forward_mode_tangent_is_refused(m3, dev):
+    """Direct launches would drop a tangent silently: such a call goes to the composed path,
+    whose autograd functions have no forward-mode rule and say so."""
+    import torch.autograd.forward_ad as fwd_ad
+    cfg = m3.SISOConfig(d_model=256, chunk=128)
+    p = m3.init_params(cfg, 3, device=dev)
+    gen = torch.Generator().manual_seed(0)
+    u, t = (torch.randn(1, 128, 256, generator=gen).to(BF16).to(dev) for _ in range(2))
+    h, n = cfg.nheads, cfg.d_state
+    st = m3.SISOState(*(torch.zeros(s, device=dev) for s in (
+        (1, h, cfg.headdim, n), (1, h, n), (1, h, cfg.headdim), (1, h, cfg.n_angles))))
+    assert m3.layer._segment_fused_ok(p, u, cfg, st)
+    with fwd_ad.dual_level():
+        assert m3.layer._segment_fused_ok(p, u, cfg, st)
+        dual = fwd_ad.make_dual(u, t)
+        assert not m3.layer._segment_fused_ok(p, dual, cfg, st)
+        with pytest.raises((NotImplementedError, RuntimeError)):
+            m3.mamba3_siso_layer(p, dual, cfg, state=st)
