@@ -1181,10 +1181,13 @@ def _gemv_fused(mode: int, x: Tensor, w: Tensor, k: int, n: int, out_dtype: torc
     rows = x.shape[0]
     tensors = [t for t in (x, w, add, gain) if t is not None]
     dev = _device_of(*tensors)
-    if (not 1 <= rows <= FUSED_ROWS_MAX or not all(t.is_contiguous() for t in tensors)
+    width = 2 * k if mode == _lib.GEMV_GATE else k
+    if (not 1 <= rows <= FUSED_ROWS_MAX or tuple(x.shape) != (rows, width)
+            or not all(t.is_contiguous() for t in tensors)
             or (add is not None and (add.dtype != torch.bfloat16 or add.shape != x.shape))
             or (gain is not None and (gain.dtype != torch.float32 or gain.shape != (k,)))):
-        raise ValueError("gemv_fused: one or two dense rows, add in bf16 like x, gain (k,) float32")
+        raise ValueError("gemv_fused: one or two dense rows of w's width, add in bf16 like x, gain (k,) "
+                         "float32")
     y = empty(rows, n, device=dev, dtype=out_dtype)
     total = x
     a = _lib.GemvFusedArgs()

@@ -375,3 +375,13 @@ def test_decode_step_with_folded_norms_and_gates(m3, dev, monkeypatch, d, di, vo
                     assert torch.equal(x, y), t
             assert got.shape == ref.shape == (rows, vocab) and got.dtype == ref.dtype
             assert float((got - ref).abs().max()) <= d ** 1.5 * 2.0 ** -24 * float(ref.abs().max())
+
+
+def test_folded_products_refuse_rows_of_another_width(m3, dev):
+    """A row narrower than its weight is an error on the host, before any launch."""
+    x, w = torch.zeros(1, 256, device=dev), torch.zeros(512, 256, device=dev, dtype=torch.bfloat16)
+    gain = torch.ones(512, device=dev)
+    with pytest.raises(ValueError, match="width"):
+        m3.kernels.gemv_norm(x, None, gain, 1e-5, w)
+    with pytest.raises(ValueError, match="width"):
+        m3.kernels.head_logits(x, None, gain, 1e-5, torch.zeros(64, 512, device=dev))
