@@ -153,7 +153,8 @@ __global__ void __launch_bounds__(kWgThreads) wgrad_kernel(const WgParams p) {
   // barrier k the first reads step k's fragments and then multiplies them, the second
   // multiplies step k - 1's and then reads step k's. Every wave writes step k + 1 to the stage
   // that phase k - 1 read. All waves in one order took 769 us where this takes 748 (65536
-  // tokens, 1024 x 6352), 241 -> 238 (32768, 768 x 4880), 104 -> 101 (32768, 768 x 2048); a strict half-step offset with a third stage and two barriers a step was 9% slower.
+  // tokens, 1024 x 6352), 241 -> 238 (32768, 768 x 4880), 104 -> 101 (32768, 768 x 2048); a strict half-step offset
+  // with a third stage and two barriers a step was 9% slower.
   if (n > 0) {
     gload(0);
     swrite(0);
