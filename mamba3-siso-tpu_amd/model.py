@@ -421,11 +421,11 @@ def _decode_step_fused(params: LMParams, x: Tensor, states: list, cfg: LMConfig)
     in the head's."""
     c, out_states, y = cfg.siso, [], None
     c.require_kernels()
-    for b, state in zip(params.blocks, states):
+    for i, b in enumerate(params.blocks):
         p = b.siso
         proj, x = K.gemv_norm(x, y, b.norm_gain, c.norm_eps, p.in_proj)
         y, st = K.decode_layer_step(
-            proj, state, nheads=c.nheads, headdim=c.headdim, state_dim=c.d_state,
+            proj, states[i], nheads=c.nheads, headdim=c.headdim, state_dim=c.d_state,
             n_angles=c.n_angles, b_norm_weight=p.b_norm_weight, c_norm_weight=p.c_norm_weight,
             dt_bias=p.dt_bias, q_bias=p.c_bias, k_bias=p.b_bias, d_skip=p.d_skip,
             a_floor=c.a_floor, norm_eps=c.norm_eps)

@@ -385,3 +385,15 @@ def test_folded_products_refuse_rows_of_another_width(m3, dev):
         m3.kernels.gemv_norm(x, None, gain, 1e-5, w)
     with pytest.raises(ValueError, match="width"):
         m3.kernels.head_logits(x, None, gain, 1e-5, torch.zeros(64, 512, device=dev))
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3])   # folded (one and two rows) and pass by pass
+def test_decode_step_refuses_too_few_states(m3, dev, rows):
+    """A step with fewer states than blocks is an error, not a shorter model."""
+    M = m3.model
+    cfg = M.LMConfig(vocab_size=64, n_layers=2, d_intermediate=0, siso=m3.SISOConfig(d_model=256))
+    params = M.decode_params(M.init_lm(cfg, 0, device=dev), cfg)
+    tok = torch.zeros(rows, dtype=torch.int64, device=dev)
+    with torch.no_grad():
+        with pytest.raises(IndexError):
+            M.lm_decode_step(params, tok, M.zero_states(cfg, rows, device=dev)[:1], cfg)
