@@ -361,8 +361,10 @@ class _LayerFn(torch.autograd.Function):
 
 def _segment_fused_ok(params: SISOParams, u: Tensor, cfg: SISOConfig, state) -> bool:
     """Whether a segment with a carried state runs as `_segment_forward`: no gradient is taken,
-    `_fused_ok` holds, the projection's own rows are 16-byte aligned, and the carry has the
-    layer's shapes on ``u``'s device (anything else is left to the composed path)."""
+    `_fused_ok` holds, the projection's own rows are 16-byte aligned, and the carry and the
+    vectors that go to the kernels by address (dt_bias, the two gains) have the layer's shapes
+    on ``u``'s device. Anything else is left to the composed path, which refuses it or takes
+    it (a gain of one entry broadcasts there)."""
     if state is None or not _fused_ok(u, cfg, None) or cfg.d_in_proj % (16 // u.element_size()):
         return False
     if torch.is_grad_enabled() and any(t.requires_grad for t in (u, *params, *state)):
@@ -371,10 +373,12 @@ def _segment_fused_ok(params: SISOParams, u: Tensor, cfg: SISOConfig, state) -> 
     if fwd_ad._current_level >= 0 and any(
             fwd_ad.unpack_dual(t).tangent is not None for t in (u, *params, *state)):
         return False
-    b, h = u.shape[0], cfg.nheads
-    shapes = ((b, h, cfg.headdim, cfg.d_state), (b, h, cfg.d_state), (b, h, cfg.headdim),
-              (b, h, cfg.n_angles))
-    return all(tuple(t.shape) == s and t.device == u.device for t, s in zip(state, shapes))
+    b, h, n = u.shape[0], cfg.nheads, cfg.d_state
+    vectors = (params.dt_bias, params.b_norm_weight, params.c_norm_weight)
+    shapes = ((b, h, cfg.headdim, n), (b, h, n), (b, h, cfg.headdim), (b, h, cfg.n_angles),
+              (h,), (n,), (n,))
+    return all(tuple(t.shape) == s and t.device == u.device
+               for t, s in zip((*state, *vectors), shapes))
 
 
 def _segment_forward(params: SISOParams, u: Tensor, cfg: SISOConfig, state: SISOState):

@@ -732,3 +732,42 @@ def test_segment_with_a_forward_mode_tangent_is_refused(m3, dev):
         assert not m3.layer._segment_fused_ok(p, dual, cfg, st)
         with pytest.raises((NotImplementedError, RuntimeError)):
             m3.mamba3_siso_layer(p, dual, cfg, state=st)
+
+
+def _segment_case(m3, dev, **kw):
+    cfg = m3.SISOConfig(d_model=256, chunk=128, **kw)
+    gen = torch.Generator().manual_seed(0)
+    p = m3.init_params(cfg, 3, device=dev)
+    u = torch.randn(2, 128, 256, generator=gen).to(BF16).to(dev)
+    h, n = cfg.nheads, cfg.d_state
+    st = m3.SISOState(*(torch.rand(2, *s, generator=gen).to(dev) for s in (
+        (h, cfg.headdim, n), (h, n), (h, cfg.headdim), (h, cfg.n_angles))))
+    return cfg, p, u, st
+
+
+@pytest.mark.parametrize("field,change", [
+    ("dt_bias", lambda t: t[:-1]), ("dt_bias", lambda t: t[:1]), ("dt_bias", lambda t: t.cpu()),
+    ("b_norm_weight", lambda t: t[:-1]), ("c_norm_weight", lambda t: t[:64]),
+    ("b_norm_weight", lambda t: t.cpu()), ("c_norm_weight", lambda t: torch.cat([t, t])),
+])
+def test_segment_refuses_vectors_of_another_shape_or_device(m3, dev, field, change):
+    """dt_bias and the gains go to the segment's kernels by address: a wrong length or a host
+    tensor is sent to the composed path, which refuses it before any kernel reads it."""
+    cfg, p, u, st = _segment_case(m3, dev)
+    q = p._replace(**{field: change(getattr(p, field))})
+    with torch.no_grad():
+        assert m3.layer._segment_fused_ok(p, u, cfg, st)
+        assert not m3.layer._segment_fused_ok(q, u, cfg, st)
+        with pytest.raises((ValueError, RuntimeError)):
+            m3.mamba3_siso_layer(q, u, cfg, state=st)
+
+
+def test_segment_takes_a_gain_of_one_entry(m3, dev):
+    """A (1,) gain broadcasts over the row, as in the composed path."""
+    cfg, p, u, st = _segment_case(m3, dev)
+    one = p._replace(b_norm_weight=torch.full((1,), 1.5, device=dev))
+    full = p._replace(b_norm_weight=torch.full((cfg.d_state,), 1.5, device=dev))
+    with torch.no_grad():
+        assert not m3.layer._segment_fused_ok(one, u, cfg, st)
+        got, ref = (m3.mamba3_siso_layer(q, u, cfg, state=st)[0] for q in (one, full))
+    assert_bf16_bound(got, cpu(ref), what="out")
