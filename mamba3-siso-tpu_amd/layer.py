@@ -367,11 +367,12 @@ def _segment_fused_ok(params: SISOParams, u: Tensor, cfg: SISOConfig, state) -> 
     it (a gain of one entry broadcasts there)."""
     if state is None or not _fused_ok(u, cfg, None) or cfg.d_in_proj % (16 // u.element_size()):
         return False
-    if torch.is_grad_enabled() and any(t.requires_grad for t in (u, *params, *state)):
+    tensors = [t for t in (u, *params, *state) if t is not None]   # d_skip may be None
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return False
     # a forward-mode tangent would be dropped here without a word; the composed path's nodes refuse it
     if fwd_ad._current_level >= 0 and any(
-            fwd_ad.unpack_dual(t).tangent is not None for t in (u, *params, *state)):
+            fwd_ad.unpack_dual(t).tangent is not None for t in tensors):
         return False
     b, h, n = u.shape[0], cfg.nheads, cfg.d_state
     vectors = (params.dt_bias, params.b_norm_weight, params.c_norm_weight)

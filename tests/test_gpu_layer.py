@@ -771,3 +771,16 @@ def test_segment_takes_a_gain_of_one_entry(m3, dev):
         assert not m3.layer._segment_fused_ok(one, u, cfg, st)
         got, ref = (m3.mamba3_siso_layer(q, u, cfg, state=st)[0] for q in (one, full))
     assert_bf16_bound(got, cpu(ref), what="out")
+
+
+@pytest.mark.parametrize("grad_mode", [False, True])
+def test_segment_without_a_skip(m3, dev, grad_mode):
+    """``d_skip=None`` (no skip term) runs a segment in and out of grad mode, as a skip of
+    zeros does: the same products and scan, but for a term that adds zero."""
+    cfg, p, u, st = _segment_case(m3, dev)
+    with torch.set_grad_enabled(grad_mode):
+        got, sg = m3.mamba3_siso_layer(p._replace(d_skip=None), u, cfg, state=st)
+        ref, sr = m3.mamba3_siso_layer(p._replace(d_skip=torch.zeros_like(p.d_skip)), u, cfg, state=st)
+    assert torch.equal(got, ref)
+    for a, b in zip(sg, sr):
+        assert torch.equal(a, b)
