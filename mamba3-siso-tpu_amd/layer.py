@@ -401,7 +401,7 @@ def _segment_forward(params: SISOParams, u: Tensor, cfg: SISOConfig, state: SISO
         seed_v=state.v, seed_coef=dt[:, :, 0] * (1.0 - lam[:, :, 0]), chunk=cfg.chunk,
         dtype_policy=cfg.policy_name)
     y2 = y.permute(0, 2, 1, 3).reshape(m, cfg.d_inner)
-    out = (y2 @ params.out_proj.to(u.dtype)).view(batch, seqlen, dm)
+    out = (y2 @ params.out_proj.to(u.dtype)).view(batch, seqlen, params.out_proj.shape[1])
     return out, SISOState(ssm=fs, k=fk, v=fv, phi=phi_final)
 
 

@@ -784,3 +784,15 @@ def test_segment_without_a_skip(m3, dev, grad_mode):
     assert torch.equal(got, ref)
     for a, b in zip(sg, sr):
         assert torch.equal(a, b)
+
+
+def test_segment_with_an_out_proj_of_another_width(m3, dev):
+    """A segment's out_proj may map to another width than d_model's: the columns of the
+    product are the wider one's first (one operand rounding where the library sums them in
+    another order)."""
+    cfg, p, u, st = _segment_case(m3, dev)
+    with torch.no_grad():
+        full = m3.mamba3_siso_layer(p, u, cfg, state=st)[0]
+        got = m3.mamba3_siso_layer(p._replace(out_proj=p.out_proj[:, :128]), u, cfg, state=st)[0]
+    assert tuple(got.shape) == (2, 128, 128)
+    assert_bf16_bound(got, cpu(full[..., :128]), what="out")
