@@ -359,6 +359,14 @@ class _LayerFn(torch.autograd.Function):
                 None)
 
 
+def has_tangent(*tensors) -> bool:
+    """Whether one of ``tensors`` (None passed over) carries a forward-mode tangent
+    (``torch.no_grad`` does not switch that mode off). Launches outside an autograd node would
+    drop it without a word; the nodes have no forward-mode rule and refuse it."""
+    return fwd_ad._current_level >= 0 and any(
+        t is not None and fwd_ad.unpack_dual(t).tangent is not None for t in tensors)
+
+
 def _segment_fused_ok(params: SISOParams, u: Tensor, cfg: SISOConfig, state) -> bool:
     """Whether a segment with a carried state runs as `_segment_forward`: no gradient is taken,
     `_fused_ok` holds, the projection's own rows are 16-byte aligned, and the carry and the
@@ -370,9 +378,7 @@ def _segment_fused_ok(params: SISOParams, u: Tensor, cfg: SISOConfig, state) -> 
     tensors = [t for t in (u, *params, *state) if t is not None]   # d_skip may be None
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return False
-    # a forward-mode tangent would be dropped here without a word; the composed path's nodes refuse it
-    if fwd_ad._current_level >= 0 and any(
-            fwd_ad.unpack_dual(t).tangent is not None for t in tensors):
+    if has_tangent(*tensors):
         return False
     b, h, n = u.shape[0], cfg.nheads, cfg.d_state
     vectors = (params.dt_bias, params.b_norm_weight, params.c_norm_weight)

@@ -389,8 +389,8 @@ def _add_residual(x: Tensor, y: Tensor) -> Tensor:
 
 def _decode_fused_ok(params: LMParams, x: Tensor, cfg: LMConfig) -> bool:
     """Whether a token step folds its norms, gates and head into the products
-    (``m3s_gemv_fused``): one or two rows without autograd, bf16 products, a tied head, widths
-    the kernels take, and dense tensors. Other steps run them one by one."""
+    (``m3s_gemv_fused``): one or two rows without autograd of either mode, bf16 products, a tied
+    head, widths the kernels take, and dense tensors. Other steps run them one by one."""
     c, d = cfg.siso, cfg.d_model
     if (torch.is_grad_enabled() or not x.is_cuda or not 1 <= x.shape[0] <= K.FUSED_ROWS_MAX
             or _mm_dtype(cfg) != torch.bfloat16 or x.dtype not in (torch.float32, torch.bfloat16)
@@ -412,7 +412,7 @@ def _decode_fused_ok(params: LMParams, x: Tensor, cfg: LMConfig) -> bool:
                    for w in ws):
             return False
     return all(g.dtype == torch.float32 and g.is_contiguous() and g.data_ptr() % 16 == 0
-               for g in gains) and bool(params.blocks)
+               for g in gains) and bool(params.blocks) and not LY.has_tangent(x, *lm_leaves(params))
 
 
 def _decode_step_fused(params: LMParams, x: Tensor, states: list, cfg: LMConfig):

@@ -397,3 +397,25 @@ def test_decode_step_refuses_too_few_states(m3, dev, rows):
     with torch.no_grad():
         with pytest.raises(IndexError):
             M.lm_decode_step(params, tok, M.zero_states(cfg, rows, device=dev)[:1], cfg)
+
+
+@pytest.mark.parametrize("rows", [1, 3])   # folded and pass by pass
+@pytest.mark.parametrize("where", ["embed", "norm_gain", "mlp_norm_gain", "final_norm"])
+def test_decode_step_refuses_a_forward_mode_tangent(m3, dev, rows, where):
+    """``torch.no_grad`` leaves forward mode on: a tangent that reaches a norm is refused by
+    its node, at one row too, and not dropped."""
+    import torch.autograd.forward_ad as fwd_ad
+    M = m3.model
+    cfg = M.LMConfig(vocab_size=64, n_layers=2, d_intermediate=256, siso=m3.SISOConfig(d_model=256))
+    params = M.decode_params(M.init_lm(cfg, 0, device=dev), cfg)
+    tok = torch.zeros(rows, dtype=torch.int64, device=dev)
+    dual = lambda t: fwd_ad.make_dual(t, torch.ones_like(t))  # noqa: E731
+    with torch.no_grad(), fwd_ad.dual_level():
+        assert M._decode_fused_ok(params, params.embed[:1], cfg)
+        if where in ("embed", "final_norm"):
+            params = params._replace(**{where: dual(getattr(params, where))})
+        else:
+            last = params.blocks[-1]
+            params.blocks[-1] = last._replace(**{where: dual(getattr(last, where))})
+        with pytest.raises((NotImplementedError, RuntimeError)):
+            M.lm_decode_step(params, tok, M.zero_states(cfg, rows, device=dev), cfg)
