@@ -390,9 +390,11 @@ def _add_residual(x: Tensor, y: Tensor) -> Tensor:
 def _decode_fused_ok(params: LMParams, x: Tensor, cfg: LMConfig) -> bool:
     """Whether a token step folds its norms, gates and head into the products
     (``m3s_gemv_fused``): one or two rows without autograd of either mode, bf16 products, a tied
-    head, widths the kernels take, and dense tensors. Other steps run them one by one."""
+    head, widths the kernels take, and dense tensors. Other steps run them one by one; so does a
+    traced one (``torch.jit.trace`` would record the launches' outputs as empty tensors, where it
+    refuses the autograd nodes)."""
     c, d = cfg.siso, cfg.d_model
-    if (torch.is_grad_enabled() or not x.is_cuda or not 1 <= x.shape[0] <= K.FUSED_ROWS_MAX
+    if (torch.is_grad_enabled() or torch.jit.is_tracing() or not x.is_cuda or not 1 <= x.shape[0] <= K.FUSED_ROWS_MAX
             or _mm_dtype(cfg) != torch.bfloat16 or x.dtype not in (torch.float32, torch.bfloat16)
             or not cfg.tie_head or d % 8 or d > K.FUSED_NORM_MAX or c.d_in_proj % 8
             or c.d_inner > 4096 or L.decode_headdim(c.policy_name, c.d_state, c.headdim) != c.headdim

@@ -419,3 +419,16 @@ def test_decode_step_refuses_a_forward_mode_tangent(m3, dev, rows, where):
             params.blocks[-1] = last._replace(**{where: dual(getattr(last, where))})
         with pytest.raises((NotImplementedError, RuntimeError)):
             M.lm_decode_step(params, tok, M.zero_states(cfg, rows, device=dev), cfg)
+
+
+def test_decode_step_refuses_a_trace(m3, dev, monkeypatch):
+    """``torch.jit.trace`` sees nothing of a launch: it stops at the step's autograd nodes
+    rather than return a graph of empty tensors. (The poisoned outputs' byte views stop a
+    trace by themselves, so they are off here.)"""
+    M = m3.model
+    monkeypatch.setattr(m3.kernels, "POISON_OUTPUTS", False)
+    cfg = M.LMConfig(vocab_size=64, n_layers=2, d_intermediate=256, siso=m3.SISOConfig(d_model=256))
+    params = M.decode_params(M.init_lm(cfg, 0, device=dev), cfg)
+    step = lambda t: M.lm_decode_step(params, t, M.zero_states(cfg, 1, device=dev), cfg)[0]  # noqa: E731
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        torch.jit.trace(step, (torch.zeros(1, dtype=torch.int64, device=dev),), check_trace=False)
