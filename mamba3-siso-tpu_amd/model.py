@@ -390,29 +390,31 @@ def _add_residual(x: Tensor, y: Tensor) -> Tensor:
 def _decode_fused_ok(params: LMParams, x: Tensor, cfg: LMConfig) -> bool:
     """Whether a token step folds its norms, gates and head into the products
     (``m3s_gemv_fused``): one or two rows without autograd of either mode, bf16 products, a tied
-    head, widths the kernels take, and dense tensors. Other steps run them one by one; so does a
-    traced one (``torch.jit.trace`` would record the launches' outputs as empty tensors, where it
-    refuses the autograd nodes)."""
+    head, widths the kernels take, and dense weights of the model's shapes. Other steps run them
+    one by one; so does a traced one (``torch.jit.trace`` would record the launches' outputs as
+    empty tensors, where it refuses the autograd nodes)."""
     c, d = cfg.siso, cfg.d_model
-    if (torch.is_grad_enabled() or torch.jit.is_tracing() or not x.is_cuda or not 1 <= x.shape[0] <= K.FUSED_ROWS_MAX
+    if (torch.is_grad_enabled() or torch.jit.is_tracing() or not x.is_cuda
+            or not 1 <= x.shape[0] <= K.FUSED_ROWS_MAX
             or _mm_dtype(cfg) != torch.bfloat16 or x.dtype not in (torch.float32, torch.bfloat16)
             or not cfg.tie_head or d % 8 or d > K.FUSED_NORM_MAX or c.d_in_proj % 8
             or c.d_inner > 4096 or L.decode_headdim(c.policy_name, c.d_state, c.headdim) != c.headdim
             or params.embed.dtype != x.dtype or not params.embed.is_contiguous()
             or params.embed.data_ptr() % 16):
         return False
-    gains = [params.final_norm]
+    gains, mats = [params.final_norm], []
     for b in params.blocks:
-        ws = [b.siso.in_proj, b.siso.out_proj]
+        mats += [(b.siso.in_proj, (d, c.d_in_proj)), (b.siso.out_proj, (c.d_inner, d))]
         gains.append(b.norm_gain)
         if b.mlp is not None:
-            ws += b.mlp
+            di = b.mlp.fc2.shape[0]
+            mats += [(b.mlp.fc1, (d, 2 * di)), (b.mlp.fc2, (di, d))]
             gains.append(b.mlp_norm_gain)
-            if b.mlp.fc2.shape[0] % 8 or b.mlp.fc2.shape[0] > 4096:
+            if di % 8 or di > 4096:
                 return False
-        if not all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0
-                   for w in ws):
-            return False
+    if not all(w.dtype == torch.bfloat16 and tuple(w.shape) == s and w.is_contiguous()
+               and w.data_ptr() % 16 == 0 for w, s in mats):
+        return False
     return all(g.dtype == torch.float32 and g.is_contiguous() and g.data_ptr() % 16 == 0
                for g in gains) and bool(params.blocks) and not LY.has_tangent(x, *lm_leaves(params))
 

@@ -432,3 +432,21 @@ def test_decode_step_refuses_a_trace(m3, dev, monkeypatch):
     step = lambda t: M.lm_decode_step(params, t, M.zero_states(cfg, 1, device=dev), cfg)[0]  # noqa: E731
     with torch.no_grad(), pytest.raises(RuntimeError):
         torch.jit.trace(step, (torch.zeros(1, dtype=torch.int64, device=dev),), check_trace=False)
+
+
+@pytest.mark.parametrize("rows", [1, 3])
+def test_decode_step_with_a_wider_in_proj(m3, dev, rows):
+    """The step reads the first d_in_proj columns of a wider product, whatever its width: as
+    with the weight itself (one bf16 rounding of a projection entry where the library sums it
+    in another order)."""
+    M = m3.model
+    cfg = M.LMConfig(vocab_size=64, n_layers=1, d_intermediate=0, siso=m3.SISOConfig(d_model=256))
+    params = M.decode_params(M.init_lm(cfg, 0, device=dev), cfg)
+    b = params.blocks[0]
+    pad = torch.cat([b.siso.in_proj, b.siso.in_proj[:, :3]], dim=1).contiguous()
+    wide = params._replace(blocks=[b._replace(siso=b.siso._replace(in_proj=pad))])
+    tok = torch.arange(rows, device=dev)
+    with torch.no_grad():
+        got, ref = (M.lm_decode_step(p, tok, M.zero_states(cfg, rows, device=dev), cfg)[0]
+                    for p in (wide, params))
+    assert_maxrel(got, cpu(ref), 3e-2, "logits")
