@@ -2056,8 +2056,9 @@ static int64_t bwd_split_floats(const Split& sp, int64_t nseq, int nc, int N, in
   return split_floats(sp, nseq, nc, N, P, true) + rows * (2 * N + N * P);
 }
 
+// `spare`: workspace bytes past the per-head rows; a split needs bwd_split_floats of them.
 template <typename MT, int C, int N, int P>
-static int32_t launch_bwd(BwdParams prm, int grid, hipStream_t stream) {
+static int32_t launch_bwd(BwdParams prm, int grid, int64_t spare, hipStream_t stream) {
   bool done = false;
   const bool strips = prm.pstr != nullptr;
   const int nseq = grid;
@@ -2065,7 +2066,8 @@ static int32_t launch_bwd(BwdParams prm, int grid, hipStream_t stream) {
   if constexpr (std::is_same<MT, bf16>::value && N % 64 == 0 && C % 64 == 0 && C <= N &&
                 N / 16 <= 8) {   // N <= 128: a strip's row pairs in one wave (phi strips)
     if (bwd_fits_rsrc(prm, N, P)) {
-      if (!strips) prm.split = plan_split(nseq, prm.nc, C, kBwdMinSaved);
+      const Split sp = plan_split(nseq, prm.nc, C, kBwdMinSaved);
+      if (!strips && 4 * bwd_split_floats(sp, nseq, prm.nc, N, P) <= spare) prm.split = sp;
       if (prm.split.segs > 1) {
         const int rem = nseq - prm.split.whole;
         const int64_t nsh = (int64_t)rem * prm.split.shares(prm.nc, true);
@@ -2143,11 +2145,15 @@ int32_t bwd_supported(int dtype, int chunk, int n, int pdim) {
 
 }  // namespace m3s
 
+// Bytes of the per-head rows.
+static int64_t bwd_rows_bytes(int dtype, int batch, int seqlen, int nheads, int state_dim) {
+  return 2 * (int64_t)batch * nheads * seqlen * state_dim * (dtype == M3S_DTYPE_BF16 ? 2 : 4);
+}
+
 extern "C" int64_t m3s_bwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t seqlen,
                                            int32_t nheads, int32_t state_dim) {
   using namespace m3s;
-  const int64_t el = dtype == M3S_DTYPE_BF16 ? 2 : 4;
-  const int64_t rows = 2 * (int64_t)batch * nheads * seqlen * state_dim * el;
+  const int64_t rows = bwd_rows_bytes(dtype, batch, seqlen, nheads, state_dim);
   // a split's scratch, at whichever chunk needs the most (the chunk is not an argument)
   int64_t split = 0;
   if (dtype == M3S_DTYPE_BF16 && batch > 0 && nheads > 0)
@@ -2160,9 +2166,8 @@ extern "C" int64_t m3s_bwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t
   return rows + 4 * split;
 }
 
-extern "C" int32_t m3s_bwd(const m3s_bwd_args* a, void* stream) {
+static int32_t bwd_run(const m3s_bwd_args* a, int64_t workspace_bytes, void* stream) {
   using namespace m3s;
-  clear_error();
   M3S_REQUIRE(a != nullptr, "m3s_bwd: args is NULL");
   M3S_REQUIRE(a->struct_size == (int32_t)sizeof(m3s_bwd_args),
               "m3s_bwd: struct_size %d != %d (ABI mismatch)", a->struct_size,
@@ -2203,6 +2208,9 @@ extern "C" int32_t m3s_bwd(const m3s_bwd_args* a, void* stream) {
                   (Nr == 0 || a->dphi) && a->workspace && aligned16(a->workspace),
               "m3s_bwd: an output or workspace pointer is NULL or misaligned");
   M3S_REQUIRE((int64_t)B * H < (1ll << 31), "m3s_bwd: B*H too large");
+  const int64_t spare = workspace_bytes - bwd_rows_bytes(a->dtype, B, L, H, N);
+  M3S_REQUIRE(spare >= 0, "m3s_bwd: workspace of %lld bytes is smaller than the per-head rows' %lld",
+              (long long)workspace_bytes, (long long)(workspace_bytes - spare));
 
   BwdParams prm{};
   prm.B = B; prm.L = L; prm.H = H; prm.Nr = Nr; prm.nc = L / C;
@@ -2231,9 +2239,20 @@ extern "C" int32_t m3s_bwd(const m3s_bwd_args* a, void* stream) {
   const int grid = B * H;
 #define X(MT, CC, NN, PP)                                              \
   if (a->dtype == bcode<MT>() && C == CC && N == NN && P == PP)        \
-    return launch_bwd<MT, CC, NN, PP>(prm, grid, s);
+    return launch_bwd<MT, CC, NN, PP>(prm, grid, spare, s);
   M3S_BWD_CONFIGS(X)
 #undef X
   set_error("m3s_bwd: unreachable dispatch");
   return M3S_ERR_UNSUPPORTED;
+}
+
+extern "C" int32_t m3s_bwd_ws(const m3s_bwd_args* a, int64_t workspace_bytes, void* stream) {
+  m3s::clear_error();
+  return bwd_run(a, workspace_bytes, stream);
+}
+
+extern "C" int32_t m3s_bwd(const m3s_bwd_args* a, void* stream) {
+  m3s::clear_error();
+  const bool ok = a && a->struct_size == (int32_t)sizeof(m3s_bwd_args);   // bwd_run refuses it otherwise
+  return bwd_run(a, ok ? bwd_rows_bytes(a->dtype, a->batch, a->seqlen, a->nheads, a->state_dim) : 0, stream);
 }

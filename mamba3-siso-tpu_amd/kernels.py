@@ -777,7 +777,8 @@ def siso_backward_kernel(
     dkb = empty(batch, nheads, state_dim, **f32)
     kfin = empty(batch, nheads, state_dim, **f32)
     dseed = empty(batch, nheads, headdim, state_dim, **f32)
-    ws_bytes = _lib.load().m3s_bwd_workspace_bytes(dcode, batch, seqlen, nheads, state_dim)
+    lib = _lib.load()
+    ws_bytes = lib.m3s_bwd_workspace_bytes(dcode, batch, seqlen, nheads, state_dim)
     workspace = empty(ws_bytes, device=dev, dtype=torch.uint8)
 
     a = _lib.BwdArgs()
@@ -797,7 +798,7 @@ def siso_backward_kernel(
     a.dphi, a.dq_bias, a.dk_bias = dphi.data_ptr(), dqb.data_ptr(), dkb.data_ptr()
     a.k_final, a.dseed_ssm = kfin.data_ptr(), dseed.data_ptr()
     a.workspace = workspace.data_ptr()
-    _lib.launch(_lib.load().m3s_bwd, a, dev, "m3s_bwd")
+    _lib.launch(lambda args, stream: lib.m3s_bwd_ws(args, ws_bytes, stream), a, dev, "m3s_bwd")
     return KernelGrads(dq=dq, dk=dk, dv=dv, dadt=dadt, dqk_diag=dqk, dscale=dscale, dphi=dphi,
                        dz=dz, uw=uw, dq_bias=dqb.sum(0), dk_bias=dkb.sum(0), k_final=kfin,
                        dseed_ssm=dseed)

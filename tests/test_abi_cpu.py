@@ -158,6 +158,30 @@ def test_workspace_size(lib):
     assert h.m3s_bwd_workspace_bytes(lib.DTYPE_F32, 1, 64, 2, 16) == 2 * 2 * 64 * 16 * 4
 
 
+def test_backward_workspace_is_checked_without_a_launch(lib):
+    """``m3s_bwd_ws`` refuses a workspace below the per-head rows, 2 B H L N elements, which
+    are all that ``m3s_bwd`` asks for; the size for cut sequences is not monotone in B*H."""
+    h = lib.load()
+    rows = lambda n_seq, L: 2 * n_seq * L * 128 * 2  # noqa: E731
+    assert h.m3s_bwd_workspace_bytes(lib.DTYPE_BF16, 1, 1024, 128, 128) > rows(128, 1024)
+    assert h.m3s_bwd_workspace_bytes(lib.DTYPE_BF16, 1, 1024, 130, 128) == rows(130, 1024)
+    assert rows(130, 1024) < h.m3s_bwd_workspace_bytes(lib.DTYPE_BF16, 1, 1024, 128, 128)
+    a = lib.BwdArgs()
+    a.struct_size = ctypes.sizeof(lib.BwdArgs)
+    a.batch, a.seqlen, a.nheads, a.headdim, a.state_dim, a.n_angles, a.chunk = 1, 512, 2, 64, 128, 0, 128
+    a.dtype = lib.DTYPE_BF16
+    dense = lib.Bhlp(0x1000, 2 * 512 * 64, 512 * 64, 64)
+    a.dy = a.v = a.dv = dense
+    for f in ("ybar", "q", "k", "adt", "gamma", "scale", "phi", "q_bias", "k_bias", "chunk_states", "dq",
+              "dk", "dadt", "dqk_diag", "dscale", "uw", "dphi", "dq_bias", "dk_bias", "k_final",
+              "dseed_ssm", "workspace"):
+        setattr(a, f, 0x1000)
+    for size in (rows(2, 512) - 1, 0, -1):
+        assert h.m3s_bwd_ws(ctypes.byref(a), size, None) == lib.ERR_INVALID
+        assert b"workspace" in h.m3s_last_error() and b"per-head rows" in h.m3s_last_error()
+    assert h.m3s_bwd_ws(None, 0, None) == h.m3s_bwd(None, None) == lib.ERR_INVALID
+
+
 def test_prep_arguments_are_checked_without_a_launch(lib):
     h = lib.load()
     assert h.m3s_prep_fwd(None, None) == lib.ERR_INVALID

@@ -144,3 +144,44 @@ def test_split_backward_equals_whole(m3, dev, h, nc, chunk, n, nr, gate, final):
     for name in ("dq_bias", "dk_bias"):   # at most 16 segments' f32 sums in another order
         a, b = getattr(got, name), getattr(ref, name)[:h]
         assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max()), name
+
+
+@pytest.mark.parametrize("entry", ["m3s_bwd", "m3s_bwd_ws"])
+def test_backward_with_the_rows_alone_is_not_split(m3, dev, monkeypatch, entry):
+    """``m3s_bwd``, and ``m3s_bwd_ws`` with a workspace too small for a split, stay within the
+    per-head rows (a guard after them keeps its bytes) and give the split scan's bits,
+    the bias sums to f32 rounding."""
+    b, h, L, n, p = 1, 3, 896, 128, 64
+    lib, K = m3._lib, m3.kernels
+    _, d = boundary_inputs(b, h, L, n, p, 32, "bf16", seed=5)
+    args = fwd_args(d)
+    res = m3.siso_forward(*args, chunk=128, save_residuals=True)[4]
+
+    def run():
+        return m3.siso_backward_kernel(d["dy"], res.ybar, d["z"], *args[:9], res.chunk_states,
+                                       d_skip=d["d_skip"], chunk=128)
+
+    ref = run()
+    rows, need = 2 * h * L * n * 2, lib.load().m3s_bwd_workspace_bytes(lib.DTYPE_BF16, b, L, h, n)
+    assert need > rows
+    guard = torch.full((need,), 0x5A, dtype=torch.uint8, device=dev)
+    launch, seen = lib.launch, []
+
+    def whole(fn, a, dev_, what):
+        if what != "m3s_bwd":
+            return launch(fn, a, dev_, what)
+        seen.append(a.workspace)
+        a.workspace = guard.data_ptr()
+        if entry == "m3s_bwd":
+            return launch(lib.load().m3s_bwd, a, dev_, what)
+        return launch(lambda x, s: lib.load().m3s_bwd_ws(x, rows + 4096, s), a, dev_, what)
+
+    monkeypatch.setattr(lib, "launch", whole)
+    got = run()
+    assert len(seen) == 1 and bool((guard[rows:] == 0x5A).all()) and not bool((guard[:rows] == 0x5A).all())
+    for name in got._fields:
+        x, y = getattr(got, name), getattr(ref, name)
+        if name in ("dq_bias", "dk_bias"):   # at most 16 segments' f32 sums in another order
+            assert float((x - y).abs().max()) <= 1e-5 * float(y.abs().max()), name
+        else:
+            assert torch.equal(x, y), name
