@@ -521,7 +521,8 @@ int64_t m3s_rms_bwd_workspace_bytes(int32_t width);
 
 /* Bytes of m3s_fwd_ws's workspace: the states and decays of the pieces of the sequences
  * that the scan cuts into segments, where B*H sequences leave its last round of workgroups
- * half empty or emptier; 0 where none is cut. No counterpart in the reference. -1 on bad
+ * half empty or emptier; 0 where none is cut, and where the states would take more than
+ * 1 GiB. No counterpart in the reference. -1 on bad
  * dimensions or a shape without a kernel. */
 int64_t m3s_fwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t seqlen, int32_t nheads,
                                 int32_t headdim, int32_t state_dim, int32_t chunk);

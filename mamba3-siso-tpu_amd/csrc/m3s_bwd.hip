@@ -2066,7 +2066,7 @@ static int32_t launch_bwd(BwdParams prm, int grid, int64_t spare, hipStream_t st
   if constexpr (std::is_same<MT, bf16>::value && N % 64 == 0 && C % 64 == 0 && C <= N &&
                 N / 16 <= 8) {   // N <= 128: a strip's row pairs in one wave (phi strips)
     if (bwd_fits_rsrc(prm, N, P)) {
-      const Split sp = plan_split(nseq, prm.nc, C, kBwdMinSaved);
+      const Split sp = plan_split(nseq, prm.nc, C, kBwdMinSaved, N * P * 4);
       if (!strips && 4 * bwd_split_floats(sp, nseq, prm.nc, N, P) <= spare) prm.split = sp;
       if (prm.split.segs > 1) {
         const int rem = nseq - prm.split.whole;
@@ -2160,7 +2160,7 @@ extern "C" int64_t m3s_bwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t
     for (int c : {64, 128})
       if (bwd_supported(dtype, c, state_dim, 64) && seqlen > 0 && seqlen % c == 0) {
         const int64_t nseq = (int64_t)batch * nheads;
-        const Split sp = plan_split(nseq, seqlen / c, c, kBwdMinSaved);
+        const Split sp = plan_split(nseq, seqlen / c, c, kBwdMinSaved, (int64_t)state_dim * 64 * 4);
         split = std::max(split, bwd_split_floats(sp, nseq, seqlen / c, state_dim, 64));
       }
   return rows + 4 * split;

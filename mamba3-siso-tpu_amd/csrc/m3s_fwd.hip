@@ -1961,7 +1961,7 @@ static int32_t launch_fwd(FwdParams prm, int grid, hipStream_t stream) {
   prm.split = Split{grid, 1};
   if constexpr (can_split<MT, C, N, P>()) {
     if (prm.shares != nullptr && !strips) {
-      prm.split = plan_split(grid, prm.nc, C, kFwdMinSaved);
+      prm.split = plan_split(grid, prm.nc, C, kFwdMinSaved, N * P * 4);
       prm.decay = prm.shares + (int64_t)(grid - prm.split.whole) * prm.split.shares(prm.nc, false) * N * P;
     }
   }
@@ -2080,8 +2080,8 @@ extern "C" int64_t m3s_fwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t
 #undef X
   const int64_t nseq = (int64_t)batch * nheads;
   const int nc = seqlen / chunk;
-  return 4 * split_floats(plan_split(nseq, nc, chunk, kFwdMinSaved), nseq, nc, state_dim, headdim,
-                          false);
+  const Split sp = plan_split(nseq, nc, chunk, kFwdMinSaved, (int64_t)state_dim * headdim * 4);
+  return 4 * split_floats(sp, nseq, nc, state_dim, headdim, false);
 }
 
 extern "C" int32_t m3s_fwd(const m3s_fwd_args* a, void* stream) {

@@ -35,8 +35,13 @@ struct Split {
 // L=4096 207 -> 78, L=8192 403 -> 131 (of which the shares 14 / 20 / 40 and the chain 7 / 10
 // / 17); three sequences' worth of rounds, B=16 L=2048 H=24: 247 -> 229; B=1 L=896 H=24, six
 // chunks saved: 53 -> 37; B=4 L=512, two chunks saved, was slower split (37 -> 41).
+// No split either where its states, `state_bytes` per chunk of each cut sequence (256 B a token
+// and head at N = 128, P = 64; a layer's x, z and y rows are 384), come to more than kMaxBytes.
+// Up to there it is always the faster: H=32 L=131072 (1 GiB) 6.25 -> 2.35 ms, H=4 L=1048576
+// (1 GiB) 50 -> 17 ms, though each raw-mode share walks the angles of the chunks before it.
 constexpr int kMaxSegs = 16;
-inline Split plan_split(int64_t nseq, int nc, int chunk, int min_saved) {
+constexpr int64_t kMaxBytes = int64_t(1) << 30;
+inline Split plan_split(int64_t nseq, int nc, int chunk, int min_saved, int64_t state_bytes) {
   Split sp{(int)nseq, 1};
   const int rem = (int)(nseq % kFirstRound);
   if (rem == 0) return sp;
@@ -44,6 +49,7 @@ inline Split plan_split(int64_t nseq, int nc, int chunk, int min_saved) {
   segs = segs < nc ? segs : nc;
   segs = segs < kMaxSegs ? segs : kMaxSegs;
   if (segs < 2 || (nc - (nc + segs - 1) / segs) * chunk < min_saved) return sp;
+  if (rem * (int64_t)nc * state_bytes > kMaxBytes) return sp;
   sp.whole = (int)(nseq - rem);
   sp.segs = segs;
   return sp;

@@ -196,12 +196,23 @@ def _head_sum(t: Tensor, r: int, dim: int = 1) -> Tensor:
     return t.unflatten(dim, (t.shape[dim] // r, r)).sum(dim + 1)
 
 
+def _scratch(nbytes: int, dev: torch.device, least: int = 0) -> Optional[Tensor]:
+    """``nbytes`` of scratch for a scan that cuts sequences into segments; where the device has
+    no room for them, the ``least`` bytes that the scan of whole sequences needs (None: 0)."""
+    if nbytes > least:
+        try:
+            return empty(nbytes, device=dev, dtype=torch.uint8)
+        except torch.cuda.OutOfMemoryError:
+            pass
+    return empty(least, device=dev, dtype=torch.uint8) if least > 0 else None
+
+
 def _launch_fwd(a: "_lib.FwdArgs", dev: torch.device) -> None:
     """``m3s_fwd_ws`` on the current stream, with the scratch its shape asks for."""
     lib = _lib.load()
     nbytes = lib.m3s_fwd_workspace_bytes(a.dtype, a.batch, a.seqlen, a.nheads, a.headdim,
                                          a.state_dim, a.chunk)
-    ws = empty(nbytes, device=dev, dtype=torch.uint8) if nbytes > 0 else None
+    ws = _scratch(nbytes, dev)
     _lib.launch(lambda args, stream: lib.m3s_fwd_ws(args, _lib.ptr(ws), max(nbytes, 0), stream),
                 a, dev, "m3s_fwd")
 
@@ -778,8 +789,8 @@ def siso_backward_kernel(
     kfin = empty(batch, nheads, state_dim, **f32)
     dseed = empty(batch, nheads, headdim, state_dim, **f32)
     lib = _lib.load()
-    ws_bytes = lib.m3s_bwd_workspace_bytes(dcode, batch, seqlen, nheads, state_dim)
-    workspace = empty(ws_bytes, device=dev, dtype=torch.uint8)
+    workspace = _scratch(lib.m3s_bwd_workspace_bytes(dcode, batch, seqlen, nheads, state_dim), dev,
+                         2 * batch * nheads * seqlen * state_dim * mt.itemsize)
 
     a = _lib.BwdArgs()
     a.struct_size = ctypes.sizeof(_lib.BwdArgs)
@@ -798,7 +809,7 @@ def siso_backward_kernel(
     a.dphi, a.dq_bias, a.dk_bias = dphi.data_ptr(), dqb.data_ptr(), dkb.data_ptr()
     a.k_final, a.dseed_ssm = kfin.data_ptr(), dseed.data_ptr()
     a.workspace = workspace.data_ptr()
-    _lib.launch(lambda args, stream: lib.m3s_bwd_ws(args, ws_bytes, stream), a, dev, "m3s_bwd")
+    _lib.launch(lambda args, stream: lib.m3s_bwd_ws(args, workspace.numel(), stream), a, dev, "m3s_bwd")
     return KernelGrads(dq=dq, dk=dk, dv=dv, dadt=dadt, dqk_diag=dqk, dscale=dscale, dphi=dphi,
                        dz=dz, uw=uw, dq_bias=dqb.sum(0), dk_bias=dkb.sum(0), k_final=kfin,
                        dseed_ssm=dseed)

@@ -182,6 +182,23 @@ def test_backward_workspace_is_checked_without_a_launch(lib):
     assert h.m3s_bwd_ws(None, 0, None) == h.m3s_bwd(None, None) == lib.ERR_INVALID
 
 
+def test_split_scratch_is_bounded(lib):
+    """The states of cut sequences take at most 1 GiB; past it nothing is cut, either way."""
+    h = lib.load()
+    fwd = lambda b, L, nh, n=128: h.m3s_fwd_workspace_bytes(lib.DTYPE_BF16, b, L, nh, 64, n, 128)  # noqa: E731
+    bwd = lambda b, L, nh, n=128: (h.m3s_bwd_workspace_bytes(lib.DTYPE_BF16, b, L, nh, n)  # noqa: E731
+                                   - 2 * b * nh * L * n * 2)
+    for size in (fwd, bwd):
+        assert size(1, 65536, 32) > 0
+        assert size(1, 262144, 32) == size(4, 131072, 32) == size(1, 1 << 21, 4) == 0
+        for L in (2 ** i * 128 for i in range(1, 16)):
+            for nh in (1, 3, 32, 100, 128, 129, 300):
+                for n in (64, 128):
+                    # the decays, bias rows and the backward's one state a segment ride on top
+                    assert 0 <= size(1, L, nh, n) <= (1 << 30) + (1 << 25), (L, nh, n)
+    assert 0 < fwd(1, 131072, 32) <= 1 << 30 and fwd(1, 131072 + 128, 32) == 0
+
+
 def test_prep_arguments_are_checked_without_a_launch(lib):
     h = lib.load()
     assert h.m3s_prep_fwd(None, None) == lib.ERR_INVALID
