@@ -519,13 +519,17 @@ int64_t m3s_norm_bwd_workspace_bytes(int32_t width);
  * counterpart in the reference. -1 on a bad width. */
 int64_t m3s_rms_bwd_workspace_bytes(int32_t width);
 
-/* Bytes of m3s_fwd_ws's workspace: the states and decays of the pieces of the sequences
+/* The most bytes of m3s_fwd_ws's workspace for a shape: the states and decays of the pieces of the sequences
  * that the scan cuts into segments, where B*H sequences leave its last round of workgroups
  * half empty or emptier; 0 where none is cut, and where the states would take more than
  * 1 GiB. No counterpart in the reference. -1 on bad
  * dimensions or a shape without a kernel. */
 int64_t m3s_fwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t seqlen, int32_t nheads,
                                 int32_t headdim, int32_t state_dim, int32_t chunk);
+/* The bytes that this very call uses: as above, or 0 where its mode, angles or strides leave
+ * every sequence whole (compact phi; what the bf16 kernel cannot address). Looks at the
+ * sizes, strides and which pointers are set. -1 as above. */
+int64_t m3s_fwd_scratch_bytes(const m3s_fwd_args* args);
 
 /* Bytes of m3s_decode_scan_ws's workspace: the carried k and phi of a run whose few states are
  * split by rows; 0 where none is. No counterpart in the reference. -1 on bad dimensions. */
@@ -534,8 +538,8 @@ int64_t m3s_decode_scan_workspace_bytes(int32_t batch, int32_t steps, int32_t nh
 
 /* m3s_fwd is m3s_fwd_ws without a workspace: every sequence stays in one workgroup. */
 int32_t m3s_fwd(const m3s_fwd_args* args, void* stream);
-/* `workspace`: m3s_fwd_workspace_bytes() bytes of scratch (16-aligned; `workspace_bytes` is
- * its size), or NULL. Same results to float32 rounding of the carried state. */
+/* `workspace`: m3s_fwd_scratch_bytes() bytes of scratch (16-aligned; `workspace_bytes` is its
+ * size), or NULL. The same bits with and without. */
 int32_t m3s_fwd_ws(const m3s_fwd_args* args, void* workspace, int64_t workspace_bytes,
                    void* stream);
 /* m3s_bwd is m3s_bwd_ws with a workspace of the per-head rows alone: no sequence is cut. */

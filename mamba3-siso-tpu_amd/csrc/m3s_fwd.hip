@@ -1955,20 +1955,40 @@ static int launch_shares(const FwdParams& prm, hipStream_t stream) {
 template <typename MT, int C, int N, int P>
 constexpr bool can_split() { return std::is_same<MT, bf16>::value && N % 64 == 0 && C % 64 == 0; }
 
+// Raw mode on the bf16 kernel: it addresses the raw slices and every stream through buffer
+// descriptors, and compiles raw_nrb_max blocks of built angles.
+template <typename MT, int C, int N, int P>
+static bool raw_fast(const FwdParams& p) {
+  return fits_rsrc(p, N, P) && p.Nr <= 32 * raw_nrb_max<MT, C, N, P>() &&
+         ((int64_t)(p.L - 1) * p.sc_st + p.sc_span) * (int64_t)sizeof(MT) < (1ll << 31);
+}
+
+// Scratch bytes of this call: 0 where launch_fwd cuts nothing (compact phi and what the
+// generic kernel takes are never cut).
+template <typename MT, int C, int N, int P>
+static int64_t scratch_bytes(const FwdParams& p) {
+  if constexpr (can_split<MT, C, N, P>()) {
+    const bool fast = p.sc ? raw_fast<MT, C, N, P>(p) : !p.pstr && fits_rsrc(p, N, P);
+    const int64_t nseq = (int64_t)p.B * p.H;
+    if (fast)
+      return 4 * split_floats(plan_split(nseq, p.nc, C, kFwdMinSaved, N * P * 4), nseq, p.nc, N, P, false);
+  }
+  return 0;
+}
+
+// `prm.shares` is set where scratch_bytes asks for it and the caller brings it.
 template <typename MT, int C, int N, int P>
 static int32_t launch_fwd(FwdParams prm, int grid, hipStream_t stream) {
   const bool strips = prm.pstr != nullptr;
   prm.split = Split{grid, 1};
   if constexpr (can_split<MT, C, N, P>()) {
-    if (prm.shares != nullptr && !strips) {
+    if (prm.shares != nullptr) {
       prm.split = plan_split(grid, prm.nc, C, kFwdMinSaved, N * P * 4);
       prm.decay = prm.shares + (int64_t)(grid - prm.split.whole) * prm.split.shares(prm.nc, false) * N * P;
     }
   }
   if (prm.sc != nullptr) {   // raw mode: the bf16 kernel where it applies, else the generic one
-    // the bf16 kernel addresses the raw slices and every stream through buffer descriptors
-    const bool fast = fits_rsrc(prm, N, P) &&
-                      ((int64_t)(prm.L - 1) * prm.sc_st + prm.sc_span) * (int64_t)sizeof(MT) < (1ll << 31);
+    const bool fast = raw_fast<MT, C, N, P>(prm);
     if constexpr (raw_nrb_max<MT, C, N, P>() >= 1) {
       if (fast && prm.Nr <= 32) {
         grid = launch_shares<C, N, P, 1, true>(prm, stream);
@@ -1977,7 +1997,7 @@ static int32_t launch_fwd(FwdParams prm, int grid, hipStream_t stream) {
       }
     }
     if constexpr (raw_nrb_max<MT, C, N, P>() >= 2) {
-      if (fast && prm.Nr <= 64) {
+      if (fast) {
         grid = launch_shares<C, N, P, 2, true>(prm, stream);
         hipLaunchKernelGGL((fwd_bf16_kernel<C, N, P, 2, true>), dim3(grid), dim3(C / 16 * 64), 0, stream, prm);
         return launch_status("m3s_fwd");
@@ -2064,6 +2084,54 @@ int32_t fwd_raw_supported_impl(int dtype, int chunk, int n, int pdim, int nr) {
   return fwd_supported(dtype, chunk, n, pdim);
 }
 
+// The kernels' parameters of a call (no pointer is followed; chunk > 0).
+static FwdParams fwd_params(const m3s_fwd_args* a) {
+  const bool raw = a->raw != 0;
+  const bool strips = !raw && (a->theta_table || a->phi_dt || a->phi_strips);
+  FwdParams prm{};
+  prm.B = a->batch; prm.L = a->seqlen; prm.H = a->nheads; prm.Nr = a->n_angles;
+  prm.nc = a->seqlen / a->chunk;
+  prm.has_d = a->has_d; prm.has_z = a->has_z; prm.has_seed = a->has_seed;
+  prm.save = a->save_residuals;
+  prm.q = a->q; prm.k = a->k;
+  prm.v = a->v.ptr; prm.v_sb = a->v.stride_b; prm.v_sh = a->v.stride_h; prm.v_st = a->v.stride_t;
+  prm.z = a->has_z ? a->z.ptr : nullptr;
+  prm.z_sb = a->z.stride_b; prm.z_sh = a->z.stride_h; prm.z_st = a->z.stride_t;
+  prm.adt = a->adt; prm.gamma = a->gamma; prm.scale = a->scale; prm.phi = a->phi;
+  prm.tht = (strips || raw) ? a->theta_table : nullptr;
+  prm.pdt = strips ? a->phi_dt : nullptr;
+  prm.pstr = strips ? a->phi_strips : nullptr;
+  prm.qb = a->q_bias; prm.kb = a->k_bias; prm.dsk = a->d_skip;
+  prm.seed_ssm = a->seed_ssm; prm.seed_k = a->seed_k; prm.seed_v = a->seed_v;
+  prm.seed_coef = a->seed_coef;
+  prm.y = a->y.ptr; prm.y_sb = a->y.stride_b; prm.y_sh = a->y.stride_h; prm.y_st = a->y.stride_t;
+  prm.ybar = a->ybar; prm.cstates = a->chunk_states;
+  prm.fssm = a->final_ssm; prm.fk = a->final_k; prm.fv = a->final_v;
+  if (raw) {
+    prm.sc = a->dt_raw.ptr; prm.sc_sb = a->dt_raw.stride_b; prm.sc_st = a->dt_raw.stride_t;
+    const int esz = a->dtype == M3S_DTYPE_BF16 ? 2 : 4;
+    prm.a_off = (int)(((const char*)a->a_raw.ptr - (const char*)a->dt_raw.ptr) / esz);
+    prm.t_off = (int)(((const char*)a->trap_raw.ptr - (const char*)a->dt_raw.ptr) / esz);
+    prm.sc_span = std::max(prm.a_off, prm.t_off) + 1;
+    prm.a_floor = a->a_floor;
+    prm.dt_bias = a->dt_bias;
+    prm.tpre = a->theta_prefix;
+    prm.ctot = a->theta_chunk_totals;
+    prm.phi_init = a->phi_init;
+    prm.phi_final = a->phi_final;
+  }
+  return prm;
+}
+
+static int64_t scratch_of(const m3s_fwd_args* a, const FwdParams& prm) {
+#define X(MT, CC, NN, PP)                                                                        \
+  if (a->dtype == dtype_code<MT>() && a->chunk == CC && a->state_dim == NN && a->headdim == PP)  \
+    return scratch_bytes<MT, CC, NN, PP>(prm);
+  M3S_FWD_CONFIGS(X)
+#undef X
+  return 0;
+}
+
 }  // namespace m3s
 
 extern "C" int64_t m3s_fwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t seqlen,
@@ -2082,6 +2150,14 @@ extern "C" int64_t m3s_fwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t
   const int nc = seqlen / chunk;
   const Split sp = plan_split(nseq, nc, chunk, kFwdMinSaved, (int64_t)state_dim * headdim * 4);
   return 4 * split_floats(sp, nseq, nc, state_dim, headdim, false);
+}
+
+extern "C" int64_t m3s_fwd_scratch_bytes(const m3s_fwd_args* a) {
+  using namespace m3s;
+  if (a == nullptr || a->struct_size != (int32_t)sizeof(m3s_fwd_args) || a->batch <= 0 || a->seqlen <= 0 ||
+      a->nheads <= 0 || !fwd_supported(a->dtype, a->chunk, a->state_dim, a->headdim))
+    return -1;
+  return scratch_of(a, fwd_params(a));
 }
 
 extern "C" int32_t m3s_fwd(const m3s_fwd_args* a, void* stream) {
@@ -2116,7 +2192,6 @@ extern "C" int32_t m3s_fwd_ws(const m3s_fwd_args* a, void* workspace, int64_t wo
   M3S_REQUIRE(bhlp_ok(a->y, vec), "m3s_fwd: y null, misaligned or bad strides");
   const bool raw = a->raw != 0;
   const bool strips = !raw && (a->theta_table || a->phi_dt || a->phi_strips);
-  int a_off = 0, t_off = 0;
   if (raw) {
     M3S_REQUIRE(!a->adt && !a->gamma && !a->scale && !a->phi && !a->phi_dt && !a->phi_strips,
                 "m3s_fwd: raw mode takes the raw slices, not adt / gamma / scale / phi");
@@ -2142,8 +2217,6 @@ extern "C" int32_t m3s_fwd_ws(const m3s_fwd_args* a, void* workspace, int64_t wo
                     da / esz + H <= a->dt_raw.stride_t && dtr / esz + H <= a->dt_raw.stride_t,
                 "m3s_fwd: a_raw / trap_raw must start a fixed number of elements after dt_raw "
                 "within each row");
-    a_off = (int)(da / esz);
-    t_off = (int)(dtr / esz);
     if (!fwd_raw_supported_impl(a->dtype, C, N, P, Nr)) {
       set_error("m3s_fwd: no raw-mode kernel for dtype=%s chunk=%d state_dim=%d headdim=%d "
                 "n_angles=%d", a->dtype == M3S_DTYPE_BF16 ? "bf16" : "f32", C, N, P, Nr);
@@ -2167,40 +2240,12 @@ extern "C" int32_t m3s_fwd_ws(const m3s_fwd_args* a, void* workspace, int64_t wo
               "m3s_fwd: residual outputs NULL or misaligned");
   M3S_REQUIRE(a->final_ssm && a->final_k && a->final_v, "m3s_fwd: final state outputs NULL");
   M3S_REQUIRE((int64_t)B * H < (1ll << 31), "m3s_fwd: B*H too large");
-  const int64_t ws_need = m3s_fwd_workspace_bytes(a->dtype, B, L, H, P, N, C);
+  FwdParams prm = fwd_params(a);
+  const int64_t ws_need = scratch_of(a, prm);
   M3S_REQUIRE(workspace == nullptr || (aligned16(workspace) && workspace_bytes >= ws_need),
-              "m3s_fwd: workspace misaligned or smaller than the %lld bytes of this shape",
+              "m3s_fwd: workspace misaligned or smaller than the %lld bytes of this call",
               (long long)ws_need);
-
-  FwdParams prm{};
   prm.shares = ws_need > 0 ? static_cast<float*>(workspace) : nullptr;
-  prm.B = B; prm.L = L; prm.H = H; prm.Nr = Nr; prm.nc = L / C;
-  prm.has_d = a->has_d; prm.has_z = a->has_z; prm.has_seed = a->has_seed;
-  prm.save = a->save_residuals;
-  prm.q = a->q; prm.k = a->k;
-  prm.v = a->v.ptr; prm.v_sb = a->v.stride_b; prm.v_sh = a->v.stride_h; prm.v_st = a->v.stride_t;
-  prm.z = a->has_z ? a->z.ptr : nullptr;
-  prm.z_sb = a->z.stride_b; prm.z_sh = a->z.stride_h; prm.z_st = a->z.stride_t;
-  prm.adt = a->adt; prm.gamma = a->gamma; prm.scale = a->scale; prm.phi = a->phi;
-  prm.tht = (strips || raw) ? a->theta_table : nullptr;
-  prm.pdt = strips ? a->phi_dt : nullptr;
-  prm.pstr = strips ? a->phi_strips : nullptr;
-  prm.qb = a->q_bias; prm.kb = a->k_bias; prm.dsk = a->d_skip;
-  prm.seed_ssm = a->seed_ssm; prm.seed_k = a->seed_k; prm.seed_v = a->seed_v;
-  prm.seed_coef = a->seed_coef;
-  prm.y = a->y.ptr; prm.y_sb = a->y.stride_b; prm.y_sh = a->y.stride_h; prm.y_st = a->y.stride_t;
-  prm.ybar = a->ybar; prm.cstates = a->chunk_states;
-  prm.fssm = a->final_ssm; prm.fk = a->final_k; prm.fv = a->final_v;
-  if (raw) {
-    prm.sc = a->dt_raw.ptr; prm.sc_sb = a->dt_raw.stride_b; prm.sc_st = a->dt_raw.stride_t;
-    prm.a_off = a_off; prm.t_off = t_off; prm.sc_span = std::max(a_off, t_off) + 1;
-    prm.a_floor = a->a_floor;
-    prm.dt_bias = a->dt_bias;
-    prm.tpre = a->theta_prefix;
-    prm.ctot = a->theta_chunk_totals;
-    prm.phi_init = a->phi_init;
-    prm.phi_final = a->phi_final;
-  }
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int grid = B * H;
 #define X(MT, CC, NN, PP)                                                     \

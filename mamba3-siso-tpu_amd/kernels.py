@@ -208,10 +208,9 @@ def _scratch(nbytes: int, dev: torch.device, least: int = 0) -> Optional[Tensor]
 
 
 def _launch_fwd(a: "_lib.FwdArgs", dev: torch.device) -> None:
-    """``m3s_fwd_ws`` on the current stream, with the scratch its shape asks for."""
+    """``m3s_fwd_ws`` on the current stream, with the scratch this call uses."""
     lib = _lib.load()
-    nbytes = lib.m3s_fwd_workspace_bytes(a.dtype, a.batch, a.seqlen, a.nheads, a.headdim,
-                                         a.state_dim, a.chunk)
+    nbytes = lib.m3s_fwd_scratch_bytes(ctypes.byref(a))
     ws = _scratch(nbytes, dev)
     _lib.launch(lambda args, stream: lib.m3s_fwd_ws(args, _lib.ptr(ws), max(nbytes, 0), stream),
                 a, dev, "m3s_fwd")
@@ -789,8 +788,10 @@ def siso_backward_kernel(
     kfin = empty(batch, nheads, state_dim, **f32)
     dseed = empty(batch, nheads, headdim, state_dim, **f32)
     lib = _lib.load()
-    workspace = _scratch(lib.m3s_bwd_workspace_bytes(dcode, batch, seqlen, nheads, state_dim), dev,
-                         2 * batch * nheads * seqlen * state_dim * mt.itemsize)
+    rows = 2 * batch * nheads * seqlen * state_dim * mt.itemsize
+    workspace = _scratch(   # compact phi is never cut: the per-head rows alone
+        rows if isinstance(phi, PhiStrips)
+        else lib.m3s_bwd_workspace_bytes(dcode, batch, seqlen, nheads, state_dim), dev, rows)
 
     a = _lib.BwdArgs()
     a.struct_size = ctypes.sizeof(_lib.BwdArgs)

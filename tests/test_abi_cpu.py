@@ -199,6 +199,37 @@ def test_split_scratch_is_bounded(lib):
     assert 0 < fwd(1, 131072, 32) <= 1 << 30 and fwd(1, 131072 + 128, 32) == 0
 
 
+def test_split_scratch_is_for_calls_that_are_cut(lib):
+    """A call is asked for scratch only where its scan is cut: not with compact phi, not in raw
+    mode past the angles that the bf16 kernel builds, not where a stream's strides are past its
+    addressing; and the most for the shape otherwise."""
+    h = lib.load()
+
+    def need(seqlen=2048, stride_t=64, n=128, chunk=128, nr=32, **fields):
+        a = lib.FwdArgs()
+        a.struct_size = ctypes.sizeof(lib.FwdArgs)
+        a.batch, a.seqlen, a.nheads, a.headdim, a.state_dim, a.n_angles, a.chunk = 1, seqlen, 4, 64, n, nr, chunk
+        a.dtype = lib.DTYPE_BF16
+        a.v = a.y = lib.Bhlp(0x1000, 0, 0, stride_t)
+        raw = lib.Blx(0x1000, 0, 4480)
+        if fields.pop("raw", 0):
+            a.raw, a.theta_table, a.dt_raw, a.a_raw, a.trap_raw = 1, 0x1000, raw, raw, raw
+        else:
+            a.phi = 0x1000
+        for k, v in fields.items():
+            setattr(a, k, v)
+        got = h.m3s_fwd_scratch_bytes(ctypes.byref(a))
+        return got, h.m3s_fwd_workspace_bytes(lib.DTYPE_BF16, 1, seqlen, 4, 64, n, chunk)
+
+    for kw in (dict(), dict(raw=1), dict(n=64, nr=32), dict(n=64, chunk=64, nr=32, raw=1)):
+        got, most = need(**kw)
+        assert got == most > 0, kw
+    assert need(phi=None, theta_table=0x1000, phi_dt=0x1000, phi_strips=0x1000)[0] == 0
+    assert need(raw=1, nr=64)[0] == 0            # one block of 32 angles is built at chunk 128
+    assert need(stride_t=1 << 20)[0] == 0        # 2048 rows of 2 MB: past 31-bit offsets
+    assert need(chunk=96)[0] == -1 and h.m3s_fwd_scratch_bytes(None) == -1
+
+
 def test_prep_arguments_are_checked_without_a_launch(lib):
     h = lib.load()
     assert h.m3s_prep_fwd(None, None) == lib.ERR_INVALID
