@@ -30,6 +30,8 @@
 extern "C" {
 #endif
 
+/* Rises when a struct or what an entry point asks of its caller changes. Entry points are added
+ * without it: a caller built against this header needs a library that has those it calls. */
 #define M3S_ABI_VERSION 10
 
 #define M3S_DTYPE_F32 0  /* f32 operands, v_mfma_f32_16x16x4_f32 ("f32" policy)  */

@@ -255,6 +255,13 @@ def load(path: str = LIB_PATH) -> C.CDLL:
             "(the HIP kernels are the only compute path)")
     lib = C.CDLL(path)
     lib.m3s_abi_version.restype = i32
+    ver = lib.m3s_abi_version()
+    if ver != ABI_VERSION:
+        raise RuntimeError(f"{path} has ABI version {ver}, expected {ABI_VERSION}; rebuild it")
+    # a version's entry points only grow in number: a library built before one was added lacks it
+    missing = [name for name in EXPORTS if not hasattr(lib, name)]
+    if missing:
+        raise RuntimeError(f"{path} is older than this package (no {', '.join(missing)}); rebuild it")
     lib.m3s_last_error.restype = C.c_char_p
     lib.m3s_supported.restype = i32
     lib.m3s_supported.argtypes = [i32, i32, i32, i32, i32]
@@ -320,9 +327,6 @@ def load(path: str = LIB_PATH) -> C.CDLL:
     lib.m3s_gemv.argtypes = [C.POINTER(GemvArgs), vp]
     lib.m3s_gemv_fused.restype = i32
     lib.m3s_gemv_fused.argtypes = [C.POINTER(GemvFusedArgs), vp]
-    ver = lib.m3s_abi_version()
-    if ver != ABI_VERSION:
-        raise RuntimeError(f"{path} has ABI version {ver}, expected {ABI_VERSION}; rebuild it")
     _lib = lib
     return lib
 

@@ -36,6 +36,19 @@ def test_library_loads_and_exports_every_declared_symbol(lib):
     assert handle.m3s_abi_version() == lib.ABI_VERSION == 10
 
 
+@pytest.mark.parametrize("version,match", [(9, "ABI version 9"), (10, "no m3s_last_error, .*m3s_bwd_ws.*rebuild")])
+def test_a_stale_library_is_named_as_such(lib, monkeypatch, tmp_path, version, match):
+    """A library of another version, or of this one from before an entry point was added, is
+    refused with the advice to rebuild it."""
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text(f"int m3s_abi_version(void) {{ return {version}; }}")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    monkeypatch.setattr(lib, "_lib", None)
+    with pytest.raises(RuntimeError, match=match):
+        lib.load(str(so))
+    assert lib._lib is None
+
+
 def test_struct_layouts_match_the_header(lib):
     """Compile the header with gcc and compare sizeof/offsetof with the ctypes mirror."""
     src = r"""
