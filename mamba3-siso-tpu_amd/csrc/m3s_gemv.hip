@@ -463,13 +463,18 @@ extern "C" int32_t m3s_gemv_fused(const m3s_gemv_fused_args* a, void* stream) {
                 a->k, kGvNormMax);
     M3S_REQUIRE(a->gain && aligned16(a->x) && aligned16(a->gain) && (!a->add || aligned16(a->add)),
                 "m3s_gemv_fused: stream, gain or add NULL or misaligned");
-    M3S_REQUIRE(a->mode == M3S_GEMV_HEAD || !a->add || a->sum, "m3s_gemv_fused: add without sum");
+    // every workgroup reads the stream and add while the first one writes the sum
+    M3S_REQUIRE(a->mode == M3S_GEMV_HEAD || !a->add ||
+                    (a->sum && a->sum != a->x && a->sum != a->add && aligned16(a->sum)),
+                "m3s_gemv_fused: add needs an aligned sum that is neither x nor add");
     p.stream = a->x; p.add = static_cast<const bf16*>(a->add); p.gain = a->gain; p.sum = a->sum;
     p.eps = a->eps;
   }
   const bool x32 = a->x_dtype == M3S_DTYPE_F32;
   if (a->mode == M3S_GEMV_HEAD) {
     M3S_REQUIRE(aligned16(a->w), "m3s_gemv_fused: the table is misaligned");
+    M3S_REQUIRE(a->w_dtype == M3S_DTYPE_F32 || a->w_dtype == M3S_DTYPE_BF16,
+                "m3s_gemv_fused: bad w_dtype %d", a->w_dtype);
     const dim3 grid((unsigned)((a->n + 3) / 4));
     float* out = static_cast<float*>(a->y);
 #define M3S_HEAD(TX, TE) \

@@ -451,6 +451,26 @@ def test_gemv_arguments_are_checked_without_a_launch(lib):
     assert h.m3s_gemv(ctypes.byref(a), None) == lib.ERR_INVALID   # the tiles: x row stride
 
 
+def test_gemv_fused_arguments_are_checked_without_a_launch(lib):
+    h = lib.load()
+    assert h.m3s_gemv_fused(None, None) == lib.ERR_INVALID
+    a = lib.GemvFusedArgs()
+    a.struct_size = ctypes.sizeof(lib.GemvFusedArgs)
+    a.rows, a.k, a.n, a.mode = 1, 256, 64, lib.GEMV_NORM
+    a.x_dtype, a.w_dtype, a.eps = lib.DTYPE_F32, lib.DTYPE_BF16, 1e-5
+    a.x, a.add, a.gain, a.w, a.y = 0x1000, 0x2000, 0x3000, 0x4000, 0x5000
+    for bad in (None, a.x, a.add, 0x6002):                    # no sum, an alias, a misaligned one
+        a.sum = bad
+        assert h.m3s_gemv_fused(ctypes.byref(a), None) == lib.ERR_INVALID
+        assert b"sum" in h.m3s_last_error()
+    a.mode, a.sum, a.w_dtype = lib.GEMV_HEAD, None, 7          # the table's type
+    assert h.m3s_gemv_fused(ctypes.byref(a), None) == lib.ERR_INVALID
+    assert b"w_dtype" in h.m3s_last_error()
+    a.rows = 3
+    assert h.m3s_gemv_fused(ctypes.byref(a), None) == lib.ERR_INVALID
+    assert b"rows" in h.m3s_last_error()
+
+
 def test_adamw_arguments_are_checked_without_a_launch(lib):
     h = lib.load()
     assert h.m3s_adamw(None, None) == lib.ERR_INVALID
