@@ -60,14 +60,21 @@ def test_split_scan_equals_whole(m3, dev, whole, b, h, nc, chunk, n, p, nr, seed
     assert torch.equal(got[4].chunk_states, ref[4].chunk_states), "chunk_states"
 
 
-@pytest.mark.parametrize("b,h,nc,chunk,n,p,nr", [s for s in SHAPES if s[6] % 4 == 0])
+# raw mode's own: of SHAPES those whose angle tables fit (a chunk's, for all heads, in 64 KiB),
+# and whole sequences before the split ones (256 of 264, 288 and 384; two segments of 128)
+RAW_SHAPES = [s for s in SHAPES if s[6] % 4 == 0 and s[1] < 64] + [
+    (11, 24, 5, 128, 128, 64, 32), (9, 32, 4, 128, 128, 64, 32), (16, 24, 8, 128, 128, 64, 32),
+    (4, 32, 8, 128, 128, 64, 32), (20, 16, 9, 64, 64, 64, 16)]
+
+
+@pytest.mark.parametrize("b,h,nc,chunk,n,p,nr", RAW_SHAPES)
 @pytest.mark.parametrize("phi_init", [False, True])
 def test_split_raw_scan_equals_whole(m3, dev, whole, b, h, nc, chunk, n, p, nr, phi_init):
     K, L = m3.kernels, nc * chunk
+    assert _split_bytes(m3, b, h, L, n, p, chunk) > 0, "the shape does not split"
     _, d = raw_case(b, h, L, n, p, nr, seed=nc, phi_init=phi_init)
     dt, a, trap, ang = views(d, h, nr)
-    if not K.raw_forward_ok("bf16", chunk, n, p, nr, L, h):
-        pytest.skip("no raw-mode kernel for this shape")
+    assert K.raw_forward_ok("bf16", chunk, n, p, nr, L, h), "no raw-mode kernel for this shape"
     (k, q), _, angs = K.bcnorm_forward([d["kr"], d["qr"]], [d["wb"], d["wc"]], 1e-5,
                                        theta=(ang, dt, d["bias"], chunk))
 
