@@ -163,11 +163,17 @@ template <> __device__ __forceinline__ float buf_load<float>(__amdgpu_buffer_rsr
 template <> __device__ __forceinline__ bf16 buf_load<bf16>(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
   return __builtin_bit_cast(bf16, __builtin_amdgcn_raw_buffer_load_b16(r, v, s, 0));
 }
+// A 16-byte store reads its data registers over several cycles, and a vector instruction
+// behind it may overwrite them first. The compiler keeps two wait states between the two where
+// the store's soffset is zero, and takes one with an SGPR soffset for safe. It is not: with two
+// workgroups on a CU the first dword of lanes 12-15 of every 16 went out as the next address
+// product (chunk 64, state 64, 320 sequences, 1 in 1000 entries of y). So the uniform offset
+// goes into the lane's.
 __device__ __forceinline__ void buf_store(bf16x8 x, __amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, x), r, v, s, 0);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, x), r, v + s, 0, 0);
 }
 __device__ __forceinline__ void buf_store(f32x4 x, __amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, x), r, v, s, 0);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, x), r, v + s, 0, 0);
 }
 __device__ __forceinline__ void buf_store(bf16x4 x, __amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, x), r, v, s, 0);

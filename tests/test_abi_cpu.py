@@ -5,6 +5,7 @@ No kernel is launched here."""
 import ctypes
 import os
 import re
+import shutil
 import subprocess
 import tempfile
 
@@ -497,3 +498,27 @@ def test_adamw_arguments_are_checked_without_a_launch(lib):
     a.bias_correction2_sqrt = 0.1
     assert h.m3s_adamw(ctypes.byref(a), None) == lib.ERR_INVALID   # negative numel
     assert b"numel" in h.m3s_last_error()
+
+
+def test_wide_buffer_stores_carry_no_scalar_offset(lib, tmp_path):
+    """A vector instruction may overwrite a 16-byte buffer store's data before the store has read
+    it; the compiler keeps them apart only where the store's soffset is zero (`buf_store`). In
+    the built scans every such store has it so."""
+    objdump = "/opt/rocm/llvm/bin/llvm-objdump"
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
+    shutil.copy(lib.LIB_PATH, tmp_path / "lib.so")
+    subprocess.run([objdump, "--offloading", "lib.so"], check=True, cwd=tmp_path, capture_output=True)
+    found = 0
+    for obj in tmp_path.glob("lib.so.*gfx950"):
+        if not any(name in obj.read_bytes() for name in (b"fwd_bf16_kernel", b"bwd_bf16_kernel")):
+            continue
+        out = tmp_path / "code.txt"
+        with open(out, "w") as f:
+            subprocess.run([objdump, "-d", "--no-show-raw-insn", str(obj)], check=True, stdout=f)
+        for line in open(out):
+            m = re.search(r"buffer_store_dwordx[34] \S+ \S+ s\[\d+:\d+\], (\S+)", line)
+            if m:
+                found += 1
+                assert m.group(1) == "0", line
+    assert found > 0
