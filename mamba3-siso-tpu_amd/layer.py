@@ -187,9 +187,12 @@ _DIRECT_MAX = 2048 * 1024
 
 def _weights_direct(u: Tensor, in_proj: Tensor, out_proj: Tensor, cfg: SISOConfig) -> bool:
     """Whether a forward without gradients skips the weights' layout copies: few tokens,
-    weights already in u's dtype, and projection rows that stay 16-byte aligned unpadded."""
+    weights already in u's dtype and dense from a 16-byte boundary (a view into a flat buffer
+    may start anywhere; the copies align it for the library), and projection rows that stay
+    16-byte aligned unpadded."""
     return (u.numel() <= _DIRECT_MAX and in_proj.dtype == out_proj.dtype == u.dtype
             and in_proj.is_contiguous() and out_proj.is_contiguous()
+            and in_proj.data_ptr() % 16 == 0 and out_proj.data_ptr() % 16 == 0
             and cfg.d_in_proj % (16 // u.element_size()) == 0)
 
 

@@ -796,3 +796,24 @@ def test_segment_with_an_out_proj_of_another_width(m3, dev):
         got = m3.mamba3_siso_layer(p._replace(out_proj=p.out_proj[:, :128]), u, cfg, state=st)[0]
     assert tuple(got.shape) == (2, 128, 128)
     assert_bf16_bound(got, cpu(full[..., :128]), what="out")
+
+
+@pytest.mark.parametrize("field", ["in_proj", "out_proj"])
+def test_forward_with_weights_off_a_16_byte_boundary(m3, dev, field):
+    """A weight that is a view into a flat buffer may start at any element: it goes through the
+    layout copy, with the aligned weight's result (one operand rounding where the library sums
+    in another order)."""
+    LY = m3.layer
+    cfg = m3.SISOConfig(d_model=256)
+    p = m3.init_params(cfg, 5, device=dev)
+    p = p._replace(in_proj=p.in_proj.to(BF16), out_proj=p.out_proj.to(BF16))
+    u = torch.randn(1, 128, 256, generator=torch.Generator().manual_seed(2)).to(BF16).to(dev)
+    w = getattr(p, field)
+    flat = torch.empty(w.numel() + 1, dtype=BF16, device=dev)
+    flat[1:] = w.reshape(-1)
+    q = p._replace(**{field: flat[1:].view(w.shape)})
+    assert LY._weights_direct(u, p.in_proj, p.out_proj, cfg)
+    assert not LY._weights_direct(u, q.in_proj, q.out_proj, cfg)
+    with torch.no_grad():
+        got, ref = (m3.mamba3_siso_layer(x, u, cfg)[0] for x in (q, p))
+    assert_bf16_bound(got, cpu(ref), what="out")
