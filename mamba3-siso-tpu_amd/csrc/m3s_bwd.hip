@@ -931,7 +931,7 @@ struct Bwd2Cfg {
   static_assert(C <= N, "the dv rows are staged in the adjoint's N-row slot");
 };
 
-// dy silu(z), the hardware exp2 and reciprocal (sg is sigma(z))
+// sigma(z) by the hardware exp2 and reciprocal, and dy silu(z)
 __device__ __forceinline__ float gate_sig(float z) {
   return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-z * kLog2e));
 }

@@ -388,7 +388,7 @@ struct DecScanParams {
 // instructions a step, and leaves most CUs idle. There the next window's inputs are read
 // into registers under the steps, too. The parts cannot write the carried k~ and phi in
 // place, since another part may not have started: part 0 leaves them in `carry`, which
-// dec_carry_kernel copies back. B=1, H=32: 512 steps 408 -> 209 us, 48 steps
+// dec_carry_kernel copies back. B=1, H=32: 512 steps 408 -> 205 us, 48 steps
 // 43 -> 26; B=8, 256 steps (4 parts) 217 -> 186.
 template <typename MT, int N, int P, int PARTS>
 __global__ void __launch_bounds__(kDecThreads)

@@ -37,8 +37,10 @@ constexpr int kWgStage = 2 * kWgK * kWgLd;   // A then B, bf16 elements per stag
 constexpr int kWgMaxSplit = 16;
 // Tiles are taken in bands of this many tile rows, down the rows first: the 32 blocks that run
 // on one XCD then share 6 row and about 6 column panels of a step instead of 1-2 and 25, so
-// its L2 passes less on. 4 x 25 tiles of 65536 tokens: 800 -> 769 us; 3 x 20 of 32768: 248 -> 241;
-// grids that fit one XCD whole (8 x 4) are the same either way.
+// its L2 passes less on. The layer's in_proj at d_model 1024 (65536 tokens, 1024 x 4480, 4 x 18
+// tiles): 576 us row by row, 552 in bands; bands of 4 or 8 rows are the same. The LM's widths at
+// 32768 tokens do not tell (768 x 3432 169 us, 768 x 3072 144, 1536 x 768 80 either way), nor does
+// out_proj at 65536 (2048 x 1024, 8 x 4 tiles, which fit one XCD whole: 245).
 constexpr int kWgBand = 6;
 
 struct WgParams {
@@ -152,9 +154,10 @@ __global__ void __launch_bounds__(kWgThreads) wgrad_kernel(const WgParams p) {
   // one of each on every SIMD (waves w and w + 4), in opposite order: in the phase after
   // barrier k the first reads step k's fragments and then multiplies them, the second
   // multiplies step k - 1's and then reads step k's. Every wave writes step k + 1 to the stage
-  // that phase k - 1 read. All waves in one order took 769 us where this takes 748 (65536
-  // tokens, 1024 x 6352), 241 -> 238 (32768, 768 x 4880), 104 -> 101 (32768, 768 x 2048); a strict half-step offset
-  // with a third stage and two barriers a step was 9% slower.
+  // that phase k - 1 read. All waves in one order, in the same bands, took 563 us where this takes
+  // 552 (65536 tokens, 1024 x 4480), 252 -> 244 (2048 x 1024), and at 32768 tokens 181 -> 168
+  // (768 x 3432), 150 -> 143 (768 x 3072), 81 -> 79 (1536 x 768); a strict half-step offset with a
+  // third stage and two barriers a step was 9% slower.
   if (n > 0) {
     gload(0);
     swrite(0);

@@ -1186,6 +1186,9 @@ def matmul(x: Tensor, w: Tensor) -> Tensor:
 
 
 #: Rows and widths of the products with a norm or the gate folded in (``m3s_gemv_fused``).
+#: A recorded step of the 8-layer LM (d_model 768), folded against pass by pass: one row 287
+#: against 363 us, two 343 against 444. The kernel built for four rows: three 367 against 384,
+#: four 405 against 388, as every workgroup normalises every row for itself.
 FUSED_ROWS_MAX, FUSED_NORM_MAX = 2, 1024
 
 
