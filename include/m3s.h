@@ -156,7 +156,7 @@ typedef struct m3s_bwd_args {
   float* dk_bias;              /* out (B, H, N)                                        */
   float* k_final;              /* out (B, H, N) rotated k at the last position         */
   float* dseed_ssm;            /* out (B, H, P, N) adjoint of the seeded state         */
-  void* workspace;             /* scratch, m3s_bwd_workspace_bytes() bytes, 16-aligned */
+  void* workspace;             /* scratch, the per-head rows (m3s_bwd) or what m3s_bwd_ws is told, 16-aligned */
 } m3s_bwd_args;
 
 /* Single-token decode, in place. Replaces `kernel_decode.siso_decode_folded` /
@@ -521,11 +521,11 @@ int64_t m3s_norm_bwd_workspace_bytes(int32_t width);
  * counterpart in the reference. -1 on a bad width. */
 int64_t m3s_rms_bwd_workspace_bytes(int32_t width);
 
-/* The most bytes of m3s_fwd_ws's workspace for a shape: the states and decays of the pieces of the sequences
- * that the scan cuts into segments, where B*H sequences leave its last round of workgroups
- * half empty or emptier; 0 where none is cut, and where the states would take more than
- * 1 GiB. No counterpart in the reference. -1 on bad
- * dimensions or a shape without a kernel. */
+/* The most bytes of m3s_fwd_ws's workspace for a shape: the states and decays of the pieces of
+ * the sequences that the scan cuts into segments, where B*H sequences leave its last round of
+ * workgroups half empty or emptier; 0 where none is cut, and where the states would take more
+ * than 1 GiB. No counterpart in the reference. -1 on bad dimensions or a shape without a
+ * kernel. */
 int64_t m3s_fwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t seqlen, int32_t nheads,
                                 int32_t headdim, int32_t state_dim, int32_t chunk);
 /* The bytes that this very call uses: as above, or 0 where its mode, angles or strides leave
