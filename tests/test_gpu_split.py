@@ -64,7 +64,9 @@ def test_split_scan_equals_whole(m3, dev, whole, b, h, nc, chunk, n, p, nr, seed
 # and whole sequences before the split ones (256 of 264, 288 and 384; two segments of 128)
 RAW_SHAPES = [s for s in SHAPES if s[6] % 4 == 0 and s[1] < 64] + [
     (11, 24, 5, 128, 128, 64, 32), (9, 32, 4, 128, 128, 64, 32), (16, 24, 8, 128, 128, 64, 32),
-    (4, 32, 8, 128, 128, 64, 32), (20, 16, 9, 64, 64, 64, 16)]
+    (4, 32, 8, 128, 128, 64, 32), (20, 16, 9, 64, 64, 64, 16),
+    # more chunks than the angles entering a segment are staged for at once (67 at 64 angles)
+    (1, 1, 150, 64, 128, 64, 64)]
 
 
 @pytest.mark.parametrize("b,h,nc,chunk,n,p,nr", RAW_SHAPES)
