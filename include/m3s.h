@@ -494,13 +494,17 @@ int32_t m3s_supported(int32_t which, int32_t dtype, int32_t chunk, int32_t state
 int32_t m3s_fwd_raw_supported(int32_t dtype, int32_t chunk, int32_t state_dim, int32_t headdim,
                               int32_t n_angles);
 
-/* Bytes of m3s_bwd_args.workspace for m3s_bwd_ws: the per-head dq/dk rows, 2*B*H*L*N elements
+/* The most bytes of m3s_bwd_args.workspace for m3s_bwd_ws at a shape: the per-head dq/dk rows, 2*B*H*L*N elements
  * of the dtype (all that m3s_bwd uses), and, where the scan cuts sequences into segments
  * (m3s_fwd_workspace_bytes), the chunks' shares of the adjoint. Not monotone in B*H: 128
  * sequences are cut and need more than 130, which are not. No counterpart in the reference
  * (its head sum is an in-kernel accumulation over an H-innermost grid, kernel_bwd.py:324-333). */
 int64_t m3s_bwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t seqlen, int32_t nheads,
                                 int32_t state_dim);
+/* The bytes that this very call uses: the rows alone where its kernel, phi or strides leave
+ * every sequence whole. Looks at the sizes, strides and which pointers are set. -1 on bad
+ * dimensions or a shape without a kernel. */
+int64_t m3s_bwd_scratch_bytes(const m3s_bwd_args* args);
 
 /* Bytes of m3s_prep_fwd_args.workspace: the tanh(angles) pi table (B, L, Nr) and the
  * theta totals per 16-token strip (B, ceil(L/16), H, Nr), f32 (per 64-token block when phi
@@ -547,7 +551,7 @@ int32_t m3s_fwd_ws(const m3s_fwd_args* args, void* workspace, int64_t workspace_
 /* m3s_bwd is m3s_bwd_ws with a workspace of the per-head rows alone: no sequence is cut. */
 int32_t m3s_bwd(const m3s_bwd_args* args, void* stream);
 /* `workspace_bytes`: the size of args->workspace, at least the per-head rows. Sequences are cut
- * only where m3s_bwd_workspace_bytes() of the shape are there. Same bits, but for the bias
+ * only where m3s_bwd_scratch_bytes() of the call are there. Same bits, but for the bias
  * gradients, whose float32 sums run per segment first. */
 int32_t m3s_bwd_ws(const m3s_bwd_args* args, int64_t workspace_bytes, void* stream);
 int32_t m3s_decode(const m3s_decode_args* args, void* stream);

@@ -232,7 +232,7 @@ EXPORTS = ("m3s_abi_version", "m3s_last_error", "m3s_supported", "m3s_fwd_raw_su
            "m3s_bwd_workspace_bytes",
            "m3s_prep_fwd_workspace_bytes", "m3s_prep_bwd_workspace_bytes", "m3s_fwd", "m3s_fwd_ws",
            "m3s_fwd_workspace_bytes", "m3s_fwd_scratch_bytes", "m3s_decode_scan_ws", "m3s_decode_scan_workspace_bytes",
-           "m3s_bwd", "m3s_bwd_ws", "m3s_decode", "m3s_decode_scan",
+           "m3s_bwd", "m3s_bwd_ws", "m3s_bwd_scratch_bytes", "m3s_decode", "m3s_decode_scan",
            "m3s_prep_fwd", "m3s_prep_bwd", "m3s_norm_bwd_workspace_bytes", "m3s_norm_fwd",
            "m3s_norm_bwd", "m3s_decode_layer", "m3s_transpose", "m3s_swiglu_fwd",
            "m3s_swiglu_bwd", "m3s_rms_fwd", "m3s_rms_bwd", "m3s_rms_bwd_workspace_bytes",
@@ -281,6 +281,8 @@ def load(path: str = LIB_PATH) -> C.CDLL:
     lib.m3s_bwd.argtypes = [C.POINTER(BwdArgs), vp]
     lib.m3s_bwd_ws.restype = i32
     lib.m3s_bwd_ws.argtypes = [C.POINTER(BwdArgs), i64, vp]
+    lib.m3s_bwd_scratch_bytes.restype = i64
+    lib.m3s_bwd_scratch_bytes.argtypes = [C.POINTER(BwdArgs)]
     lib.m3s_decode.restype = i32
     lib.m3s_decode.argtypes = [C.POINTER(DecodeArgs), vp]
     lib.m3s_decode_scan.restype = i32

@@ -2056,18 +2056,34 @@ static int64_t bwd_split_floats(const Split& sp, int64_t nseq, int nc, int N, in
   return split_floats(sp, nseq, nc, N, P, true) + rows * (2 * N + N * P);
 }
 
-// `spare`: workspace bytes past the per-head rows; a split needs bwd_split_floats of them.
+// Whether a call runs the bf16 kernel, which alone may be cut (with phi read).
+template <typename MT, int C, int N, int P>
+constexpr bool bwd_fast() {   // N <= 128: a strip's row pairs in one wave (phi strips)
+  return std::is_same<MT, bf16>::value && N % 64 == 0 && C % 64 == 0 && C <= N && N / 16 <= 8;
+}
+
+// The split of a call, and its scratch past the per-head rows.
+template <typename MT, int C, int N, int P>
+static Split bwd_plan(const BwdParams& p, int64_t& bytes) {
+  const int64_t nseq = (int64_t)p.B * p.H;
+  Split sp{(int)nseq, 1};
+  if constexpr (bwd_fast<MT, C, N, P>())
+    if (!p.pstr && bwd_fits_rsrc(p, N, P)) sp = plan_split(nseq, p.nc, C, kBwdMinSaved, N * P * 4);
+  bytes = 4 * bwd_split_floats(sp, nseq, p.nc, N, P);
+  return sp;
+}
+
+// `spare`: workspace bytes past the per-head rows, enough for the split or none is made.
 template <typename MT, int C, int N, int P>
 static int32_t launch_bwd(BwdParams prm, int grid, int64_t spare, hipStream_t stream) {
   bool done = false;
   const bool strips = prm.pstr != nullptr;
   const int nseq = grid;
-  prm.split = Split{nseq, 1};
-  if constexpr (std::is_same<MT, bf16>::value && N % 64 == 0 && C % 64 == 0 && C <= N &&
-                N / 16 <= 8) {   // N <= 128: a strip's row pairs in one wave (phi strips)
+  int64_t need;
+  prm.split = bwd_plan<MT, C, N, P>(prm, need);
+  if (need > spare) prm.split = Split{nseq, 1};
+  if constexpr (bwd_fast<MT, C, N, P>()) {
     if (bwd_fits_rsrc(prm, N, P)) {
-      const Split sp = plan_split(nseq, prm.nc, C, kBwdMinSaved, N * P * 4);
-      if (!strips && 4 * bwd_split_floats(sp, nseq, prm.nc, N, P) <= spare) prm.split = sp;
       if (prm.split.segs > 1) {
         const int rem = nseq - prm.split.whole;
         const int64_t nsh = (int64_t)rem * prm.split.shares(prm.nc, true);
@@ -2143,6 +2159,36 @@ int32_t bwd_supported(int dtype, int chunk, int n, int pdim) {
   return 0;
 }
 
+// The kernels' parameters of a call (no pointer is followed; chunk > 0).
+static BwdParams bwd_params(const m3s_bwd_args* a) {
+  const bool strips = a->theta_table || a->phi_dt || a->phi_strips;
+  BwdParams prm{};
+  prm.B = a->batch; prm.L = a->seqlen; prm.H = a->nheads; prm.Nr = a->n_angles;
+  prm.nc = a->seqlen / a->chunk;
+  prm.has_d = a->has_d; prm.has_z = a->has_z;
+  prm.dy = a->dy.ptr; prm.dy_sb = a->dy.stride_b; prm.dy_sh = a->dy.stride_h; prm.dy_st = a->dy.stride_t;
+  prm.ybar = a->ybar;
+  prm.z = a->has_z ? a->z.ptr : nullptr;
+  prm.z_sb = a->z.stride_b; prm.z_sh = a->z.stride_h; prm.z_st = a->z.stride_t;
+  prm.q = a->q; prm.k = a->k;
+  prm.v = a->v.ptr; prm.v_sb = a->v.stride_b; prm.v_sh = a->v.stride_h; prm.v_st = a->v.stride_t;
+  prm.adt = a->adt; prm.gamma = a->gamma; prm.scale = a->scale; prm.phi = a->phi;
+  prm.tht = strips ? a->theta_table : nullptr;
+  prm.pdt = strips ? a->phi_dt : nullptr;
+  prm.pstr = strips ? a->phi_strips : nullptr;
+  prm.qb = a->q_bias; prm.kb = a->k_bias; prm.dsk = a->d_skip;
+  prm.cstates = a->chunk_states; prm.dfs = a->dfinal_ssm; prm.dfv = a->dfinal_v;
+  prm.dq = a->dq; prm.dk = a->dk;
+  prm.dv = a->dv.ptr; prm.dv_sb = a->dv.stride_b; prm.dv_sh = a->dv.stride_h; prm.dv_st = a->dv.stride_t;
+  prm.dz = a->has_z ? a->dz.ptr : nullptr;
+  prm.dz_sb = a->dz.stride_b; prm.dz_sh = a->dz.stride_h; prm.dz_st = a->dz.stride_t;
+  prm.dadt = a->dadt; prm.dqk = a->dqk_diag; prm.dscale = a->dscale; prm.uw = a->uw;
+  prm.dphi = a->dphi; prm.dqb = a->dq_bias; prm.dkb = a->dk_bias; prm.kfin = a->k_final;
+  prm.dseed = a->dseed_ssm;
+  prm.part = a->workspace;
+  return prm;
+}
+
 }  // namespace m3s
 
 // Bytes of the per-head rows.
@@ -2164,6 +2210,21 @@ extern "C" int64_t m3s_bwd_workspace_bytes(int32_t dtype, int32_t batch, int32_t
         split = std::max(split, bwd_split_floats(sp, nseq, seqlen / c, state_dim, 64));
       }
   return rows + 4 * split;
+}
+
+extern "C" int64_t m3s_bwd_scratch_bytes(const m3s_bwd_args* a) {
+  using namespace m3s;
+  if (a == nullptr || a->struct_size != (int32_t)sizeof(m3s_bwd_args) || a->batch <= 0 || a->seqlen <= 0 ||
+      a->nheads <= 0 || !bwd_supported(a->dtype, a->chunk, a->state_dim, a->headdim))
+    return -1;
+  const BwdParams prm = bwd_params(a);
+  int64_t split = 0;
+#define X(MT, CC, NN, PP)                                                                            \
+  if (a->dtype == bcode<MT>() && a->chunk == CC && a->state_dim == NN && a->headdim == PP)           \
+    bwd_plan<MT, CC, NN, PP>(prm, split);
+  M3S_BWD_CONFIGS(X)
+#undef X
+  return bwd_rows_bytes(a->dtype, a->batch, a->seqlen, a->nheads, a->state_dim) + split;
 }
 
 static int32_t bwd_run(const m3s_bwd_args* a, int64_t workspace_bytes, void* stream) {
@@ -2212,29 +2273,7 @@ static int32_t bwd_run(const m3s_bwd_args* a, int64_t workspace_bytes, void* str
   M3S_REQUIRE(spare >= 0, "m3s_bwd: workspace of %lld bytes is smaller than the per-head rows' %lld",
               (long long)workspace_bytes, (long long)(workspace_bytes - spare));
 
-  BwdParams prm{};
-  prm.B = B; prm.L = L; prm.H = H; prm.Nr = Nr; prm.nc = L / C;
-  prm.has_d = a->has_d; prm.has_z = a->has_z;
-  prm.dy = a->dy.ptr; prm.dy_sb = a->dy.stride_b; prm.dy_sh = a->dy.stride_h; prm.dy_st = a->dy.stride_t;
-  prm.ybar = a->ybar;
-  prm.z = a->has_z ? a->z.ptr : nullptr;
-  prm.z_sb = a->z.stride_b; prm.z_sh = a->z.stride_h; prm.z_st = a->z.stride_t;
-  prm.q = a->q; prm.k = a->k;
-  prm.v = a->v.ptr; prm.v_sb = a->v.stride_b; prm.v_sh = a->v.stride_h; prm.v_st = a->v.stride_t;
-  prm.adt = a->adt; prm.gamma = a->gamma; prm.scale = a->scale; prm.phi = a->phi;
-  prm.tht = strips ? a->theta_table : nullptr;
-  prm.pdt = strips ? a->phi_dt : nullptr;
-  prm.pstr = strips ? a->phi_strips : nullptr;
-  prm.qb = a->q_bias; prm.kb = a->k_bias; prm.dsk = a->d_skip;
-  prm.cstates = a->chunk_states; prm.dfs = a->dfinal_ssm; prm.dfv = a->dfinal_v;
-  prm.dq = a->dq; prm.dk = a->dk;
-  prm.dv = a->dv.ptr; prm.dv_sb = a->dv.stride_b; prm.dv_sh = a->dv.stride_h; prm.dv_st = a->dv.stride_t;
-  prm.dz = a->has_z ? a->dz.ptr : nullptr;
-  prm.dz_sb = a->dz.stride_b; prm.dz_sh = a->dz.stride_h; prm.dz_st = a->dz.stride_t;
-  prm.dadt = a->dadt; prm.dqk = a->dqk_diag; prm.dscale = a->dscale; prm.uw = a->uw;
-  prm.dphi = a->dphi; prm.dqb = a->dq_bias; prm.dkb = a->dk_bias; prm.kfin = a->k_final;
-  prm.dseed = a->dseed_ssm;
-  prm.part = a->workspace;
+  const BwdParams prm = bwd_params(a);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int grid = B * H;
 #define X(MT, CC, NN, PP)                                              \

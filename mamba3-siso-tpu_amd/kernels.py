@@ -787,11 +787,6 @@ def siso_backward_kernel(
     dkb = empty(batch, nheads, state_dim, **f32)
     kfin = empty(batch, nheads, state_dim, **f32)
     dseed = empty(batch, nheads, headdim, state_dim, **f32)
-    lib = _lib.load()
-    rows = 2 * batch * nheads * seqlen * state_dim * mt.itemsize
-    workspace = _scratch(   # compact phi is never cut: the per-head rows alone
-        rows if isinstance(phi, PhiStrips)
-        else lib.m3s_bwd_workspace_bytes(dcode, batch, seqlen, nheads, state_dim), dev, rows)
 
     a = _lib.BwdArgs()
     a.struct_size = ctypes.sizeof(_lib.BwdArgs)
@@ -809,6 +804,9 @@ def siso_backward_kernel(
     a.dadt, a.dqk_diag, a.dscale, a.uw = (t.data_ptr() for t in (dadt, dqk, dscale, uw))
     a.dphi, a.dq_bias, a.dk_bias = dphi.data_ptr(), dqb.data_ptr(), dkb.data_ptr()
     a.k_final, a.dseed_ssm = kfin.data_ptr(), dseed.data_ptr()
+    lib = _lib.load()
+    workspace = _scratch(lib.m3s_bwd_scratch_bytes(ctypes.byref(a)), dev,
+                         2 * batch * nheads * seqlen * state_dim * mt.itemsize)
     a.workspace = workspace.data_ptr()
     _lib.launch(lambda args, stream: lib.m3s_bwd_ws(args, workspace.numel(), stream), a, dev, "m3s_bwd")
     return KernelGrads(dq=dq, dk=dk, dv=dv, dadt=dadt, dqk_diag=dqk, dscale=dscale, dphi=dphi,

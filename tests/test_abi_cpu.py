@@ -244,6 +244,30 @@ def test_split_scratch_is_for_calls_that_are_cut(lib):
     assert need(chunk=96)[0] == -1 and h.m3s_fwd_scratch_bytes(None) == -1
 
 
+def test_backward_scratch_is_for_calls_that_are_cut(lib):
+    h = lib.load()
+
+    def need(stride_t=64, n=128, chunk=128, **fields):
+        a = lib.BwdArgs()
+        a.struct_size = ctypes.sizeof(lib.BwdArgs)
+        a.batch, a.seqlen, a.nheads, a.headdim, a.state_dim, a.n_angles, a.chunk = 1, 2048, 4, 64, n, 32, chunk
+        a.dtype, a.phi = lib.DTYPE_BF16, 0x1000
+        a.v = a.dy = a.dv = lib.Bhlp(0x1000, 0, 0, stride_t)
+        for k, v in fields.items():
+            setattr(a, k, v)
+        rows = 2 * 4 * 2048 * n * 2
+        return (h.m3s_bwd_scratch_bytes(ctypes.byref(a)) - rows,
+                h.m3s_bwd_workspace_bytes(lib.DTYPE_BF16, 1, 2048, 4, n) - rows)
+
+    for kw in (dict(), dict(chunk=64), dict(n=64, chunk=64)):
+        got, most = need(**kw)
+        assert 0 < got <= most, kw
+    assert need(n=64, chunk=128)[0] == 0         # a chunk longer than the state: the generic kernel
+    assert need(phi=None, theta_table=0x1000, phi_dt=0x1000, phi_strips=0x1000)[0] == 0
+    assert need(stride_t=1 << 20)[0] == 0        # past 31-bit offsets
+    assert h.m3s_bwd_scratch_bytes(None) == -1
+
+
 def test_prep_arguments_are_checked_without_a_launch(lib):
     h = lib.load()
     assert h.m3s_prep_fwd(None, None) == lib.ERR_INVALID
