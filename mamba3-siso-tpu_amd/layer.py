@@ -387,8 +387,8 @@ def _segment_fused_ok(params: SISOParams, u: Tensor, cfg: SISOConfig, state) -> 
     vectors = (params.dt_bias, params.b_norm_weight, params.c_norm_weight)
     shapes = ((b, h, cfg.headdim, n), (b, h, n), (b, h, cfg.headdim), (b, h, cfg.n_angles),
               (h,), (n,), (n,))
-    return all(tuple(t.shape) == s and t.device == u.device
-               for t, s in zip((*state, *vectors), shapes))
+    dev = u.device
+    return all(t.shape == s and t.device == dev for t, s in zip((*state, *vectors), shapes))
 
 
 def _segment_forward(params: SISOParams, u: Tensor, cfg: SISOConfig, state: SISOState):
